@@ -71,15 +71,10 @@ BYTES_PER_UNIT = {
     "k_ext_classify": [(32, "segments")],
     "k_ext_shadow": [(68, "shadow_segments")],
     "k_ext_shade_lambert": [(160, "lambert_hits")],
-    # reference mode (SoA scalar records):
-    #   k_ref_intersect: queue index 4 + ray 24 + hit (t, normal, material, light) 24 = 52 B per segment
-    #   k_ref_shade: reads queue 4, hit 24, ray 24, throughput 16, MIS weight 4, seed 4, hero
-    #     wavelength 4; writes ray 24, throughput 16, weight 4, seed 4, next-queue 4 = 132 B per
-    #     segment; + shadow record (path 4, ray 24, light object 4, contribution 16) 48 B per shadow ray
-    #   k_ref_shadow: reads ray 24 + light object 4, writes hit distance 4 + object 4 = 36 B per shadow ray
-    "k_ref_intersect": [(52, "segments")],
-    "k_ref_shade": [(132, "segments"), (48, "shadow_segments")],
-    "k_ref_shadow": [(36, "shadow_segments")],
+    # reference mode: a path stays in its lane's registers and leaves its XYZ, 16 B, which the
+    # fold reads (the kernel is bound by VALU issue, the shader's transcendentals restated)
+    "k_ref_path": [(16, "paths")],
+    "k_ref_fold": [(16, "paths")],
 }
 
 # Sphere-tracing kernels are bound by FP32 VALU work, not HBM. Their algorithmic

@@ -259,7 +259,7 @@ pt_status pt_sync(pt_ctx* ctx);
 /* No counterpart in the reference: pt_dispatch(..., PT_MODE_REF) that allocates
  * no device memory, for callers that cannot allocate (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). The path state
- * lives in a static device array of 65,536 paths (11,010,304 B), held by each
+ * lives in a static device array of 65,536 paths (1,843,456 B), held by each
  * device the library runs on until the process ends; a dispatch of more paths
  * runs as several waves through it, so it has no size limit beyond
  * pt_dispatch's. Texels equal pt_dispatch's bit for bit. All contexts on one

@@ -91,6 +91,10 @@ pt_status pt_create(pt_ctx** out, int device_ordinal, const pt_config* cfg) {
     }
     hipError_t e = hipSetDevice(device_ordinal);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
+    int cu = 0;
+    if (e == hipSuccess && hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, device_ordinal) == hipSuccess &&
+        cu > 0)
+        ctx->cus = cu;
     const size_t stat_bytes = (size_t)ptd::kStatLines * ptd::kStatStride * sizeof(unsigned long long);
     if (e == hipSuccess) e = hipMalloc(&ctx->d_stats, stat_bytes);
     if (e == hipSuccess) e = hipMemset(ctx->d_stats, 0, stat_bytes);
@@ -466,10 +470,10 @@ pt_status pt_dispatch(pt_ctx* ctx, const pt_scene* s, pt_accum* acc, const pt_pu
         } else if (mode == PT_MODE_EXT) {
             if (!s->has_model) return set_err(ctx, PT_ERR_STATE, "extended mode needs a scene loaded from JSON");
             st = ptk::ext_dispatch(ctx, s, acc, pc);
+            if (st == PT_OK) st = ptk::count_dispatch(ctx);
         } else {
             return set_err(ctx, PT_ERR_INVALID_ARG, "pt_dispatch: unknown mode");
         }
-        if (st == PT_OK) st = ptk::count_dispatch(ctx);
         return st;
     } catch (const std::exception& e) {
         return set_err(ctx, PT_ERR_HIP, std::string("pt_dispatch: ") + e.what());
@@ -492,9 +496,7 @@ pt_status pt_dispatch_noalloc(pt_ctx* ctx, const pt_scene* s, pt_accum* acc, con
     // kernel timing records events, which this entry point does not create
     if (ctx->prof) return set_err(ctx, PT_ERR_STATE, "pt_dispatch_noalloc: kernel profiling is enabled");
     (void)hipSetDevice(ctx->device);
-    int st = ptk::ref_dispatch_static(ctx, s, acc, pc);
-    if (st == PT_OK) st = ptk::count_dispatch(ctx);
-    return st;
+    return ptk::ref_dispatch_static(ctx, s, acc, pc);
 }
 
 pt_status pt_render_features(pt_ctx* ctx, const pt_scene* s, const pt_push_constants* pc, float* host, size_t n_floats) {

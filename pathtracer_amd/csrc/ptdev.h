@@ -109,6 +109,19 @@ __device__ __forceinline__ T ld_ro(const T* p) {
     return *(const __attribute__((address_space(4))) T*)p;
 }
 
+// The same for a whole record (a plain struct of 4-byte fields).
+template <typename T>
+__device__ __forceinline__ T ld_ro_rec(const T* p) {
+    static_assert(sizeof(T) % 4 == 0 && alignof(T) == 4, "4-byte fields");
+    uint32_t w[sizeof(T) / 4];
+    const __attribute__((address_space(4))) uint32_t* src = (const __attribute__((address_space(4))) uint32_t*)p;
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(T) / 4; ++i) w[i] = src[i];
+    T r;
+    __builtin_memcpy(&r, w, sizeof(T));
+    return r;
+}
+
 // Appends `pred` lanes of the calling wave to a queue whose length lives at
 // *counter: one atomic per wave (ballot + popcount), slot order = lane order.
 // Returns the slot for a predicated lane, -1 otherwise. Every active lane of

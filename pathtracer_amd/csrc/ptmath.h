@@ -256,6 +256,22 @@ PTM_FN float ptm_pow(float x, float y) {
     return (float)ptm__exp_d(t);
 }
 
+/* ptm_pow(x, n) for a whole n, from y = x^n by binary64 products (relative error
+ * below 1e-15). ptm_pow rounds a binary64 value of relative error below 1e-13
+ * (at most 5e-16 times its exponent |t| <= 104), so wherever y (1 - 1e-12) and
+ * y (1 + 1e-12) round to one binary32 value, that is ptm_pow's value too; the
+ * others (about one in 10^5) and x <= 0 or NaN take ptm_pow itself. About 10
+ * operations instead of the log and exp series' 60. */
+PTM_FN float ptm__pow_round(double y, float x, float n) {
+    float lo = (float)(y * (1.0 - 1e-12)), hi = (float)(y * (1.0 + 1e-12));
+    if (lo == hi && x > 0.0f) return hi;
+    return ptm_pow(x, n);
+}
+PTM_FN float ptm_pow_m5(float x) {
+    double d = (double)x, d2 = d * d;
+    return ptm__pow_round(1.0 / (d2 * d2 * d), x, -5.0f);
+}
+
 /* ---- acos ----------------------------------------------------------------------- */
 /* asin(z) for |z| <= 1/2: sum_n (2n)! / (4^n (n!)^2 (2n+1)) z^(2n+1), 30 terms. */
 PTM_FN double ptm__asin_series_d(double z) {

@@ -2,14 +2,16 @@
 // (src/shader.comp) as a wavefront of gfx950 kernels.
 //
 // The reference runs one invocation per pixel that loops over samples and
-// bounces (src/shader.comp:1393-1533). Here one wave holds pixels
-// [p0, p0 + pc) x samples [k0, k0 + m) as independent paths whose state lives
-// in SoA arrays; every bounce runs
-//     intersect (analytic closest hit) -> march<kind> (SDF sphere tracing)
-//     -> shade (emission, BRDF sampling, NEE setup, Russian roulette)
-//     -> shadow (closest-hit visibility with object-ID match) [-> march -> resolve]
-// over a compacted queue of live paths, appended with wave64 ballots. The
-// sequential PCG chain travels in the path state, so every path draws the
+// bounces (src/shader.comp:1393-1533). Here a dispatch is a set of independent
+// paths, pixels [p0, p0 + pc) x samples [k0, k0 + m), that one persistent kernel
+// traces from camera to end: a lane keeps its path in registers through all its
+// bounces (closest hit, shading, the shadow ray, Russian roulette) and takes the
+// next path from a queue when it ends, so nothing of a path goes through memory
+// but its XYZ, and lanes stay busy whatever the spread of path lengths. Sphere
+// tracing is a state of the lane: every marching lane of a wave takes one
+// distance evaluation per iteration, and the lanes that wait for shading, an
+// intersection or a new path do that together once enough of them wait.
+// The sequential PCG chain travels with the path, so every path draws the
 // same numbers in the same order as the shader, and each path's arithmetic is
 // the shader's (same operations, same order, ptmath.h built-ins). Radiance is
 // folded per pixel in sample order, so the texels match the reference method
@@ -17,12 +19,16 @@
 #include <algorithm>
 #include <cstring>
 #include <mutex>
+#include <utility>
 
 #include "tracer.hpp"
 
 namespace ptk {
 
 using namespace ptd;
+
+// in namespace ptk: the header holds device helpers only, no includes
+#include "wave_queue.h"
 
 constexpr float kPi = 3.14159265358979f;  // PI, src/shader.comp:9 (binary32)
 constexpr float kOneByThree = 0.3333333f; // ONEBYTHREE, src/shader.comp:10
@@ -55,15 +61,24 @@ __device__ __forceinline__ float spd(float l, float peak, float sig, int invert)
     float r = ptm_exp(-x * x);
     return ptm_mix(r, 1.0f - r, (float)invert);
 }
-__device__ __forceinline__ float planck(float l, float T) {
-    return (1.1910429724e-16f * ptm_pow(l, -5.0f)) / (ptm_exp(0.014387768775f / (l * T)) - 1.0f);
+// The reference's emitter at the path's wavelengths l (nm): Planck's law over
+// its Wien peak, times luminosity. pw holds the path's numerators
+// 1.19...e-16 (l 1e-9)^-5 and `peak` 4.09...e-6 T^5 of the light: binary64 powers
+// that the shader evaluates at every vertex (they were most of the shading
+// time), here taken once per path and per scene with the same operations.
+__device__ __forceinline__ f4 planck_numerators(f4 l) {
+    return f4{1.1910429724e-16f * ptm_pow_m5(l.x * 1e-9f), 1.1910429724e-16f * ptm_pow_m5(l.y * 1e-9f),
+              1.1910429724e-16f * ptm_pow_m5(l.z * 1e-9f), 1.1910429724e-16f * ptm_pow_m5(l.w * 1e-9f)};
 }
-__device__ __forceinline__ f4 emit(f4 l, float T, float lum) {
+PT_HD float wien_peak(float T) { return 4.0956746759e-6f * ptm_pow(fmaxf(T, 0.0f), 5.0f); }
+__device__ __forceinline__ float planck(float pw, float l, float T) {
+    return pw / (ptm_exp(0.014387768775f / (l * T)) - 1.0f);
+}
+__device__ __forceinline__ f4 emit(f4 pw, f4 l, float T, float lum, float peak) {
     float t = fmaxf(T, 0.0f);
-    float peak = 4.0956746759e-6f * ptm_pow(t, 5.0f);
     float L = fmaxf(lum, 0.0f);
-    return f4{(planck(l.x * 1e-9f, t) / peak) * L, (planck(l.y * 1e-9f, t) / peak) * L,
-              (planck(l.z * 1e-9f, t) / peak) * L, (planck(l.w * 1e-9f, t) / peak) * L};
+    return f4{(planck(pw.x, l.x * 1e-9f, t) / peak) * L, (planck(pw.y, l.y * 1e-9f, t) / peak) * L,
+              (planck(pw.z, l.z * 1e-9f, t) / peak) * L, (planck(pw.w, l.w * 1e-9f, t) / peak) * L};
 }
 __host__ __device__ __forceinline__ float bk7(float l) {
     l *= 1e-3f;
@@ -89,6 +104,12 @@ __device__ __forceinline__ void light_mix(const float* u, float id, float& T, fl
     if (idx == -1) { T = 5500.0f; lum = 0.0f; return; }
     T = ubo_at(u, kUboLight + 2 * idx);
     lum = ubo_at(u, kUboLight + 2 * idx + 1);
+}
+// wien_peak of light `id` (temperature T): from the scene's table, or computed
+// for an id outside it (a packed buffer may hold any number).
+__device__ __forceinline__ float light_peak(const RefSceneDev& S, float id, float T) {
+    const int idx = (int)id;
+    return idx >= 0 && idx < kRefLights ? S.peak[idx] : wien_peak(T);
 }
 __device__ __forceinline__ f4 brdf(f4 l, const RMat& m) {
     int inv = (int)m.invert;
@@ -329,26 +350,26 @@ __device__ bool hit_cyclide(f3 ro, f3 rd, const RefCyclide& C, Hit& h) {
 __device__ int closest_analytic(const RefSceneDev& S, f3 o, f3 d, Hit& h) {
     int id = -1, base = 0;
     for (int i = 0; i < S.ns; ++i)
-        if (hit_sphere(o, d, S.sph[i], h)) id = i;
+        if (hit_sphere(o, d, ld_ro_rec(S.sph + i), h)) id = i;
     base += S.ns;
     for (int i = 0; i < S.np; ++i)
-        if (hit_plane(o, d, S.pln[i], h)) id = base + i;
+        if (hit_plane(o, d, ld_ro_rec(S.pln + i), h)) id = base + i;
     base += S.np;
     for (int i = 0; i < S.nb; ++i) {
-        const RefBox& b = S.box[i];
+        const RefBox b = ld_ro_rec(S.box + i);
         if (!bounding_sphere(o, d, b.pos, b.bsr2)) continue;
         if (hit_box(o, d, b, h)) id = base + i;
     }
     base += S.nb;
     for (int i = 0; i < S.nl; ++i) {
-        const RefLens& L = S.lens[i];
+        const RefLens L = ld_ro_rec(S.lens + i);
         if (!bounding_sphere(o, d, L.pos, L.br2)) continue;
         int outside = 1;
         if (hit_lens(o, d, L, h, outside)) id = base + i;
     }
     base += S.nl;
     for (int i = 0; i < S.nc; ++i) {
-        const RefCyclide& C = S.cyc[i];
+        const RefCyclide C = ld_ro_rec(S.cyc + i);
         if (!bounding_sphere(o, d, C.pos, C.brad2)) continue;
         if (hit_cyclide(o, d, C, h)) id = base + i;
     }
@@ -356,18 +377,59 @@ __device__ int closest_analytic(const RefSceneDev& S, f3 o, f3 d, Hit& h) {
 }
 
 // ---- SDFs (sdfs/{mandelbulb,menger,blob,terrain}.glsl) -----------------------------
+// Correctly rounded quotient and square root for operands and results well
+// inside the normal range: the compiler's own refinement sequences without the
+// scaling and special-case instructions around them, which change nothing there
+// (8 instead of 11 instructions, 9 instead of 15).
+__device__ __forceinline__ float div_mid(float a, float b) {
+    const float y0 = __builtin_amdgcn_rcpf(b);
+    const float y = fmaf(fmaf(-b, y0, 1.0f), y0, y0);
+    float q = a * y;
+    q = fmaf(fmaf(-b, q, a), y, q);
+    return fmaf(fmaf(-b, q, a), y, q);
+}
+__device__ __forceinline__ float sqrt_mid(float x) {
+    const float s = __builtin_amdgcn_sqrtf(x);
+    const float lo = __uint_as_float(__float_as_uint(s) - 1u), hi = __uint_as_float(__float_as_uint(s) + 1u);
+    const float r = fmaf(-lo, s, x) <= 0.0f ? lo : s;
+    return fmaf(-hi, s, x) > 0.0f ? hi : r;
+}
+// One iteration's terms that need rounding care: r^7, 1 / r, 1 / l and sin(phi)
+// from r = |z| and l2 = x^2 + z^2, as ptm_pow, the divisions and the square root
+// of the shader's expressions give them. In the middle of the range (all but
+// points far outside or on the polar axis) without special cases: a march is a
+// chain of hundreds of these iterations, and its length in instructions is what
+// the longest paths of a launch cost. r^7 in binary64 has its ptm_pow value
+// unless it lies within 2^-40 of a binary32 rounding boundary (ptm__pow_round):
+// the 29 bits that rounding drops are then near 2^28.
+__device__ __forceinline__ void mandelbulb_terms(float r, float l2, float& r7, float& invr, float& invl, float& sinp) {
+    if (r >= 0x1p-16f && r <= 0x1p16f && l2 >= 0x1p-80f) {
+        const double d = (double)r, d2 = d * d, d3 = d2 * d, y = d3 * d3 * d;
+        r7 = (float)y;
+        const uint32_t dropped = (uint32_t)ptm_d2u(y) & 0x1fffffffu;
+        if (dropped - (0x10000000u - 8192u) <= 2u * 8192u) r7 = (float)ptm__exp_d(7.0 * ptm__log_d(d));  // ptm_pow
+        invr = div_mid(1.0f, r);
+        invl = div_mid(1.0f, sqrt_mid(l2));
+        sinp = div_mid(invr, invl);
+    } else {
+        r7 = ptm_pow(r, 7.0f);
+        invr = 1.0f / r;
+        invl = ptm_rsqrt(l2);
+        sinp = invr / invl;
+    }
+}
 __device__ __forceinline__ float de_mandelbulb(f3 p, int iters, float bailout) {
     f3 z = p;
     float r = length(z);
     float dr = 1.0f;
     for (int i = 0; i < iters; ++i) {
-        dr = 8.0f * ptm_pow(r, 7.0f) * dr + 1.0f;
-        float invr = 1.0f / r;
-        float invl = ptm_rsqrt(z.x * z.x + z.z * z.z);
+        float r7, invr, invl, sinp;
+        mandelbulb_terms(r, z.x * z.x + z.z * z.z, r7, invr, invl, sinp);
+        dr = 8.0f * r7 * dr + 1.0f;
         r *= r;
         r *= r;
         r *= r;
-        float cost = z.z * invl, cosp = z.y * invr, sint = z.x * invl, sinp = invr / invl;
+        float cost = z.z * invl, cosp = z.y * invr, sint = z.x * invl;
         float ct2 = cost * cost, cp2 = cosp * cosp;
         float cost8 = fmaf(fmaf(fmaf(fmaf(128.0f, ct2, -256.0f), ct2, 160.0f), ct2, -32.0f), ct2, 1.0f);
         float cosp8 = fmaf(fmaf(fmaf(fmaf(128.0f, cp2, -256.0f), cp2, 160.0f), cp2, -32.0f), cp2, 1.0f);
@@ -375,7 +437,9 @@ __device__ __forceinline__ float de_mandelbulb(f3 p, int iters, float bailout) {
         float sinp8 = fmaf(fmaf(fmaf(128.0f, cp2, -192.0f), cp2, 80.0f), cp2, -8.0f) * sinp * cosp;
         z = r * mk3(sint8 * sinp8, cosp8, cost8 * sinp8);
         z = z + p;
-        r = length(z);
+        const float r2 = dot(z, z);
+        r = sqrt_mid(r2);
+        if (!(r2 >= 0x1p-80f && r2 <= 0x1p80f)) r = sqrtf(r2);
         if (r > bailout) break;
     }
     return 0.5f * ptm_log(r) * r / dr;
@@ -431,12 +495,12 @@ __device__ __forceinline__ float terrain_height(float x) {
 }
 __device__ __forceinline__ float de_terrain(f3 p) { return p.y - (terrain_height(p.x) + terrain_height(p.z)); }
 
+// Distance to an SDF of `kind` (KIND when it is known at compile time).
 template <int KIND>
-__device__ __forceinline__ float de_eval(const pt_sdf_desc& d, f3 p) {
-    const int kind = KIND ? KIND : d.kind;
-    switch (kind) {
-        case PT_SDF_MANDELBULB: return de_mandelbulb(p, d.iterations, d.bailout);
-        case PT_SDF_MENGER: return de_menger(p, d.iterations);
+__device__ __forceinline__ float de_eval(int kind, int iterations, float bailout, f3 p) {
+    switch (KIND ? KIND : kind) {
+        case PT_SDF_MANDELBULB: return de_mandelbulb(p, iterations, bailout);
+        case PT_SDF_MENGER: return de_menger(p, iterations);
         case PT_SDF_BLOB: return de_blob(p);
         case PT_SDF_TERRAIN: return de_terrain(p);
         default: return kMaxDist;
@@ -457,40 +521,15 @@ __device__ __forceinline__ float sdf_material(const pt_sdf_desc& d, f3 p) {
     return d.material[0];
 }
 
-// The spliced SDF(): min over the SDFs of the set (src/pathtracer.cpp:2004-2054).
-template <int KIND>
-__device__ __forceinline__ float sdf_set(const RefSceneDev& S, f3 p, uint32_t set, unsigned& steps) {
-    float s = kMaxDist;
-    for (int i = 0; i < S.nsdf; ++i) {
-        uint32_t code = 1u << (uint32_t)i;
-        if ((set & code) == code) s = fminf(s, de_eval<KIND>(S.sdf[i].d, p - S.sdf[i].pos));
-    }
-    ++steps;
-    return s;
-}
-// The spliced SDFMATERIAL(): material of the nearest SDF, ties to the later one.
-template <int KIND>
-__device__ float sdf_set_material(const RefSceneDev& S, f3 p, uint32_t set) {
-    float s = kMaxDist, m = 0.0f;
-    for (int i = 0; i < S.nsdf; ++i) {
-        uint32_t code = 1u << (uint32_t)i;
-        if ((set & code) == code) {
-            f3 q = p - S.sdf[i].pos;
-            float di = de_eval<KIND>(S.sdf[i].d, q);
-            m = (s < di) ? m : sdf_material(S.sdf[i].d, q);
-            s = fminf(s, di);
-        }
-    }
-    return m;
-}
 // SearchSDF (src/shader.comp:732-777).
 __device__ bool search_sdf(const RefSceneDev& S, f3 p, f3 invdir, float& tmn, float& tmx, uint32_t& set) {
     bool found = false;
     set = 0;
     for (int i = 0; i < S.nsdf; ++i) {
-        f3 lo = p - S.sdf[i].pos;
-        f3 t0 = fma3(S.sdf[i].size, mk3(-0.5f, -0.5f, -0.5f), -lo) * invdir;
-        f3 t1 = fma3(S.sdf[i].size, mk3(0.5f, 0.5f, 0.5f), -lo) * invdir;
+        const f3 pos = ld_ro_rec(&S.sdf[i].pos), size = ld_ro_rec(&S.sdf[i].size);
+        f3 lo = p - pos;
+        f3 t0 = fma3(size, mk3(-0.5f, -0.5f, -0.5f), -lo) * invdir;
+        f3 t1 = fma3(size, mk3(0.5f, 0.5f, 0.5f), -lo) * invdir;
         f3 a = min3(t0, t1), b = max3(t0, t1);
         float bx = fmaxf(fmaxf(a.x, a.y), a.z);
         float by = fminf(fminf(b.x, b.y), b.z);
@@ -510,67 +549,141 @@ __device__ bool search_sdf(const RefSceneDev& S, f3 p, f3 invdir, float& tmn, fl
     return found;
 }
 // SphereTracing (src/shader.comp:779-860): over-relaxed sphere tracing after
-// Keinert et al., "Enhanced Sphere Tracing" (2014).
-template <int KIND>
-__device__ bool sphere_trace(const RefSceneDev& S, f3 o, f3 d, Hit& h, unsigned& steps) {
-    float t = 1e-3f, insT = 0.0f;
-    const float omegaMax = 1.70f, omegaSpeed = 0.20f;
-    float omega = omegaMax, prev = 0.0f;
-    f3 p = o;
+// Keinert et al., "Enhanced Sphere Tracing" (2014), one distance evaluation at a
+// time: `q` is the next point whose distance the march needs, and march_advance
+// takes it. A lane's march lasts from 1 to over 512 evaluations, so marching to
+// the end in one loop ran at the pace of the wave's longest ray.
+enum : int {
+    MP_SIGN = 0,      // the distance at the origin (its sign)
+    MP_STEP = 1,      // a step of the march
+    MP_NORMAL = 2,    // 2..7: the six differences of the normal
+    MP_MATERIAL = 8,  // the material of the nearest SDF
+};
+struct March {
+    f3 q;
+    float t, insT, omega, prev, k, tmx;
+    uint32_t set;
+    int points, i, phase;
+};
+// Starts the march of the ray (o, d); false when it enters no SDF's box.
+__device__ __forceinline__ bool march_start(const RefSceneDev& S, f3 o, f3 d, March& M) {
     f3 invdir = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-    int points = 0;
     float tmn = kMaxDist, tmx = kMaxDist;
-    uint32_t set = 0;
-    if (!search_sdf(S, p, invdir, tmn, tmx, set)) return false;
-    t = fmaxf(tmn, t);
-    p = fma3s(d, t, o);
-    float k = ptm_sign(sdf_set<KIND>(S, o, set, steps));
-    for (int i = 0; i < 512; ++i) {
-        float rad = sdf_set<KIND>(S, p, set, steps);
-        if (insT > (fabsf(prev) + fabsf(rad))) {
-            t -= insT;
-            omega = 1.0f;
-            insT = prev * omega * k;
-            t += insT;
-            p = fma3s(d, t, o);
-            continue;
+    if (!search_sdf(S, o, invdir, tmn, tmx, M.set)) return false;
+    M.t = fmaxf(tmn, 1e-3f);
+    M.tmx = tmx;
+    M.insT = 0.0f;
+    M.omega = 1.70f;
+    M.prev = 0.0f;
+    M.k = 0.0f;
+    M.points = 0;
+    M.i = 0;
+    M.phase = MP_SIGN;
+    M.q = o;
+    return true;
+}
+// The spliced SDF() at M.q: min over the SDFs of the set (src/pathtracer.cpp:
+// 2004-2054). With `want_mat` also SDFMATERIAL(): the material of the nearest SDF,
+// ties to the later one.
+template <int KIND>
+__device__ __forceinline__ float sdf_set(const RefSceneDev& S, f3 p, uint32_t set, bool want_mat, float& mat) {
+    float s = kMaxDist, m = 0.0f;
+    for (int i = 0; i < S.nsdf; ++i) {
+        uint32_t code = 1u << (uint32_t)i;
+        if ((set & code) == code) {
+            const f3 q = p - ld_ro_rec(&S.sdf[i].pos);
+            const pt_sdf_desc& desc = S.sdf[i].d;
+            const int kind = KIND ? KIND : ld_ro(&desc.kind);
+            const float di = de_eval<KIND>(kind, ld_ro(&desc.iterations), ld_ro(&desc.bailout), q);
+            if (want_mat) m = (s < di) ? m : sdf_material(desc, q);
+            s = fminf(s, di);
         }
-        if (fabsf(rad) < 1e-4f) break;
-        if (t > tmx) points += 1;
-        else points = 0;
-        if (points >= 2) {
-            t = tmx + 1e-3f;
-            tmn = kMaxDist;
-            tmx = kMaxDist;
-            if (search_sdf(S, fma3s(d, t, o), invdir, tmn, tmx, set)) {
-                tmn += t;
-                tmx += t;
-                t = fmaxf(tmn, t);
-                p = fma3s(d, t, o);
-                continue;
+    }
+    mat = m;
+    return s;
+}
+// Takes the distance v at M.q. Returns 0 while the march (or its normal and
+// material) needs another one, 1 when the ray hits nothing before h.t, 2 at a
+// hit. SHADOW rays need only the fact of the hit: the six distances the method
+// evaluates for its normal are counted in `steps` but not evaluated.
+template <bool SHADOW>
+__device__ __forceinline__ int march_advance(const RefSceneDev& S, f3 o, f3 d, March& M, float v, float mat, Hit& h,
+                                             unsigned& steps) {
+    const float omegaMax = 1.70f, omegaSpeed = 0.20f;
+    if (M.phase == MP_STEP) {
+        ++steps;
+        const float rad = v;
+        bool end = false;
+        if (M.insT > (fabsf(M.prev) + fabsf(rad))) {
+            M.t -= M.insT;
+            M.omega = 1.0f;
+            M.insT = M.prev * M.omega * M.k;
+            M.t += M.insT;
+        } else if (fabsf(rad) < 1e-4f) {
+            end = true;
+        } else {
+            if (M.t > M.tmx) M.points += 1;
+            else M.points = 0;
+            if (M.points >= 2) {
+                M.t = M.tmx + 1e-3f;
+                float tmn = kMaxDist;
+                M.tmx = kMaxDist;
+                const f3 invdir = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+                if (!search_sdf(S, fma3s(d, M.t, o), invdir, tmn, M.tmx, M.set)) return 1;
+                tmn += M.t;
+                M.tmx += M.t;
+                M.t = fmaxf(tmn, M.t);
+            } else {
+                M.insT = rad * M.omega * M.k;
+                M.t += M.insT;
+                float f = fminf(rad / M.prev, 0.99f);
+                M.omega += omegaSpeed * (fminf(1.0f / (1.0f - f), omegaMax) - M.omega);
+                M.prev = rad;
             }
-            return false;
         }
-        insT = rad * omega * k;
-        t += insT;
-        p = fma3s(d, t, o);
-        float f = fminf(rad / prev, 0.99f);
-        omega += omegaSpeed * (fminf(1.0f / (1.0f - f), omegaMax) - omega);
-        prev = rad;
+        M.q = fma3s(d, M.t, o);
+        if (!end && ++M.i < 512) return 0;
+        // converged, or out of steps: a hit when nearer than the analytic one
+        if (!(M.t < h.t)) return 1;
+        h.t = M.t - 1e-3f;
+        if (SHADOW) {
+            steps += 6;
+            return 2;
+        }
+    } else if (M.phase == MP_SIGN) {
+        ++steps;
+        M.k = ptm_sign(v);
+        M.q = fma3s(d, M.t, o);
+        M.phase = MP_STEP;
+        return 0;
+    } else {
+        // the distance at the hit point displaced along an axis: + then -
+        switch (M.phase) {
+            case MP_NORMAL + 0: h.n.x = v; break;
+            case MP_NORMAL + 1: h.n.x -= v; break;
+            case MP_NORMAL + 2: h.n.y = v; break;
+            case MP_NORMAL + 3: h.n.y -= v; break;
+            case MP_NORMAL + 4: h.n.z = v; break;
+            case MP_NORMAL + 5: h.n.z -= v; break;
+            default:
+                h.mat = mat;
+                h.light = -1.0f;
+                h.n = normalize(h.n);
+                return 2;
+        }
+        ++steps;
     }
-    if (t < h.t) {
-        h.t = t - 1e-3f;
-        p = fma3s(d, t, o);
-        const float e = 1e-4f;
-        f3 n = mk3(sdf_set<KIND>(S, p + mk3(e, 0.0f, 0.0f), set, steps) - sdf_set<KIND>(S, p - mk3(e, 0.0f, 0.0f), set, steps),
-                   sdf_set<KIND>(S, p + mk3(0.0f, e, 0.0f), set, steps) - sdf_set<KIND>(S, p - mk3(0.0f, e, 0.0f), set, steps),
-                   sdf_set<KIND>(S, p + mk3(0.0f, 0.0f, e), set, steps) - sdf_set<KIND>(S, p - mk3(0.0f, 0.0f, e), set, steps));
-        h.n = normalize(n);
-        h.mat = sdf_set_material<KIND>(S, p, set);
-        h.light = -1.0f;
-        return true;
+    ++M.phase;  // the normal's first difference after the march, else the next one, then the material
+    const f3 p = fma3s(d, M.t, o);
+    M.q = p;
+    if (M.phase < MP_MATERIAL) {
+        // p + e and p - e along one axis; the other components add a zero of e's
+        // sign, which is what the vector sum and difference do
+        const int k = M.phase - MP_NORMAL;
+        const float e = (k & 1) ? -1e-4f : 1e-4f, z = copysignf(0.0f, e);
+        M.q = p + mk3((k >> 1) == 0 ? e : z, (k >> 1) == 1 ? e : z, (k >> 1) == 2 ? e : z);
     }
-    return false;
+    return 0;
 }
 
 // ---- sampling (src/shader.comp:976-1028, 1093-1119, 1225-1296) ----------------------
@@ -646,29 +759,34 @@ __device__ int sample_light(const RefSceneDev& S, uint32_t& seed, float& brad, f
 }
 
 // ---- kernels ---------------------------------------------------------------------------
-__global__ void k_ref_counts(int* counts, int c0, int c1, int c2) {
-    counts[0] = c0;
-    counts[1] = c1;
-    counts[2] = c2;
-}
-__global__ void k_ref_reset(int* counts, int which) {
-    counts[which] = 0;
-    counts[2] = 0;
+struct RefFinish {
+    int spf, currentSamples, frame, ISO;
+    float apSize, FPS, persistence;
+};
+// Exposure and Accumulate into the texel buffer (src/shader.comp:1492-1532):
+// `sum` is the sum over the dispatch's samples, tx the texel before it.
+__device__ __forceinline__ float4 finish_texel(const RefFinish& F, f3 sum, float4 tx) {
+    f3 out = sum / (float)F.spf;
+    out = out * (F.apSize * F.apSize * (float)F.ISO);
+    f3 in = mk3(tx.x, tx.y, tx.z);
+    if (F.currentSamples == F.spf && F.frame > F.spf) {
+        float wgt = ptm_pow(2.0f, -8.0f / (F.FPS * F.persistence));
+        out = (1.0f - wgt) * out + wgt * in;
+    } else {
+        int u = F.currentSamples / F.spf;
+        out = ((float)(u - 1) * in + out) / (float)u;
+    }
+    return make_float4(out.x, out.y, out.z, 1.0f);
 }
 
-// Camera rays: Rendering + Scene up to TracePath (src/shader.comp:1446-1476, 1509-1516).
-__global__ void __launch_bounds__(kBlock) k_ref_raygen(RefFrame F, RefWave Wv) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    int n = F.pc * F.m;
-    if (i == 0) atomicAdd(&Wv.stats[3], (unsigned long long)n);
-    if (i >= n) return;
-    int pix = F.p0 + i % F.pc;
-    int k = F.k0 + i / F.pc;
+// Camera ray of sample k of pixel `pix`: Rendering + Scene up to TracePath
+// (src/shader.comp:1446-1476, 1509-1516).
+__device__ __forceinline__ void camera_ray(const RefFrame& F, int pix, int k, f3& o, f3& d, uint32_t& seed, float& lh) {
     int gx = pix % F.W, gy = pix / F.W;
     uint32_t x = (uint32_t)gx, y = (uint32_t)(F.H - gy);
     float uvx = (2.0f * (float)x - (float)F.W) / (float)F.H;
     float uvy = (2.0f * (float)y - (float)F.H) / (float)F.H;
-    uint32_t seed = pcg((uint32_t)(F.frame - F.spf + k));
+    seed = pcg((uint32_t)(F.frame - F.spf + k));
     seed += x + (uint32_t)F.W * y;
     float jx = 2.0f * rand_chain(seed) - 0.5f;
     float jy = 2.0f * rand_chain(seed) - 0.5f;
@@ -677,15 +795,15 @@ __global__ void __launch_bounds__(kBlock) k_ref_raygen(RefFrame F, RefWave Wv) {
     float sc = -F.camSize * 0.5f;
     uvx *= sc;
     uvy *= sc;
-    f3 o = F.camPos + vmul(mk3(uvx, uvy, 0.0f), F.camM);
+    o = F.camPos + vmul(mk3(uvx, uvy, 0.0f), F.camM);
     float ux = rand_chain(seed), uy = rand_chain(seed);
     float phi = 2.0f * kPi * uy;
     float dr = sqrtf(ux);
     float dsx = dr * ptm_cos(phi), dsy = dr * ptm_sin(phi);
     float ap = 0.5f * F.apSize;
     f3 onAp = F.camPos + vmul(mk3(ap * dsx, ap * dsy, F.apDist), F.camM);
-    f3 d = normalize(onAp - o);
-    float lh = ptm_mix(360.0f, 800.0f, rand_chain(seed));
+    d = normalize(onAp - o);
+    lh = ptm_mix(360.0f, 800.0f, rand_chain(seed));
     // TracePathLens: two refractions through the BK7 bi-convex lens at the hero wavelength.
     float l = lh;
     for (int pass = 0; pass < 2; ++pass) {
@@ -704,245 +822,282 @@ __global__ void __launch_bounds__(kBlock) k_ref_raygen(RefFrame F, RefWave Wv) {
         o = fma3s(d, h.t, o);
         d = refract(d, h.n, n12);
     }
-    Wv.ox[i] = o.x; Wv.oy[i] = o.y; Wv.oz[i] = o.z;
-    Wv.dx[i] = d.x; Wv.dy[i] = d.y; Wv.dz[i] = d.z;
-    Wv.seed[i] = seed;
-    Wv.lh[i] = lh;
-    Wv.T[i] = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
-    Wv.L[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    Wv.w[i] = 1.0f;
-    Wv.q[0][i] = i;
 }
 
-// Closest analytic hit of every live path (Intersection without SphereTracing).
-__global__ void __launch_bounds__(kBlock) k_ref_intersect(RefSceneDev S, RefWave Wv, int cur) {
-    int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    int n = Wv.counts[cur];
-    if (idx == 0) atomicAdd(&Wv.stats[0], (unsigned long long)n);
-    if (idx >= n) return;
-    int p = Wv.q[cur][idx];
-    f3 o = mk3(Wv.ox[p], Wv.oy[p], Wv.oz[p]);
-    f3 d = mk3(Wv.dx[p], Wv.dy[p], Wv.dz[p]);
+// XYZ of a finished path (src/shader.comp:1477-1487); NaN samples become zero.
+__device__ __forceinline__ f3 path_xyz(const RefSceneDev& S, f4 l, f4 L, unsigned& nans) {
+    f3 X0 = wave_to_xyz(S.ubo, l.x), X1 = wave_to_xyz(S.ubo, l.y);
+    f3 X2 = wave_to_xyz(S.ubo, l.z), X3 = wave_to_xyz(S.ubo, l.w);
+    f3 col = L.x * X0 + L.y * X1 + L.z * X2 + L.w * X3;
+    col = mk3(0.0f, 0.0f, 0.0f) + (col * (720.0f - 390.0f)) * 0.25f;
+    if (col.x != col.x || col.y != col.y || col.z != col.z) {
+        col = mk3(0.0f, 0.0f, 0.0f);
+        ++nans;
+    }
+    return col;
+}
+
+// A lane's state in k_ref_path, what it does next.
+enum : int {
+    PS_IDLE,    // takes a path from the queue
+    PS_RAY,     // its extension ray is to be intersected
+    PS_SHADE,   // its hit is known
+    PS_SHADOW,  // the visibility of its light sample is known
+    PS_DONE,    // its path has ended and is to be stored
+    PS_MARCH,   // sphere tracing, extension or shadow ray
+};
+// When a wave with marching lanes does the scene work (a new path, an intersection,
+// shading) of the others: once kRefScene lanes wait for it, or as many as march (16
+// to 40 measured within the runs' spread on the 512 x 512 x 4 mandelbulb scene, 8
+// slower by 10 %). Ended lanes before they are stored and refilled: kRefRefill (the
+// 1080p analytic scene, ms for 8 samples: 8 -> 3.4, 16 -> 3.1, 24 and 32 -> 2.8,
+// 48 -> 2.9, 64 -> 3.5).
+constexpr int kRefScene = 24;
+constexpr int kRefRefillSdf = 16, kRefRefill = 32;
+constexpr int kRefLanes = 64;  // threads per block: one wave, so that few paths spread over all compute units
+
+// The path tracer, persistent: see the head of this file. KIND: -1 for scenes
+// without SDF objects, PT_SDF_* when all are of one kind, 0 when they are mixed.
+// It replaced a kernel per stage and bounce (36 launches for a frame of 5 bounces,
+// path records of 168 bytes in memory between them, one ray per lane in the
+// marches) and is bound by VALU issue in analytic scenes (rocprofv3: saturated, 34 of
+// 64 lanes active, about 1650 instructions of a lane per segment with its shading and
+// shadow ray): 1280x720x1 5 bounces 966 -> 230 us, 1920x1080x8 8 bounces 15.8 ->
+// 2.8 ms, 150x101x1 288 -> 81 us of kernels (one launch, its length the chain of a
+// path's bounces). SDF scenes are bound by the chain of their longest path (512x512x4
+// mandelbulb: up to 728 distance evaluations of 8 iterations, about 3.8 us each):
+// 29.2 -> 5.7 ms. Registers: 165 (analytic) and 191 (SDF) leave 3 and 2 waves per SIMD;
+// asking for 4 spills and was 20 % slower, and the path state in LDS while marching gave
+// nothing.
+// `direct`: the dispatch has one sample per pixel, all in this wave, and the
+// paths' texels are finished here instead of by k_ref_fold.
+template <int KIND>
+__global__ void __launch_bounds__(kRefLanes) k_ref_path(RefSceneDev S, RefFrame F, RefWave Wv, RefFinish Fin,
+                                                         float4* texels, int direct, int count_dispatch) {
+    constexpr bool SDF = KIND >= 0;
+    const int n = F.pc * F.m;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        atomicAdd(&Wv.stats[3], (unsigned long long)n);
+        if (count_dispatch) atomicAdd(&Wv.stats[5], 1ull);
+    }
+    unsigned segments = 0, shadows = 0, steps = 0, nans = 0;
+    // the path: index, bounce, next extension ray, RNG, wavelengths, Planck
+    // numerators, throughput, radiance, MIS weight of the next emitter hit
+    int st = PS_IDLE, p = 0, bounce = 0;
+    f3 o = mk3(0.0f, 0.0f, 0.0f), d = o;
+    uint32_t seed = 0;
+    f4 l = mk4(0.0f), pw = l, T = l, L = l;
+    float w = 1.0f;
     Hit h;
-    h.t = kMaxDist;
-    h.n = mk3(0.0f, 0.0f, 0.0f);
+    h.t = 0.0f;
+    h.n = o;
     h.mat = 0.0f;
     h.light = -1.0f;
-    closest_analytic(S, o, d, h);
-    Wv.ht[p] = h.t;
-    Wv.hnx[p] = h.n.x; Wv.hny[p] = h.n.y; Wv.hnz[p] = h.n.z;
-    Wv.hmat[p] = h.mat;
-    Wv.hlight[p] = h.light;
-}
-
-// SphereTracing of the extension rays against the current closest hit.
-template <int KIND>
-__global__ void __launch_bounds__(kBlock) k_ref_march(RefSceneDev S, RefWave Wv, int cur) {
-    int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    int n = Wv.counts[cur];
-    unsigned steps = 0;
-    if (idx < n) {
-        int p = Wv.q[cur][idx];
-        f3 o = mk3(Wv.ox[p], Wv.oy[p], Wv.oz[p]);
-        f3 d = mk3(Wv.dx[p], Wv.dy[p], Wv.dz[p]);
-        Hit h;
-        h.t = Wv.ht[p];
-        if (sphere_trace<KIND>(S, o, d, h, steps)) {
-            Wv.ht[p] = h.t;
-            Wv.hnx[p] = h.n.x; Wv.hny[p] = h.n.y; Wv.hnz[p] = h.n.z;
-            Wv.hmat[p] = h.mat;
-            Wv.hlight[p] = h.light;
+    // the light sample: direction, contribution, light object, nearest analytic
+    // object and its distance; whether the path goes on after it
+    f3 sd = o;
+    f4 contrib = l;
+    int lobj = 0, sid = 0;
+    float st_t = 0.0f;
+    bool cont = false, shadow_ray = false;
+    March M{};
+    // The queue holds blocks of 64 consecutive paths, dealt to its segments in turn
+    // (entry block e of segment s is path block e * segments + s), so that each
+    // segment, which only its own waves drain, holds a share of every part of the
+    // image; entries past the last path are dropped.
+    const int nseg = min(kSeg, (int)gridDim.x);
+    const int seg_blocks = ((n + 63) / 64 + nseg - 1) / nseg;
+    WaveChunk chunk = wave_chunk_init(Wv.cursor, seg_blocks * nseg * 64);
+    while (true) {
+        bool scene = true;
+        if (SDF) {
+            const int marching = (int)__popcll(__ballot(st == PS_MARCH));
+            const int waiting = (int)__popcll(__ballot(st != PS_MARCH && !(st == PS_IDLE && chunk.drained())));
+            scene = waiting >= min(kRefScene, max(marching, 1)) || marching == 0;
         }
-    }
-    wave_add_u64(stat_slot(Wv.stats, 2), steps);
-}
-
-// TraceRay after the hit (src/shader.comp:1352-1391) with SampleLightSource
-// (src/shader.comp:1298-1343) up to the visibility test.
-__global__ void __launch_bounds__(kBlock) k_ref_shade(RefSceneDev S, RefFrame F, RefWave Wv, int cur, int bounce) {
-    const int nxt = cur ^ 1;
-    int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    int n = Wv.counts[cur];
-    bool active = idx < n;
-    bool shadow = false, cont = false;
-    int p = 0, lobj = 0;
-    f3 no = mk3(0.0f, 0.0f, 0.0f), sd = no;
-    f4 contrib = mk4(0.0f);
-    if (active) {
-        p = Wv.q[cur][idx];
-        float t = Wv.ht[p];
-        float4 Tv = Wv.T[p];
-        f4 T = f4{Tv.x, Tv.y, Tv.z, Tv.w};
-        float w = Wv.w[p];
-        uint32_t seed = Wv.seed[p];
-        f4 l = sample_wavelengths(Wv.lh[p]);
-        RMat mat = material_mix(S.ubo, Wv.hmat[p]);
-        float LT, LL;
-        light_mix(S.ubo, Wv.hlight[p], LT, LL);
-        if (t < kMaxDist) {
-            if (LL > 0.0f) {
-                f4 e = emit(l, LT, LL) * T * w;
-                float4 Lp = Wv.L[p];
-                Wv.L[p] = make_float4(Lp.x + e.x, Lp.y + e.y, Lp.z + e.z, Lp.w + e.w);
-            } else {
-                f3 o = mk3(Wv.ox[p], Wv.oy[p], Wv.oz[p]);
-                f3 d = mk3(Wv.dx[p], Wv.dy[p], Wv.dz[p]);
-                f3 nrm = mk3(Wv.hnx[p], Wv.hny[p], Wv.hnz[p]);
-                no = fma3s(d, t, o);
-                f3 nd = normalize(nrm + sample_unit_sphere(seed));
-                float pdf = dot(nd, nrm) / kPi;
-                if (S.numLights > 0.0f) {
-                    float brad = 0.0f, lid = -1.0f;
-                    f3 lpos = mk3(0.0f, 0.0f, 0.0f);
-                    lobj = sample_light(S, seed, brad, lpos, lid);
-                    float invd = 1.0f / length(lpos - no);
-                    f3 ldir = (lpos - no) * invd;
-                    float sinMax = fminf(brad * invd, 1.0f);
-                    float cosMax = sqrtf(1.0f - sinMax * sinMax);
-                    sd = to_world(sample_cone(seed, cosMax), ldir);
-                    float lpdf = 1.0f / S.numLights;
-                    lpdf *= dot(sd, ldir) / (kPi * (1.0f - cosMax * cosMax));
-                    w = mis2(pdf, lpdf);
-                    float ct = dot(sd, nrm);
-                    float death = 1.25f * fmaxf(w - 0.2f, 0.0f);
-                    if (ct >= 0.0f) {
-                        if (rand_chain(seed) > death) {
-                            float T2, L2;
-                            light_mix(S.ubo, lid, T2, L2);
-                            f4 f = brdf(l, mat);
-                            f4 g = f4{f.x * ct / lpdf, f.y * ct / lpdf, f.z * ct / lpdf, f.w * ct / lpdf};
-                            contrib = emit(l, T2, L2) * (T * g) * (1.0f - w);
-                            shadow = true;
-                        } else {
-                            w = 1.0f;
-                        }
+        if (scene) {
+            if (SDF && st == PS_SHADOW) {
+                if (sid == lobj) L = f4{L.x + contrib.x, L.y + contrib.y, L.z + contrib.z, L.w + contrib.w};
+                st = cont ? PS_RAY : PS_DONE;
+            }
+            const bool free_lane = st == PS_IDLE || st == PS_DONE;
+            const uint64_t idle = __ballot(free_lane);
+            if (__popcll(idle) >= (SDF ? kRefRefillSdf : kRefRefill) || idle == __ballot(st != PS_MARCH)) {
+                if (st == PS_DONE) {
+                    const f3 c = path_xyz(S, l, L, nans);
+                    if (direct) {
+                        // the sum over samples starts from zero (src/shader.comp:1513-1516)
+                        const f3 sum = mk3(0.0f, 0.0f, 0.0f) + c;
+                        texels[F.p0 + p] = finish_texel(Fin, sum, texels[F.p0 + p]);
+                    } else {
+                        Wv.col[p] = make_float4(c.x, c.y, c.z, 0.0f);
                     }
-                } else {
-                    w = mis2(pdf, 0.0f);
+                    st = PS_IDLE;
                 }
-                float ct = dot(nd, nrm);
-                f4 f = brdf(l, mat);
-                T = T * f4{f.x * ct / pdf, f.y * ct / pdf, f.z * ct / pdf, f.w * ct / pdf};
-                float pr = ptm_clamp(fmaxf(T.x, fmaxf(T.y, fmaxf(T.z, T.w))), 0.0f, 0.99f);
-                if (!(rand_chain(seed) > pr)) {
-                    T = T * (1.0f / pr);
-                    Wv.ox[p] = no.x; Wv.oy[p] = no.y; Wv.oz[p] = no.z;
-                    Wv.dx[p] = nd.x; Wv.dy[p] = nd.y; Wv.dz[p] = nd.z;
-                    cont = bounce + 1 < F.pathLength;
+                if (!chunk.drained()) {
+                    const int e = wave_refill(idle, chunk);
+                    const int b = e >> 6;
+                    const int path = ((b % seg_blocks) * nseg + b / seg_blocks) * 64 + (e & 63);
+                    if (e >= 0 && path < n) {
+                        p = path;
+                        float lh;
+                        camera_ray(F, F.p0 + p % F.pc, F.k0 + p / F.pc, o, d, seed, lh);
+                        l = sample_wavelengths(lh);
+                        pw = planck_numerators(l);
+                        T = mk4(1.0f);
+                        L = mk4(0.0f);
+                        w = 1.0f;
+                        bounce = 0;
+                        st = F.pathLength > 0 ? PS_RAY : PS_DONE;
+                    }
                 }
-                Wv.T[p] = make_float4(T.x, T.y, T.z, T.w);
-                Wv.w[p] = w;
-                Wv.seed[p] = seed;
+                if (chunk.drained() && __ballot(st != PS_IDLE) == 0ull) break;
+            }
+            // closest analytic hit (Intersection without SphereTracing)
+            if (st == PS_RAY) {
+                ++segments;
+                h.t = kMaxDist;
+                h.n = mk3(0.0f, 0.0f, 0.0f);
+                h.mat = 0.0f;
+                h.light = -1.0f;
+                closest_analytic(S, o, d, h);
+                st = PS_SHADE;
+                if (SDF && march_start(S, o, d, M)) {
+                    shadow_ray = false;
+                    st = PS_MARCH;
+                }
+            }
+            // TraceRay after the hit (src/shader.comp:1352-1391) with SampleLightSource
+            // (src/shader.comp:1298-1343)
+            if (st == PS_SHADE) {
+                st = PS_DONE;
+                bool shadow = false;
+                if (h.t < kMaxDist) {
+                    float LT, LL;
+                    light_mix(S.ubo, h.light, LT, LL);
+                    if (LL > 0.0f) {
+                        f4 e = emit(pw, l, LT, LL, light_peak(S, h.light, LT)) * T * w;
+                        L = f4{L.x + e.x, L.y + e.y, L.z + e.z, L.w + e.w};
+                    } else {
+                        const RMat mat = material_mix(S.ubo, h.mat);
+                        const f4 f = brdf(l, mat);
+                        const f3 nrm = h.n;
+                        const f3 no = fma3s(d, h.t, o);
+                        f3 nd = normalize(nrm + sample_unit_sphere(seed));
+                        float pdf = dot(nd, nrm) / kPi;
+                        if (S.numLights > 0.0f) {
+                            float brad = 0.0f, lid = -1.0f;
+                            f3 lpos = mk3(0.0f, 0.0f, 0.0f);
+                            lobj = sample_light(S, seed, brad, lpos, lid);
+                            float invd = 1.0f / length(lpos - no);
+                            f3 ldir = (lpos - no) * invd;
+                            float sinMax = fminf(brad * invd, 1.0f);
+                            float cosMax = sqrtf(1.0f - sinMax * sinMax);
+                            sd = to_world(sample_cone(seed, cosMax), ldir);
+                            float lpdf = 1.0f / S.numLights;
+                            lpdf *= dot(sd, ldir) / (kPi * (1.0f - cosMax * cosMax));
+                            w = mis2(pdf, lpdf);
+                            float ct = dot(sd, nrm);
+                            float death = 1.25f * fmaxf(w - 0.2f, 0.0f);
+                            if (ct >= 0.0f) {
+                                if (rand_chain(seed) > death) {
+                                    float T2, L2;
+                                    light_mix(S.ubo, lid, T2, L2);
+                                    f4 g = f4{f.x * ct / lpdf, f.y * ct / lpdf, f.z * ct / lpdf, f.w * ct / lpdf};
+                                    contrib = emit(pw, l, T2, L2, light_peak(S, lid, T2)) * (T * g) * (1.0f - w);
+                                    shadow = true;
+                                } else {
+                                    w = 1.0f;
+                                }
+                            }
+                        } else {
+                            w = mis2(pdf, 0.0f);
+                        }
+                        float ct = dot(nd, nrm);
+                        T = T * f4{f.x * ct / pdf, f.y * ct / pdf, f.z * ct / pdf, f.w * ct / pdf};
+                        float pr = ptm_clamp(fmaxf(T.x, fmaxf(T.y, fmaxf(T.z, T.w))), 0.0f, 0.99f);
+                        cont = false;
+                        if (!(rand_chain(seed) > pr)) {
+                            T = T * (1.0f / pr);
+                            ++bounce;
+                            cont = bounce < F.pathLength;
+                        }
+                        // the shadow ray starts there too
+                        o = no;
+                        d = nd;
+                        st = cont ? PS_RAY : PS_DONE;
+                    }
+                }
+                // LightSourceVisibilityCheck (src/shader.comp:1121-1205): the light sample counts
+                // when the closest object along it is the light; an SDF closer than the
+                // analytic hit sets the object index to -1
+                if (shadow) {
+                    ++shadows;
+                    Hit sh;
+                    sh.t = kMaxDist;
+                    sid = closest_analytic(S, o, sd, sh);
+                    st_t = sh.t;
+                    if (SDF && march_start(S, o, sd, M)) {
+                        shadow_ray = true;
+                        st = PS_MARCH;
+                    } else if (sid == lobj) {
+                        L = f4{L.x + contrib.x, L.y + contrib.y, L.z + contrib.z, L.w + contrib.w};
+                    }
+                }
+            }
+        }
+        if (SDF && st == PS_MARCH) {
+            float mat;
+            const float v = sdf_set<(KIND < 0 ? 0 : KIND)>(S, M.q, M.set, M.phase == MP_MATERIAL, mat);
+            if (shadow_ray) {
+                Hit sh;
+                sh.t = st_t;
+                const int r = march_advance<true>(S, o, sd, M, v, mat, sh, steps);
+                if (r == 2) sid = -1;
+                if (r != 0) st = PS_SHADOW;
+            } else if (march_advance<false>(S, o, d, M, v, mat, h, steps) != 0) {
+                st = PS_SHADE;
             }
         }
     }
-    int slot = wave_append(&Wv.counts[2], shadow);
-    if (shadow) {
-        Wv.s_path[slot] = p;
-        Wv.sox[slot] = no.x; Wv.soy[slot] = no.y; Wv.soz[slot] = no.z;
-        Wv.sdx[slot] = sd.x; Wv.sdy[slot] = sd.y; Wv.sdz[slot] = sd.z;
-        Wv.s_lobj[slot] = lobj;
-        Wv.s_c[slot] = make_float4(contrib.x, contrib.y, contrib.z, contrib.w);
+    wave_add_u64(stat_slot(Wv.stats, 0), segments);
+    wave_add_u64(stat_slot(Wv.stats, 1), shadows);
+    if (SDF) wave_add_u64(stat_slot(Wv.stats, 2), steps);
+    wave_add_u64(stat_slot(Wv.stats, 4), nans);
+    // the last wave to end clears the cursors and the count for the next launch:
+    // every other wave has taken its entries before it counted itself
+    int last = 0;
+    if (threadIdx.x == 0) {
+        __threadfence();
+        last = atomicAdd(Wv.cursor + kSeg * kCntStride, 1) == (int)gridDim.x - 1;
     }
-    int nslot = wave_append(&Wv.counts[nxt], cont);
-    if (cont) Wv.q[nxt][nslot] = p;
-}
-
-__device__ __forceinline__ void add_contrib(RefWave& Wv, int i) {
-    int p = Wv.s_path[i];
-    float4 c = Wv.s_c[i], Lp = Wv.L[p];
-    Wv.L[p] = make_float4(Lp.x + c.x, Lp.y + c.y, Lp.z + c.z, Lp.w + c.w);
-}
-
-// LightSourceVisibilityCheck, analytic part (src/shader.comp:1121-1201). With
-// no SDFs in the scene the visible contributions are added here directly.
-__global__ void __launch_bounds__(kBlock) k_ref_shadow(RefSceneDev S, RefWave Wv, int resolve) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    int n = Wv.counts[2];
-    if (i == 0) atomicAdd(&Wv.stats[1], (unsigned long long)n);
-    if (i >= n) return;
-    f3 o = mk3(Wv.sox[i], Wv.soy[i], Wv.soz[i]);
-    f3 d = mk3(Wv.sdx[i], Wv.sdy[i], Wv.sdz[i]);
-    Hit h;
-    h.t = kMaxDist;
-    int id = closest_analytic(S, o, d, h);
-    if (resolve) {
-        if (id == Wv.s_lobj[i]) add_contrib(Wv, i);
-    } else {
-        Wv.s_t[i] = h.t;
-        Wv.s_id[i] = id;
+    if (__builtin_amdgcn_readfirstlane(last)) {
+        for (int j = (int)threadIdx.x; j <= kSeg; j += kRefLanes) Wv.cursor[j * kCntStride] = 0;
     }
 }
 
-// SphereTracing of the shadow rays: an SDF closer than the analytic hit sets
-// the object index to -1 (src/shader.comp:1203-1205), then visibility resolves.
-template <int KIND>
-__global__ void __launch_bounds__(kBlock) k_ref_shadow_march(RefSceneDev S, RefWave Wv) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    int n = Wv.counts[2];
-    unsigned steps = 0;
-    if (i < n) {
-        f3 o = mk3(Wv.sox[i], Wv.soy[i], Wv.soz[i]);
-        f3 d = mk3(Wv.sdx[i], Wv.sdy[i], Wv.sdz[i]);
-        Hit h;
-        h.t = Wv.s_t[i];
-        int id = Wv.s_id[i];
-        if (sphere_trace<KIND>(S, o, d, h, steps)) id = -1;
-        if (id == Wv.s_lobj[i]) add_contrib(Wv, i);
-    }
-    wave_add_u64(stat_slot(Wv.stats, 2), steps);
-}
-
-// Per pixel, in sample order: XYZ of each path (src/shader.comp:1477-1487)
-// added to the running sum (src/shader.comp:1513-1516).
-__global__ void __launch_bounds__(kBlock) k_ref_accum(RefSceneDev S, RefFrame F, RefWave Wv) {
+// Per pixel, in sample order: the paths' XYZ added to the running sum
+// (src/shader.comp:1513-1516); after the dispatch's last samples, the texel.
+__global__ void __launch_bounds__(kBlock) k_ref_fold(RefFrame F, RefWave Wv, RefFinish Fin, float4* texels, int last) {
     int j = blockIdx.x * blockDim.x + threadIdx.x;
-    unsigned nans = 0;
-    if (j < F.pc) {
-        f3 acc = mk3(0.0f, 0.0f, 0.0f);
-        if (F.k0 != 0) acc = mk3(Wv.sum[j], Wv.sum[F.pc + j], Wv.sum[2 * F.pc + j]);
-        for (int s = 0; s < F.m; ++s) {
-            int path = s * F.pc + j;
-            float4 R = Wv.L[path];
-            f4 l = sample_wavelengths(Wv.lh[path]);
-            f3 X0 = wave_to_xyz(S.ubo, l.x), X1 = wave_to_xyz(S.ubo, l.y);
-            f3 X2 = wave_to_xyz(S.ubo, l.z), X3 = wave_to_xyz(S.ubo, l.w);
-            f3 col = R.x * X0 + R.y * X1 + R.z * X2 + R.w * X3;
-            col = mk3(0.0f, 0.0f, 0.0f) + (col * (720.0f - 390.0f)) * 0.25f;
-            if (col.x != col.x || col.y != col.y || col.z != col.z) {
-                col = mk3(0.0f, 0.0f, 0.0f);
-                ++nans;
-            }
-            acc = acc + col;
-        }
+    if (j >= F.pc) return;
+    f3 acc = mk3(0.0f, 0.0f, 0.0f);
+    if (F.k0 != 0) acc = mk3(Wv.sum[j], Wv.sum[F.pc + j], Wv.sum[2 * F.pc + j]);
+    for (int s = 0; s < F.m; ++s) {
+        const float4 c = Wv.col[s * F.pc + j];
+        acc = acc + mk3(c.x, c.y, c.z);
+    }
+    if (last) {
+        texels[F.p0 + j] = finish_texel(Fin, acc, texels[F.p0 + j]);
+    } else {
         Wv.sum[j] = acc.x;
         Wv.sum[F.pc + j] = acc.y;
         Wv.sum[2 * F.pc + j] = acc.z;
     }
-    wave_add_u64(stat_slot(Wv.stats, 4), nans);
 }
-
-struct RefFinish {
-    int p0, pc, spf, currentSamples, frame, ISO;
-    float apSize, FPS, persistence;
-};
-// Exposure and Accumulate into the texel buffer (src/shader.comp:1492-1532).
-__global__ void __launch_bounds__(kBlock) k_ref_finish(RefFinish F, const float* sum, float4* texels) {
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= F.pc) return;
-    f3 out = mk3(sum[j], sum[F.pc + j], sum[2 * F.pc + j]);
-    out = out / (float)F.spf;
-    out = out * (F.apSize * F.apSize * (float)F.ISO);
-    float4 tx = texels[F.p0 + j];
-    f3 in = mk3(tx.x, tx.y, tx.z);
-    if (F.currentSamples == F.spf && F.frame > F.spf) {
-        float wgt = ptm_pow(2.0f, -8.0f / (F.FPS * F.persistence));
-        out = (1.0f - wgt) * out + wgt * in;
-    } else {
-        int u = F.currentSamples / F.spf;
-        out = ((float)(u - 1) * in + out) / (float)u;
-    }
-    texels[F.p0 + j] = make_float4(out.x, out.y, out.z, 1.0f);
+// Zeroes the cursors of new wave memory (a kernel, not a memset).
+__global__ void k_ref_clear(int* cursor) {
+    for (int j = (int)threadIdx.x; j <= kSeg; j += blockDim.x) cursor[j * kCntStride] = 0;
 }
 
 // ---- host side ---------------------------------------------------------------------------
@@ -956,35 +1111,18 @@ static T* carve(char*& p, size_t n) {
 constexpr size_t round256(size_t bytes) { return ((bytes + 255) / 256) * 256; }
 // Bytes of a wave of `cap` paths as carve_ref_wave lays it out.
 constexpr size_t ref_wave_bytes(int cap) {
-    const size_t f = (size_t)cap;
-    return 6 * round256(f * 4)                                            // ray
-           + 2 * round256(f * 4)                                          // seed, lh
-           + 2 * round256(f * 16) + round256(f * 4)                       // T, L, w
-           + 6 * round256(f * 4)                                          // hit
-           + 2 * round256(f * 4)                                          // queues
-           + round256(f * 4)                                              // s_path
-           + 6 * round256(f * 4)                                          // shadow ray
-           + round256(f * 4) + round256(f * 16) + 2 * round256(f * 4)     // s_lobj, s_c, s_t, s_id
-           + round256(f * 12)                                             // sums
-           + round256(64);                                                // counts
+    return round256((size_t)(kSeg + 1) * kCntStride * 4)  // cursors, count of finished waves
+           + round256((size_t)cap * 16)                    // XYZ by path
+           + round256((size_t)cap * 12);                   // sums
 }
 
-// Lays a wave of `cap` paths out over `base` (ref_wave_bytes(cap) bytes).
+// Lays a wave of `cap` paths out over `base` (ref_wave_bytes(cap) bytes). The
+// cursors come first, at one place whatever the capacity.
 static void carve_ref_wave(char* p, int cap, unsigned long long* stats, RefWave& W) {
     size_t n = (size_t)cap;
-    W.ox = carve<float>(p, n); W.oy = carve<float>(p, n); W.oz = carve<float>(p, n);
-    W.dx = carve<float>(p, n); W.dy = carve<float>(p, n); W.dz = carve<float>(p, n);
-    W.seed = carve<uint32_t>(p, n); W.lh = carve<float>(p, n);
-    W.T = carve<float4>(p, n); W.L = carve<float4>(p, n); W.w = carve<float>(p, n);
-    W.ht = carve<float>(p, n); W.hnx = carve<float>(p, n); W.hny = carve<float>(p, n); W.hnz = carve<float>(p, n);
-    W.hmat = carve<float>(p, n); W.hlight = carve<float>(p, n);
-    W.q[0] = carve<int>(p, n); W.q[1] = carve<int>(p, n);
-    W.s_path = carve<int>(p, n);
-    W.sox = carve<float>(p, n); W.soy = carve<float>(p, n); W.soz = carve<float>(p, n);
-    W.sdx = carve<float>(p, n); W.sdy = carve<float>(p, n); W.sdz = carve<float>(p, n);
-    W.s_lobj = carve<int>(p, n); W.s_c = carve<float4>(p, n); W.s_t = carve<float>(p, n); W.s_id = carve<int>(p, n);
+    W.cursor = carve<int>(p, (size_t)(kSeg + 1) * kCntStride);
+    W.col = carve<float4>(p, n);
     W.sum = carve<float>(p, 3 * n);
-    W.counts = carve<int>(p, 16);
     W.stats = stats;
     W.cap = cap;
 }
@@ -992,26 +1130,41 @@ static void carve_ref_wave(char* p, int cap, unsigned long long* stats, RefWave&
 static int ensure_ref_wave(pt_ctx* ctx, int cap) {
     if (ctx->ref_wave.cap >= cap && ctx->ref_mem.p) return PT_OK;
     dev_free(ctx, ctx->ref_mem);
+    ctx->ref_wave = RefWave{};
     int st = dev_alloc(ctx, ctx->ref_mem, ref_wave_bytes(cap));
     if (st != PT_OK) return st;
     carve_ref_wave(static_cast<char*>(ctx->ref_mem.p), cap, ctx->d_stats, ctx->ref_wave);
-    return PT_OK;
+    launch(ctx, "k_ref_clear", k_ref_clear, dim3(1), dim3(64), ctx->ref_wave.cursor);
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? PT_OK : hip_fail(ctx, e, "reference wave");
 }
 
 // ---- the allocation-free dispatch's wave --------------------------------------------
 // A wave of kStaticWavePaths paths in a static device array: pt_dispatch_noalloc
 // traces through it instead of allocating. Each device holds its own copy for
-// the life of the process. Every launch writes the records it reads (queue
-// counts by k_ref_counts, sums on the first sample chunk), so nothing needs
-// clearing between calls; calls that overlap on one device race on it.
+// the life of the process. Every launch writes the records it reads (its cursors
+// start at zero, as a static array does, and every launch leaves them so), so
+// nothing needs clearing between calls; calls that overlap on one device race on it.
 constexpr int kStaticWavePaths = 1 << 16;
-constexpr size_t kStaticWaveBytes = ref_wave_bytes(kStaticWavePaths);  // 11,010,304 B
+constexpr size_t kStaticWaveBytes = ref_wave_bytes(kStaticWavePaths);  // 1,843,456 B
 static __device__ __align__(256) char scratch[kStaticWaveBytes];
 constexpr int kMaxStaticDevices = 64;
 static std::mutex g_scratch_mu;
 static char* g_scratch[kMaxStaticDevices] = {};
 
+// Waves of k_ref_path that stay resident on a compute unit, by its KIND + 1
+// (asked once per context, so that no dispatch asks while a stream is captured).
+template <int... K>
+static void resident_waves(pt_ctx* ctx, std::integer_sequence<int, K...>) {
+    auto ask = [](auto kernel) {
+        int n = 0;
+        return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, kRefLanes, 0) == hipSuccess && n > 0 ? n : 8;
+    };
+    ((ctx->ref_waves[K] = ask(k_ref_path<K - 1>)), ...);
+}
+
 int ref_static_setup(pt_ctx* ctx) {
+    resident_waves(ctx, std::make_integer_sequence<int, 6>{});
     if (ctx->device < 0 || ctx->device >= kMaxStaticDevices) {
         ctx->err = "static dispatch wave: device ordinal beyond 63";
         return PT_ERR_CAPACITY;
@@ -1103,34 +1256,37 @@ int ref_scene_upload(pt_ctx* ctx, pt_scene* s) {
         }
         kind = (kind == -1 || kind == q.d.kind) ? q.d.kind : 0;
     }
+    std::vector<float> peak((size_t)kRefLights);
+    for (int i = 0; i < kRefLights; ++i) peak[(size_t)i] = wien_peak(U(kUboLight + 2 * i));
     size_t bytes = 0;
-    auto sz = [&](size_t b) { bytes += ((b + 255) / 256) * 256; };
-    sz(sizeof(pt_packed_scene)); sz(sph.size() * sizeof(RefSphere)); sz(pln.size() * sizeof(RefPlane));
+    auto sz = [&](size_t b) { bytes += round256(b); };
+    sz(sizeof(pt_packed_scene)); sz(peak.size() * sizeof(float)); sz(sph.size() * sizeof(RefSphere)); sz(pln.size() * sizeof(RefPlane));
     sz(box.size() * sizeof(RefBox)); sz(lens.size() * sizeof(RefLens)); sz(cyc.size() * sizeof(RefCyclide));
     sz(sdf.size() * sizeof(RefSdf));
     dev_free(ctx, s->ref_mem);
     int st = dev_alloc(ctx, s->ref_mem, bytes);
     if (st != PT_OK) return st;
+    // the tables laid out on the host, in one copy
+    std::vector<char> host(bytes);
     char* base = static_cast<char*>(s->ref_mem.p);
-    char* p = base;
+    size_t at = 0;
     auto put = [&](const void* src, size_t b) -> void* {
-        void* dst = p;
-        if (b) {
-            hipError_t e = hipMemcpy(dst, src, b, hipMemcpyHostToDevice);
-            if (e != hipSuccess) return nullptr;
-        }
-        p += ((b + 255) / 256) * 256;
+        if (b) std::memcpy(host.data() + at, src, b);
+        void* dst = base + at;
+        at += round256(b);
         return dst;
     };
     RefSceneDev& D = s->ref_dev;
     D.ubo = static_cast<const float*>(put(&s->ubo, sizeof(pt_packed_scene)));
+    D.peak = static_cast<const float*>(put(peak.data(), peak.size() * sizeof(float)));
     D.sph = static_cast<const RefSphere*>(put(sph.data(), sph.size() * sizeof(RefSphere)));
     D.pln = static_cast<const RefPlane*>(put(pln.data(), pln.size() * sizeof(RefPlane)));
     D.box = static_cast<const RefBox*>(put(box.data(), box.size() * sizeof(RefBox)));
     D.lens = static_cast<const RefLens*>(put(lens.data(), lens.size() * sizeof(RefLens)));
     D.cyc = static_cast<const RefCyclide*>(put(cyc.data(), cyc.size() * sizeof(RefCyclide)));
     D.sdf = static_cast<const RefSdf*>(put(sdf.data(), sdf.size() * sizeof(RefSdf)));
-    if (!D.ubo) return hip_fail(ctx, hipGetLastError(), "scene upload");
+    hipError_t e = hipMemcpy(base, host.data(), at, hipMemcpyHostToDevice);
+    if (e != hipSuccess) return hip_fail(ctx, e, "scene upload");
     D.ns = ns; D.np = np; D.nb = nb; D.nl = nl; D.nc = nc; D.nsdf = nsdf;
     D.numLights = U(6);
     D.sdf_kind = kind < 0 ? 0 : kind;
@@ -1164,12 +1320,11 @@ static RefFrame make_frame(const pt_push_constants* pc) {
 }
 
 template <int KIND>
-static void launch_march(pt_ctx* ctx, const RefSceneDev& S, RefWave& W, int cur, int grid) {
-    launch(ctx, "k_ref_march", k_ref_march<KIND>, dim3(grid), dim3(kBlock), S, W, cur);
-}
-template <int KIND>
-static void launch_shadow_march(pt_ctx* ctx, const RefSceneDev& S, RefWave& W, int grid) {
-    launch(ctx, "k_ref_shadow_march", k_ref_shadow_march<KIND>, dim3(grid), dim3(kBlock), S, W);
+static void launch_path(pt_ctx* ctx, const RefSceneDev& S, const RefFrame& F, RefWave& W, const RefFinish& Fin,
+                        float4* texels, int direct, int count) {
+    // as many waves as stay resident, at most one per 64 paths
+    const int grid = std::max(1, std::min((F.pc * F.m + kRefLanes - 1) / kRefLanes, ctx->cus * ctx->ref_waves[KIND + 1]));
+    launch(ctx, "k_ref_path", k_ref_path<KIND>, dim3(grid), dim3(kRefLanes), S, F, W, Fin, texels, direct, count);
 }
 
 // One dispatch through the wave Wv (capacity Wv.cap paths): pixels in chunks of
@@ -1180,6 +1335,16 @@ static int ref_dispatch_wave(pt_ctx* ctx, const pt_scene* s, pt_accum* acc, cons
     const int P = W * H;
     const int cap = Wv.cap;
     RefFrame F = make_frame(pc);
+    RefFinish Fin{};
+    Fin.spf = pc->samplesPerFrame;
+    Fin.currentSamples = pc->currentSamples;
+    Fin.frame = pc->frame;
+    Fin.ISO = pc->ISO;
+    Fin.apSize = pc->apertureSize;
+    Fin.FPS = pc->FPS;
+    Fin.persistence = pc->persistence;
+    float4* texels = reinterpret_cast<float4*>(acc->d_texels);
+    const int direct = pc->samplesPerFrame == 1;
     const int pcmax = std::min(P, cap);
     for (int p0 = 0; p0 < P; p0 += pcmax) {
         const int pcur = std::min(pcmax, P - p0);
@@ -1189,61 +1354,37 @@ static int ref_dispatch_wave(pt_ctx* ctx, const pt_scene* s, pt_accum* acc, cons
             F.pc = pcur;
             F.k0 = k0;
             F.m = std::min(m, pc->samplesPerFrame - k0);
-            const int npaths = F.pc * F.m;
-            const int grid = (npaths + kBlock - 1) / kBlock;
-            launch(ctx, "k_ref_counts", k_ref_counts, dim3(1), dim3(1), Wv.counts, npaths, 0, 0);
-            launch(ctx, "k_ref_raygen", k_ref_raygen, dim3(grid), dim3(kBlock), F, Wv);
-            for (int b = 0; b < pc->pathLength; ++b) {
-                const int cur = b & 1;
-                launch(ctx, "k_ref_reset", k_ref_reset, dim3(1), dim3(1), Wv.counts, cur ^ 1);
-                launch(ctx, "k_ref_intersect", k_ref_intersect, dim3(grid), dim3(kBlock), S, Wv, cur);
-                if (S.nsdf > 0) {
-                    switch (S.sdf_kind) {
-                        case PT_SDF_MANDELBULB: launch_march<PT_SDF_MANDELBULB>(ctx, S, Wv, cur, grid); break;
-                        case PT_SDF_MENGER: launch_march<PT_SDF_MENGER>(ctx, S, Wv, cur, grid); break;
-                        case PT_SDF_BLOB: launch_march<PT_SDF_BLOB>(ctx, S, Wv, cur, grid); break;
-                        case PT_SDF_TERRAIN: launch_march<PT_SDF_TERRAIN>(ctx, S, Wv, cur, grid); break;
-                        default: launch_march<0>(ctx, S, Wv, cur, grid); break;
-                    }
-                }
-                launch(ctx, "k_ref_shade", k_ref_shade, dim3(grid), dim3(kBlock), S, F, Wv, cur, b);
-                launch(ctx, "k_ref_shadow", k_ref_shadow, dim3(grid), dim3(kBlock), S, Wv, S.nsdf > 0 ? 0 : 1);
-                if (S.nsdf > 0) {
-                    switch (S.sdf_kind) {
-                        case PT_SDF_MANDELBULB: launch_shadow_march<PT_SDF_MANDELBULB>(ctx, S, Wv, grid); break;
-                        case PT_SDF_MENGER: launch_shadow_march<PT_SDF_MENGER>(ctx, S, Wv, grid); break;
-                        case PT_SDF_BLOB: launch_shadow_march<PT_SDF_BLOB>(ctx, S, Wv, grid); break;
-                        case PT_SDF_TERRAIN: launch_shadow_march<PT_SDF_TERRAIN>(ctx, S, Wv, grid); break;
-                        default: launch_shadow_march<0>(ctx, S, Wv, grid); break;
-                    }
-                }
+            const int count = p0 == 0 && k0 == 0;
+            switch (S.nsdf > 0 ? S.sdf_kind : -1) {
+                case -1: launch_path<-1>(ctx, S, F, Wv, Fin, texels, direct, count); break;
+                case PT_SDF_MANDELBULB: launch_path<PT_SDF_MANDELBULB>(ctx, S, F, Wv, Fin, texels, direct, count); break;
+                case PT_SDF_MENGER: launch_path<PT_SDF_MENGER>(ctx, S, F, Wv, Fin, texels, direct, count); break;
+                case PT_SDF_BLOB: launch_path<PT_SDF_BLOB>(ctx, S, F, Wv, Fin, texels, direct, count); break;
+                case PT_SDF_TERRAIN: launch_path<PT_SDF_TERRAIN>(ctx, S, F, Wv, Fin, texels, direct, count); break;
+                default: launch_path<0>(ctx, S, F, Wv, Fin, texels, direct, count); break;
             }
-            launch(ctx, "k_ref_accum", k_ref_accum, dim3((F.pc + kBlock - 1) / kBlock), dim3(kBlock), S, F, Wv);
+            if (!direct)
+                launch(ctx, "k_ref_fold", k_ref_fold, dim3((F.pc + kBlock - 1) / kBlock), dim3(kBlock), F, Wv, Fin,
+                       texels, (int)(k0 + m >= pc->samplesPerFrame));
         }
-        RefFinish Fin{};
-        Fin.p0 = p0;
-        Fin.pc = pcur;
-        Fin.spf = pc->samplesPerFrame;
-        Fin.currentSamples = pc->currentSamples;
-        Fin.frame = pc->frame;
-        Fin.ISO = pc->ISO;
-        Fin.apSize = pc->apertureSize;
-        Fin.FPS = pc->FPS;
-        Fin.persistence = pc->persistence;
-        launch(ctx, "k_ref_finish", k_ref_finish, dim3((pcur + kBlock - 1) / kBlock), dim3(kBlock), Fin,
-               (const float*)Wv.sum, reinterpret_cast<float4*>(acc->d_texels));
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(ctx, e, "reference dispatch launch");
     return PT_OK;
 }
 
+// Default paths per wave: one wave for all but the largest dispatches (28 bytes a path).
+constexpr int64_t kRefWavePaths = (int64_t)1 << 23;
+
 int ref_dispatch(pt_ctx* ctx, const pt_scene* s, pt_accum* acc, const pt_push_constants* pc) {
-    int cap = ctx->cfg.wave_paths > 0 ? ctx->cfg.wave_paths : (1 << 21);
-    cap = std::max(cap, 1024);
-    int st = ensure_ref_wave(ctx, cap);
+    int64_t cap = ctx->cfg.wave_paths > 0 ? ctx->cfg.wave_paths : kRefWavePaths;
+    cap = std::min(cap, (int64_t)pc->resolution[0] * pc->resolution[1] * pc->samplesPerFrame);
+    cap = std::max<int64_t>(cap, 1024);
+    int st = ensure_ref_wave(ctx, (int)cap);
     if (st != PT_OK) return st;
-    return ref_dispatch_wave(ctx, s, acc, pc, ctx->ref_wave);
+    RefWave Wv = ctx->ref_wave;
+    Wv.cap = (int)cap;  // a larger wave than this dispatch asks for is kept
+    return ref_dispatch_wave(ctx, s, acc, pc, Wv);
 }
 
 int ref_dispatch_static(pt_ctx* ctx, const pt_scene* s, pt_accum* acc, const pt_push_constants* pc) {

@@ -38,6 +38,8 @@ struct RefLens {
 struct RefCyclide { f3 pos, scale; m3 M; float a, b, c, d, brad2, mat, light; };
 struct RefSdf { f3 pos, size; pt_sdf_desc d; };
 
+constexpr int kRefLights = PT_MAX_LIGHTS_SIZE / 2;
+
 struct RefSceneDev {
     const float* ubo;  // the 4097-float uniform block
     const RefSphere* sph;
@@ -46,6 +48,7 @@ struct RefSceneDev {
     const RefLens* lens;
     const RefCyclide* cyc;
     const RefSdf* sdf;
+    const float* peak;  // Wien peak term of each light of the uniform block (kRefLights)
     int ns, np, nb, nl, nc, nsdf;
     float numLights;   // numObjects[6]
     int sdf_kind;      // PT_SDF_* when all SDFs share one kind, 0 when mixed or none
@@ -65,26 +68,13 @@ struct RefFrame {
     int p0, pc, k0, m;
 };
 
-// SoA path state of one wave (capacity N paths). Records are written once and
-// read once per stage.
+// One wave of paths (capacity cap): a path lives in its lane's registers and
+// leaves its XYZ here, which the fold adds per pixel in sample order.
 struct RefWave {
-    float *ox, *oy, *oz, *dx, *dy, *dz;
-    uint32_t* seed;
-    float* lh;
-    float4* T;  // throughput per wavelength
-    float4* L;  // radiance per wavelength
-    float* w;   // MIS weight of the next emitter hit
-    float *ht, *hnx, *hny, *hnz, *hmat, *hlight;
-    int* q[2];  // ping-pong path queues
-    // shadow (NEE) records
-    int* s_path;
-    float *sox, *soy, *soz, *sdx, *sdy, *sdz;
-    int* s_lobj;
-    float4* s_c;
-    float* s_t;
-    int* s_id;
+    int* cursor;     // queue cursors of the persistent kernel (wave_queue.h) and its count of finished
+                     // waves, one line each; zero between launches (the last wave clears them)
+    float4* col;     // XYZ by path
     float* sum;      // per-pixel running sums, 3 x pc
-    int* counts;     // [0..1] queue lengths, [2] shadow length
     unsigned long long* stats;  // pt_counters fields
     int cap;
 };
@@ -114,6 +104,7 @@ struct ProfTotal {
 struct pt_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
+    int cus = 256;  // compute units of the device (grid sizing)
     pt_config cfg{};
     std::string err;
     // pt_dispatch_noalloc: whether this device's static wave was found at pt_create
@@ -129,6 +120,7 @@ struct pt_ctx {
     // reference-mode wave
     DevAlloc ref_mem;
     ptk::RefWave ref_wave{};
+    int ref_waves[6] = {};  // resident waves per compute unit of k_ref_path, by its KIND + 1
     // extended-mode wave (owned by ext_tracer.hip)
     void* ext_state = nullptr;
 };
@@ -174,7 +166,7 @@ int ref_dispatch(pt_ctx* ctx, const pt_scene* s, pt_accum* acc, const pt_push_co
 void ref_wave_release(pt_ctx* ctx);
 // The allocation-free variant: the same kernels through a static device wave.
 // ref_static_setup looks the wave's address up on the context's device (once
-// per device; call with that device current).
+// per device; call with that device current) and the path kernels' occupancy.
 int ref_static_setup(pt_ctx* ctx);
 int ref_dispatch_static(pt_ctx* ctx, const pt_scene* s, pt_accum* acc, const pt_push_constants* pc);
 
