@@ -37,12 +37,19 @@ int hip_fail(pt_ctx* ctx, hipError_t e, const char* what) {
 
 int dev_alloc(pt_ctx* ctx, DevAlloc& a, size_t bytes) {
     if (bytes == 0) bytes = 256;
-    if (ctx->cfg.hbm_budget > 0 && ctx->allocated + (int64_t)bytes > ctx->cfg.hbm_budget) {
+    auto over = [&] { return ctx->cfg.hbm_budget > 0 && ctx->allocated + (int64_t)bytes > ctx->cfg.hbm_budget; };
+    if (over()) scratch_give_back(ctx);
+    if (over()) {
         ctx->err = "HBM budget exceeded: " + std::to_string(ctx->allocated + (int64_t)bytes) + " > " +
                    std::to_string(ctx->cfg.hbm_budget) + " bytes";
         return PT_ERR_BUDGET;
     }
     hipError_t e = hipMalloc(&a.p, bytes);
+    if (e != hipSuccess && ctx->scratch.p && !ctx->scratch_used) {
+        (void)hipGetLastError();
+        scratch_give_back(ctx);
+        e = hipMalloc(&a.p, bytes);
+    }
     if (e != hipSuccess) {
         a.p = nullptr;
         return hip_fail(ctx, e, "hipMalloc");
@@ -59,6 +66,28 @@ void dev_free(pt_ctx* ctx, DevAlloc& a) {
     }
     a.p = nullptr;
     a.bytes = 0;
+}
+
+void scratch_give_back(pt_ctx* ctx) {
+    if (!ctx->scratch_used) dev_free(ctx, ctx->scratch);
+}
+
+int ScratchUse::take(size_t bytes) {
+    if (!ctx->scratch.p || ctx->scratch.bytes < bytes) {
+        dev_free(ctx, ctx->scratch);
+        int st = dev_alloc(ctx, ctx->scratch, bytes);
+        if (st != PT_OK) return st;
+    }
+    ctx->scratch_used = true;
+    p = ctx->scratch.p;
+    return PT_OK;
+}
+
+void ScratchUse::release() {
+    if (!p) return;
+    p = nullptr;
+    ctx->scratch_used = false;
+    if (ctx->scratch.bytes > kScratchKeep) dev_free(ctx, ctx->scratch);
 }
 
 }  // namespace ptk
@@ -120,6 +149,7 @@ void pt_destroy(pt_ctx* ctx) {
     (void)hipStreamSynchronize(ctx->stream);
     ptk::ref_wave_release(ctx);
     ptk::ext_wave_release(ctx);
+    ptk::dev_free(ctx, ctx->scratch);
     for (const ProfPending& p : ctx->prof_pending) {
         (void)hipEventDestroy(p.start);
         (void)hipEventDestroy(p.stop);
@@ -393,6 +423,7 @@ pt_status pt_accum_create_exportable(pt_ctx* ctx, int width, int height, pt_accu
     if (gran == 0) gran = 1;
     const size_t bytes = (size_t)width * height * 16;
     const size_t sz = (bytes + gran - 1) / gran * gran;
+    if (ctx->cfg.hbm_budget > 0 && ctx->allocated + (int64_t)sz > ctx->cfg.hbm_budget) ptk::scratch_give_back(ctx);
     if (ctx->cfg.hbm_budget > 0 && ctx->allocated + (int64_t)sz > ctx->cfg.hbm_budget)
         return set_err(ctx, PT_ERR_BUDGET, "HBM budget exceeded: " + std::to_string(ctx->allocated + (int64_t)sz) +
                                                " > " + std::to_string(ctx->cfg.hbm_budget) + " bytes");
@@ -404,6 +435,11 @@ pt_status pt_accum_create_exportable(pt_ctx* ctx, int width, int height, pt_accu
     a->vmm = true;
     a->vmm_bytes = sz;
     e = hipMemCreate(&a->vmm_handle, sz, &prop, 0);
+    if (e != hipSuccess && ctx->scratch.p) {
+        (void)hipGetLastError();
+        ptk::scratch_give_back(ctx);
+        e = hipMemCreate(&a->vmm_handle, sz, &prop, 0);
+    }
     if (e != hipSuccess) {
         delete a;
         return ptk::hip_fail(ctx, e, "pt_accum_create_exportable: hipMemCreate");
@@ -512,47 +548,25 @@ pt_status pt_render_features(pt_ctx* ctx, const pt_scene* s, const pt_push_const
     const size_t P = (size_t)w * h;
     if (n_floats != P * 12) return set_err(ctx, PT_ERR_INVALID_ARG, "pt_render_features: size mismatch");
     (void)hipSetDevice(ctx->device);
-    DevAlloc m;
     const size_t feat_bytes = (P * 48 + 255) / 256 * 256;
-    int st = ptk::dev_alloc(ctx, m, feat_bytes + P * 4);
-    if (st != PT_OK) return st;
-    float* d_feat = (float*)m.p;
-    int* d_n = (int*)((char*)m.p + feat_bytes);
-    std::vector<int> n(P);
     try {
-        hipError_t e = hipMemsetAsync(m.p, 0, feat_bytes + P * 4, ctx->stream);
-        if (e != hipSuccess) st = ptk::hip_fail(ctx, e, "pt_render_features");
-        if (st == PT_OK) st = ptk::ext_dispatch_features(ctx, s, pc, d_feat, d_n);
+        ptk::ScratchUse mem(ctx);
+        int st = mem.take(feat_bytes + P * 4);
+        if (st != PT_OK) return st;
+        float* d_feat = (float*)mem.p;
+        int* d_n = (int*)((char*)mem.p + feat_bytes);
+        st = ptk::ext_dispatch_features(ctx, s, pc, d_feat, d_n, true);
         if (st == PT_OK) st = ptk::count_dispatch(ctx);
-        if (st == PT_OK) {
-            e = hipMemcpyAsync(host, d_feat, P * 48, hipMemcpyDeviceToHost, ctx->stream);
-            if (e == hipSuccess) e = hipMemcpyAsync(n.data(), d_n, P * 4, hipMemcpyDeviceToHost, ctx->stream);
-            if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-            if (e != hipSuccess) st = ptk::hip_fail(ctx, e, "pt_render_features");
-        }
+        hipError_t e = hipSuccess;
+        if (st == PT_OK) e = hipMemcpyAsync(host, d_feat, P * 48, hipMemcpyDeviceToHost, ctx->stream);
+        const hipError_t es = hipStreamSynchronize(ctx->stream);
+        if (e == hipSuccess) e = es;
+        if (st == PT_OK && e != hipSuccess) st = ptk::hip_fail(ctx, e, "pt_render_features");
+        return st;
     } catch (const std::exception& ex) {
-        st = set_err(ctx, PT_ERR_HIP, std::string("pt_render_features: ") + ex.what());
+        (void)hipStreamSynchronize(ctx->stream);
+        return set_err(ctx, PT_ERR_HIP, std::string("pt_render_features: ") + ex.what());
     }
-    (void)hipStreamSynchronize(ctx->stream);
-    ptk::dev_free(ctx, m);
-    if (st != PT_OK) return st;
-    // XYZ in the accumulator's units: exposure apertureSize^2 * ISO per sample,
-    // as the texel resolve applies it
-    const float ex = pc->apertureSize * pc->apertureSize * (float)pc->ISO;
-    for (size_t i = 0; i < P; ++i) {
-        float* f = host + i * 12;
-        const double sy = f[1], syy = f[10];
-        const float inv = n[i] > 0 ? 1.0f / (float)n[i] : 0.0f;
-        const float e = n[i] > 0 ? ex / (float)n[i] : 0.0f;
-        for (int c = 0; c < 3; ++c) f[c] *= e;
-        for (int c = 3; c < 10; ++c) f[c] *= inv;
-        // standard error of the mean of Y: sqrt(sample variance / n)
-        double var = 0.0;
-        if (n[i] > 1) var = std::max(syy - sy * sy / n[i], 0.0) / ((double)n[i] - 1.0) / (double)n[i];
-        f[10] = (float)(std::sqrt(var) * (double)ex);
-        f[11] = (float)n[i];
-    }
-    return PT_OK;
 }
 
 pt_status pt_sync(pt_ctx* ctx) {

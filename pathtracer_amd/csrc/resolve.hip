@@ -46,14 +46,14 @@ __global__ void k_resolve(const float4* texels, int n, int tm, uint8_t* rgb) {
 
 int resolve_srgb8(pt_ctx* ctx, pt_accum* acc, int tonemap, uint8_t* host_rgb) {
     int n = acc->w * acc->h;
-    DevAlloc buf;
-    int st = dev_alloc(ctx, buf, (size_t)n * 3);
+    ScratchUse buf(ctx);
+    int st = buf.take((size_t)n * 3);
     if (st != PT_OK) return st;
     launch(ctx, "k_resolve", k_resolve, dim3((n + 255) / 256), dim3(256), reinterpret_cast<const float4*>(acc->d_texels),
            n, tonemap, static_cast<uint8_t*>(buf.p));
     hipError_t e = hipMemcpyAsync(host_rgb, buf.p, (size_t)n * 3, hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    dev_free(ctx, buf);
+    const hipError_t es = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) e = es;
     if (e != hipSuccess) return hip_fail(ctx, e, "pt_resolve_srgb8");
     return PT_OK;
 }

@@ -166,7 +166,7 @@ int admit(pt_server* s, Request& r, double now) {
         fc.samplesPerFrame = 4;
         fc.frame = 4;
         fc.currentSamples = 4;
-        st = ptk::ext_dispatch_features(ctx, r.scene, &fc, r.aov, r.aov_n);
+        st = ptk::ext_dispatch_features(ctx, r.scene, &fc, r.aov, r.aov_n, false);
         if (st != PT_OK) return fail(s, st, ctx->err);
     }
     int64_t sb = 0;

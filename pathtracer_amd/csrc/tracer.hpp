@@ -111,6 +111,8 @@ struct pt_ctx {
     int static_wave_status = PT_OK;
     std::string static_wave_err;
     int64_t allocated = 0;
+    DevAlloc scratch;  // ptk::ScratchUse
+    bool scratch_used = false;
     unsigned long long* d_stats = nullptr;  // pt_counters fields, 16 slots
     // kernel timing (pt_profile_enable)
     bool prof = false;
@@ -158,6 +160,23 @@ namespace ptk {
 // PT_ERR_BUDGET or PT_ERR_HIP (message in ctx->err).
 int dev_alloc(pt_ctx* ctx, DevAlloc& a, size_t bytes);
 void dev_free(pt_ctx* ctx, DevAlloc& a);
+// The context's scratch memory for the length of a call, which has waited for its
+// work on the stream when it ends: kept between calls up to kScratchKeep (an
+// allocation and a free cost more than a small call's kernels), and given back
+// when another allocation needs the room.
+constexpr size_t kScratchKeep = (size_t)512 << 20;
+struct ScratchUse {
+    pt_ctx* ctx;
+    void* p = nullptr;
+    explicit ScratchUse(pt_ctx* c) : ctx(c) {}
+    ~ScratchUse() { release(); }
+    ScratchUse(const ScratchUse&) = delete;
+    ScratchUse& operator=(const ScratchUse&) = delete;
+    int take(size_t bytes);  // at least `bytes` at p; a pt_status
+    void release();
+};
+// Frees the scratch memory unless a call uses it.
+void scratch_give_back(pt_ctx* ctx);
 int hip_fail(pt_ctx* ctx, hipError_t e, const char* what);
 
 // Reference mode (ref_tracer.hip).
@@ -180,8 +199,11 @@ int ext_dispatch_moments(pt_ctx* ctx, const pt_scene* s, const pt_push_constants
                          int* nsamp);
 // The samples [frame - spf, frame) of every pixel: per-pixel sums of the
 // per-sample XYZ, first-hit features (albedo, normal, distance) and Y^2 into
-// feat (12 floats per pixel, the last unused), sample counts into nsamp.
-int ext_dispatch_features(pt_ctx* ctx, const pt_scene* s, const pt_push_constants* pc, float* feat, int* nsamp);
+// feat (12 floats per pixel, the last unused), sample counts into nsamp. With
+// `means`, feat receives what pt_render_features returns instead (nsamp: scratch
+// of the dispatch's waves). Nothing needs clearing before.
+int ext_dispatch_features(pt_ctx* ctx, const pt_scene* s, const pt_push_constants* pc, float* feat, int* nsamp,
+                          bool means);
 // One request of a batched wave: its scene, the push constants of its quantum
 // (camera, resolution, pathLength; samples [frame - samplesPerFrame, frame)),
 // and its per-pixel moments.
