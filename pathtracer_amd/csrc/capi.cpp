@@ -506,7 +506,6 @@ pt_status pt_dispatch(pt_ctx* ctx, const pt_scene* s, pt_accum* acc, const pt_pu
         } else if (mode == PT_MODE_EXT) {
             if (!s->has_model) return set_err(ctx, PT_ERR_STATE, "extended mode needs a scene loaded from JSON");
             st = ptk::ext_dispatch(ctx, s, acc, pc);
-            if (st == PT_OK) st = ptk::count_dispatch(ctx);
         } else {
             return set_err(ctx, PT_ERR_INVALID_ARG, "pt_dispatch: unknown mode");
         }
@@ -556,7 +555,6 @@ pt_status pt_render_features(pt_ctx* ctx, const pt_scene* s, const pt_push_const
         float* d_feat = (float*)mem.p;
         int* d_n = (int*)((char*)mem.p + feat_bytes);
         st = ptk::ext_dispatch_features(ctx, s, pc, d_feat, d_n, true);
-        if (st == PT_OK) st = ptk::count_dispatch(ctx);
         hipError_t e = hipSuccess;
         if (st == PT_OK) e = hipMemcpyAsync(host, d_feat, P * 48, hipMemcpyDeviceToHost, ctx->stream);
         const hipError_t es = hipStreamSynchronize(ctx->stream);

@@ -58,7 +58,10 @@ constexpr int shadow_cnt(int b) { return (b & 1) ? CNT_SHADOW1 : CNT_SHADOW0; }
 // (wave_queue.h).
 // Cursor sets: persistent intersect, persistent shadow, and one per SDF kind for
 // the persistent march kernels (CUR_MARCH + kind - 1).
-enum : int { CUR_ISECT = 0, CUR_SHADOW = 1, CUR_MARCH = 2, N_CUR = 6 };
+// After them the whole-path kernel's set and its count of finished waves: zero
+// between launches (its last wave clears them).
+enum : int { CUR_ISECT = 0, CUR_SHADOW = 1, CUR_MARCH = 2, N_CUR = 6, CUR_PATH = N_CUR };
+constexpr int kPathCursors = kSeg + 1;
 
 struct ExtMat {
     int type;        // pt::MaterialType
@@ -190,7 +193,7 @@ struct ExtWave {
     uint32_t* smask;  // SDF scenes, by entry like hit: bit k set when the ray enters the box of an SDF of kind k before its analytic hit
     float* sum;
     int* counts;   // N_CNT queue lengths, kCntStride apart
-    int* cursor;   // N_CUR x kSeg persistent-kernel cursors, kCntStride apart
+    int* cursor;   // N_CUR x kSeg persistent-kernel cursors and kPathCursors of the whole-path kernel, kCntStride apart
     unsigned long long* stats;
     int cap;
 };
@@ -1098,9 +1101,14 @@ __global__ void k_ext_counts_batch(int* counts, const ExtBatchHdr* hdr) {
     int i = threadIdx.x;
     if (i < N_CNT) counts[i * kCntStride] = (i == 0) ? hdr->npaths : 0;
 }
-__global__ void k_ext_counts(int* counts, int n0) {
+__global__ void k_ext_counts(int* counts, int n0, unsigned long long* stats, int count_dispatch) {
     int i = threadIdx.x;
     if (i < N_CNT) counts[i * kCntStride] = (i == 0) ? n0 : 0;
+    if (i == 0 && count_dispatch) atomicAdd(&stats[5], 1ull);
+}
+// Zeroes the whole-path kernel's cursors in new wave memory (a kernel, not a memset).
+__global__ void k_ext_clear(int* cursor) {
+    for (int j = (int)threadIdx.x; j < kPathCursors; j += blockDim.x) cursor[(CUR_PATH * kSeg + j) * kCntStride] = 0;
 }
 // Start of bounce b: empty the next extension queue, the material queues, the
 // shadow queue bounce b appends to (read by bounce b - 1 at the latest), and
@@ -1120,18 +1128,17 @@ __device__ __forceinline__ float bk7_index(float lnm) {
     return sqrtf(n2);
 }
 
-// Camera ray of sample k of pixel `pix` of frame F (scene S) into wave slot i,
-// request slot rid.
-__device__ __forceinline__ void gen_ray(const ExtSceneDev& S, const ExtFrame& F, int pix, int k, ExtWave& Wv, int i,
-                                        uint32_t rid, PathRec& rec) {
+// Camera ray of sample k of pixel `pix` of frame F (scene S): origin, direction,
+// hero wavelength and RNG key.
+__device__ __forceinline__ void camera_ray(const ExtSceneDev& S, const ExtFrame& F, int pix, int k, f3& o, f3& d,
+                                           float& l0, uint32_t& key) {
     int gx = pix % F.W, gy = pix / F.W;
     uint32_t sample = (uint32_t)(F.frame - F.spf + k);
-    uint32_t key = path_key(S.seed, (uint32_t)pix, sample);
+    key = path_key(S.seed, (uint32_t)pix, sample);
     float ju = rnd(key, kCamBounce, 0), jv = rnd(key, kCamBounce, 1);
     float uvx = (2.0f * ((float)gx + ju) - (float)F.W) / (float)F.H;
     float uvy = (2.0f * ((float)(F.H - gy) - jv) - (float)F.H) / (float)F.H;
-    float l0 = S.lmin + S.lrange * rnd(key, kCamBounce, 4);
-    f3 o, d;
+    l0 = S.lmin + S.lrange * rnd(key, kCamBounce, 4);
     if (S.camera == 1) {
         float h = 0.5f * F.camSize;
         o = F.camPos;
@@ -1187,6 +1194,15 @@ __device__ __forceinline__ void gen_ray(const ExtSceneDev& S, const ExtFrame& F,
             d = refract(d, nb, n12);
         }
     }
+}
+
+// The same into wave slot i, request slot rid.
+__device__ __forceinline__ void gen_ray(const ExtSceneDev& S, const ExtFrame& F, int pix, int k, ExtWave& Wv, int i,
+                                        uint32_t rid, PathRec& rec) {
+    f3 o, d;
+    float l0;
+    uint32_t key;
+    camera_ray(S, F, pix, k, o, d, l0, key);
     // the camera ray in queue 0's records for the traversal, and in the path's
     // record (stored by the caller) for the shading
     Wv.rq_org[0][i] = make_float4(o.x, o.y, o.z, l0);
@@ -1709,10 +1725,31 @@ __global__ void __launch_bounds__(kBlk) k_ext_classify(ExtSceneDev S0, ExtBatch 
     }
 }
 
-// First-hit features of the camera paths (queue 0 right after bounce 0's
-// trace): an albedo triple (reflectance at 450 / 550 / 650 nm; 1 for glass and
+// First-hit features of a camera path: an albedo triple (reflectance at 450 / 550 / 650 nm; 1 for glass and
 // emitters; the normal-incidence reflectance of a conductor), the shading
 // normal facing the camera and the hit distance; zeros for a miss.
+__device__ __forceinline__ void store_aov(const ExtSceneDev& S, ExtWave& Wv, int p, uint32_t ref, f3 o, f3 d, float t) {
+    float4 a0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), a1 = a0;
+    if (hit_class(S, ref) != Q_MISS) {
+        Surf sf = surface(S, ref, o, d, t);
+        f3 N = dot(sf.n, d) < 0.0f ? sf.n : -sf.n;
+        f3 al = mk3(1.0f, 1.0f, 1.0f);
+        const ExtMat& M = S.mat[sf.mat];
+        if (sf.light < 0) {
+            if (M.type == pt::MAT_CONDUCTOR) {
+                float f0 = fresnel_conductor(1.0f, M.p[0], M.p[1]);
+                al = mk3(f0, f0, f0);
+            } else if (M.type != pt::MAT_DIELECTRIC) {
+                al = mk3(reflectance(M, 450.0f), reflectance(M, 550.0f), reflectance(M, 650.0f));
+            }
+        }
+        a0 = make_float4(al.x, al.y, al.z, t);
+        a1 = make_float4(N.x, N.y, N.z, 0.0f);
+    }
+    Wv.aov0[p] = a0;
+    Wv.aov1[p] = a1;
+}
+// The features of queue 0 right after bounce 0's trace.
 template <bool MULTI>
 __global__ void __launch_bounds__(kBlk) k_ext_aov(ExtSceneDev S0, ExtBatch B, ExtWave Wv) {
     const int n = *qlen(Wv, 0);
@@ -1720,27 +1757,7 @@ __global__ void __launch_bounds__(kBlk) k_ext_aov(ExtSceneDev S0, ExtBatch B, Ex
         const int p = Wv.q[0][idx];
         const ExtSceneDev& S = scene_of<MULTI>(S0, B, MULTI ? Wv.pr[p].aux.w : 0u);
         const float2 h = Wv.hit[idx];
-        const uint32_t ref = __float_as_uint(h.y);
-        float4 a0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), a1 = a0;
-        if (hit_class(S, ref) != Q_MISS) {
-            f3 o = xyz(Wv.rq_org[0][p]), d = xyz(Wv.rq_dir[0][p]);  // bounce 0: the camera ray
-            Surf sf = surface(S, ref, o, d, h.x);
-            f3 N = dot(sf.n, d) < 0.0f ? sf.n : -sf.n;
-            f3 al = mk3(1.0f, 1.0f, 1.0f);
-            const ExtMat& M = S.mat[sf.mat];
-            if (sf.light < 0) {
-                if (M.type == pt::MAT_CONDUCTOR) {
-                    float f0 = fresnel_conductor(1.0f, M.p[0], M.p[1]);
-                    al = mk3(f0, f0, f0);
-                } else if (M.type != pt::MAT_DIELECTRIC) {
-                    al = mk3(reflectance(M, 450.0f), reflectance(M, 550.0f), reflectance(M, 650.0f));
-                }
-            }
-            a0 = make_float4(al.x, al.y, al.z, h.x);
-            a1 = make_float4(N.x, N.y, N.z, 0.0f);
-        }
-        Wv.aov0[p] = a0;
-        Wv.aov1[p] = a1;
+        store_aov(S, Wv, p, __float_as_uint(h.y), xyz(Wv.rq_org[0][p]), xyz(Wv.rq_dir[0][p]), h.x);
     }
 }
 
@@ -1814,7 +1831,217 @@ __device__ __forceinline__ bool roulette(const ExtSceneDev& S, uint32_t key, int
     return true;
 }
 
-// Escaped paths (environment) and emitter hits (weighted by MIS against NEE).
+// A path at a hit: its ray, hero wavelength, RNG key and state (PathRec), as the
+// shading takes it and leaves it for the next bounce.
+struct Vertex {
+    f3 o, d;          // the ray; on return the next ray when the path goes on
+    float l0;
+    f4 T;
+    uint32_t key, flags;
+    float pdf;        // BSDF pdf of the ray
+};
+// A shadow ray from the vertex (its origin the next ray's) with its unoccluded contribution.
+struct ShadowRay {
+    f3 o, d, c;
+    float tmax;
+};
+
+// Escaped paths (environment): the radiance gathered.
+__device__ __forceinline__ f3 shade_miss(const ExtSceneDev& S, const Vertex& v) {
+    float l[4];
+    wavelengths(S, v.l0, l);
+    return to_xyz(S, l, v.T * S.env);
+}
+// Emitter hits, weighted by MIS against NEE.
+__device__ __forceinline__ f3 shade_emit(const ExtSceneDev& S, const Vertex& v, uint32_t ref, float t) {
+    float l[4];
+    wavelengths(S, v.l0, l);
+    Surf sf = surface(S, ref, v.o, v.d, t);
+    const ExtLight& L = S.light[sf.light];
+    float w = 1.0f;
+    // emitters that NEE does not sample (lenses, cyclides) count with weight 1
+    if (!(v.flags & 2u) && sf.light < S.nlight_nee) {
+        // pdf with which next-event estimation from the previous vertex picks this point
+        float pl;
+        if (L.type == REF_QUAD) {
+            float cl = fabsf(dot(L.n, v.d));
+            pl = (t * t) / fmaxf(cl * L.area, 1e-30f);
+        } else {
+            f3 dc = L.p - v.o;
+            float sin2 = (L.radius * L.radius) / dot(dc, dc);
+            float cmax = sqrtf(fmaxf(1.0f - sin2, 0.0f));
+            pl = 1.0f / (2.0f * kPiF * fmaxf(1.0f - cmax, 1e-12f));
+        }
+        pl *= 1.0f / (float)S.nlight_nee;
+        w = v.pdf * v.pdf / (v.pdf * v.pdf + pl * pl);
+    }
+    f4 Le = f4{planck_norm(l[0], L.T, L.lum), 0.0f, 0.0f, 0.0f};
+    if (S.n_lambda > 1)
+        Le = f4{Le.x, planck_norm(l[1], L.T, L.lum), planck_norm(l[2], L.T, L.lum), planck_norm(l[3], L.T, L.lum)};
+    return to_xyz(S, l, v.T * Le * w);
+}
+// Lambert vertices: next-event estimation (one shadow ray) + cosine sampling.
+// Returns whether the path goes on; `shadow` whether sh is to be traced.
+__device__ __forceinline__ bool shade_lambert(const ExtSceneDev& S, Vertex& v, uint32_t ref, float t, int bounce,
+                                              int maxDepth, bool& shadow, ShadowRay& sh) {
+    Surf sf = surface(S, ref, v.o, v.d, t);
+    f3 N = dot(sf.n, v.d) < 0.0f ? sf.n : -sf.n;
+    const ExtMat& M = S.mat[sf.mat];
+    float l[4];
+    wavelengths(S, v.l0, l);
+    const bool multi = S.n_lambda > 1;
+    f4 rho = f4{reflectance(M, l[0]), 0.0f, 0.0f, 0.0f};
+    if (multi) rho = f4{rho.x, reflectance(M, l[1]), reflectance(M, l[2]), reflectance(M, l[3])};
+    f4 T = v.T;
+    const uint32_t key = v.key;
+    f3 P = sf.p + N * offset_scale(sf.p);
+    shadow = false;
+    if (S.nlight_nee > 0) {
+        float ul = rnd(key, (uint32_t)bounce, 3);
+        int li = min((int)(ul * (float)S.nlight_nee), S.nlight_nee - 1);
+        const ExtLight& L = S.light[li];
+        float u4 = rnd(key, (uint32_t)bounce, 4), u5 = rnd(key, (uint32_t)bounce, 5);
+        f3 wi;
+        float dist, pl;
+        bool ok = true;
+        if (L.type == REF_QUAD) {
+            f3 y = L.p + L.e1 * u4 + L.e2 * u5;
+            f3 u = y - P;
+            float d2 = dot(u, u);
+            dist = sqrtf(d2);
+            wi = u * (1.0f / dist);
+            float cl = fabsf(dot(L.n, wi));
+            ok = cl > 1e-7f;
+            pl = d2 / fmaxf(cl * L.area, 1e-30f);
+        } else {
+            f3 dc = L.p - P;
+            float dc2 = dot(dc, dc);
+            float sin2 = (L.radius * L.radius) / dc2;
+            ok = sin2 < 1.0f;
+            float cmax = sqrtf(fmaxf(1.0f - sin2, 0.0f));
+            float ct = 1.0f - u4 * (1.0f - cmax);
+            float st = sqrtf(fmaxf(1.0f - ct * ct, 0.0f));
+            float phi = 2.0f * kPiF * u5;
+            f3 ax = dc * rsqrtf(dc2), tb, bb;
+            onb(ax, tb, bb);
+            wi = tb * (st * __cosf(phi)) + bb * (st * __sinf(phi)) + ax * ct;
+            float th = 0.0f;
+            ok = ok && isect_sphere(make_float4(L.p.x, L.p.y, L.p.z, L.radius), P, wi, 1e30f, th);
+            dist = th;
+            pl = 1.0f / (2.0f * kPiF * fmaxf(1.0f - cmax, 1e-12f));
+        }
+        pl *= 1.0f / (float)S.nlight_nee;
+        float cs = dot(N, wi);
+        if (ok && cs > 0.0f) {
+            float pb = cs * (1.0f / kPiF);
+            float w = pl * pl / (pl * pl + pb * pb);
+            f4 Le = f4{planck_norm(l[0], L.T, L.lum), 0.0f, 0.0f, 0.0f};
+            if (multi)
+                Le = f4{Le.x, planck_norm(l[1], L.T, L.lum), planck_norm(l[2], L.T, L.lum),
+                        planck_norm(l[3], L.T, L.lum)};
+            float g = cs * (1.0f / kPiF) / pl * w;
+            sh.c = to_xyz(S, l, T * rho * Le * g);
+            sh.o = P;
+            sh.d = wi;
+            sh.tmax = dist * (1.0f - 1e-4f);
+            shadow = true;
+        }
+    }
+    // cosine-weighted hemisphere (Malley's method)
+    float u0 = rnd(key, (uint32_t)bounce, 0), u1 = rnd(key, (uint32_t)bounce, 1);
+    float rr = sqrtf(u0), phi = 2.0f * kPiF * u1;
+    float z = sqrtf(fmaxf(1.0f - u0, 0.0f));
+    f3 tb, bb;
+    onb(N, tb, bb);
+    f3 wo = tb * (rr * __cosf(phi)) + bb * (rr * __sinf(phi)) + N * z;
+    T = T * rho;
+    if (!(bounce + 1 < maxDepth && z > 0.0f && roulette(S, key, bounce, T))) return false;
+    v.o = P;
+    v.d = wo;
+    v.T = T;
+    v.flags &= ~2u;
+    v.pdf = z * (1.0f / kPiF);
+    return true;
+}
+// Smooth dielectric: Fresnel-weighted choice of reflection or refraction at the
+// hero wavelength; a dispersive interface keeps only the hero.
+__device__ __forceinline__ bool shade_dielectric(const ExtSceneDev& S, Vertex& v, uint32_t ref, float t, int bounce,
+                                                 int maxDepth) {
+    Surf sf = surface(S, ref, v.o, v.d, t);
+    const ExtMat& M = S.mat[sf.mat];
+    const f3 d = v.d;
+    f3 N = sf.n;
+    float ci = -dot(d, N);
+    bool entering = ci > 0.0f;
+    if (!entering) { N = -N; ci = -ci; }
+    float eta = ior(M, v.l0);
+    float ei = entering ? 1.0f : eta, et = entering ? eta : 1.0f;
+    float er = ei / et;
+    float s2t = er * er * fmaxf(1.0f - ci * ci, 0.0f);
+    float Fr = 1.0f, ct = 0.0f;
+    if (s2t < 1.0f) {
+        ct = sqrtf(1.0f - s2t);
+        Fr = fresnel_dielectric(ci, ct, ei, et);
+    }
+    f3 wo, P;
+    float os = offset_scale(sf.p);
+    if (rnd(v.key, (uint32_t)bounce, 2) < Fr) {
+        wo = d + N * (2.0f * ci);
+        P = sf.p + N * os;
+    } else {
+        wo = normalize(d * er + N * (er * ci - ct));
+        P = sf.p - N * os;
+    }
+    f4 T = v.T;
+    uint32_t fl = v.flags;
+    if (M.dispersive && S.n_lambda > 1 && !(fl & 1u)) {
+        T = f4{T.x * (float)S.n_lambda, 0.0f, 0.0f, 0.0f};
+        fl |= 1u;
+    }
+    if (!(bounce + 1 < maxDepth && roulette(S, v.key, bounce, T))) return false;
+    v.o = P;
+    v.d = wo;
+    v.T = T;
+    v.flags = fl | 2u;
+    return true;
+}
+// Smooth conductor: mirror reflection weighted by the complex-index Fresnel term.
+__device__ __forceinline__ bool shade_conductor(const ExtSceneDev& S, Vertex& v, uint32_t ref, float t, int bounce,
+                                                int maxDepth) {
+    Surf sf = surface(S, ref, v.o, v.d, t);
+    const ExtMat& M = S.mat[sf.mat];
+    const f3 d = v.d;
+    f3 N = dot(sf.n, d) < 0.0f ? sf.n : -sf.n;
+    float ci = -dot(d, N);
+    float Fr = fresnel_conductor(ci, M.p[0], M.p[1]);
+    f4 T = v.T * Fr;
+    f3 wo = d + N * (2.0f * ci);
+    f3 P = sf.p + N * offset_scale(sf.p);
+    if (!(bounce + 1 < maxDepth && roulette(S, v.key, bounce, T))) return false;
+    v.o = P;
+    v.d = wo;
+    v.T = T;
+    v.flags |= 2u;
+    return true;
+}
+
+// Path p's record as a vertex (the ray of its current bounce), and its request slot.
+__device__ __forceinline__ Vertex load_vertex(const ExtWave& Wv, int p, const uint4& aux) {
+    float4 org, dir;  // org.w: hero wavelength
+    path_ray(Wv, p, org, dir);
+    return Vertex{xyz(org), xyz(dir), org.w, f4of(Wv.pr[p].T), aux.x, aux.y, __uint_as_float(aux.z)};
+}
+// The path goes on: its record, and (ro, rd) for its queue entry.
+__device__ __forceinline__ void store_vertex(ExtWave& Wv, int p, const Vertex& v, uint32_t rid, float4& ro, float4& rd) {
+    ro = make_float4(v.o.x, v.o.y, v.o.z, v.l0);
+    rd = make_float4(v.d.x, v.d.y, v.d.z, 0.0f);
+    Wv.pr[p].org = ro;
+    Wv.pr[p].dir = rd;
+    Wv.pr[p].T = make_float4(v.T.x, v.T.y, v.T.z, v.T.w);
+    Wv.pr[p].aux = make_uint4(v.key, v.flags, __float_as_uint(v.pdf), rid);
+}
+
+// Escaped paths and emitter hits.
 template <bool MULTI>
 __global__ void __launch_bounds__(kBlk) k_ext_shade_terminal(ExtSceneDev S0, ExtBatch B, ExtWave Wv, int which) {
     const int n = *qlen(Wv, CNT_MAT + which);
@@ -1822,46 +2049,16 @@ __global__ void __launch_bounds__(kBlk) k_ext_shade_terminal(ExtSceneDev S0, Ext
     for (int idx = blockIdx.x * blockDim.x + threadIdx.x; idx < n; idx += gridDim.x * blockDim.x) {
         const MatEntry me = Wv.mq[which][idx];
         const int p = me.p;
-        const ExtSceneDev& S = scene_of<MULTI>(S0, B, MULTI ? Wv.pr[p].aux.w : 0u);
-        f4 T = f4of(Wv.pr[p].T);
-        float4 org, dir;  // org.w: hero wavelength
-        path_ray(Wv, p, org, dir);
-        float l[4];
-        wavelengths(S, org.w, l);
+        const uint4 aux = Wv.pr[p].aux;
+        const ExtSceneDev& S = scene_of<MULTI>(S0, B, aux.w);
         if (which == Q_MISS) {
-            if (S.has_env) add_xyz(Wv, p, to_xyz(S, l, T * S.env));
+            if (S.has_env) add_xyz(Wv, p, shade_miss(S, load_vertex(Wv, p, aux)));
             continue;
         }
-        f3 o = xyz(org), d = xyz(dir);
-        Surf sf = surface(S, me.ref, o, d, me.t);
-        const ExtLight& L = S.light[sf.light];
-        uint4 aux = Wv.pr[p].aux;
-        float w = 1.0f;
-        // emitters that NEE does not sample (lenses, cyclides) count with weight 1
-        if (!(aux.y & 2u) && sf.light < S.nlight_nee) {
-            // pdf with which next-event estimation from the previous vertex picks this point
-            float pl;
-            if (L.type == REF_QUAD) {
-                float cl = fabsf(dot(L.n, d));
-                pl = (me.t * me.t) / fmaxf(cl * L.area, 1e-30f);
-            } else {
-                f3 dc = L.p - o;
-                float sin2 = (L.radius * L.radius) / dot(dc, dc);
-                float cmax = sqrtf(fmaxf(1.0f - sin2, 0.0f));
-                pl = 1.0f / (2.0f * kPiF * fmaxf(1.0f - cmax, 1e-12f));
-            }
-            pl *= 1.0f / (float)S.nlight_nee;
-            float pb = __uint_as_float(aux.z);
-            w = pb * pb / (pb * pb + pl * pl);
-        }
-        f4 Le = f4{planck_norm(l[0], L.T, L.lum), 0.0f, 0.0f, 0.0f};
-        if (S.n_lambda > 1)
-            Le = f4{Le.x, planck_norm(l[1], L.T, L.lum), planck_norm(l[2], L.T, L.lum), planck_norm(l[3], L.T, L.lum)};
-        add_xyz(Wv, p, to_xyz(S, l, T * Le * w));
+        add_xyz(Wv, p, shade_emit(S, load_vertex(Wv, p, aux), me.ref, me.t));
     }
 }
 
-// Lambert vertices: next-event estimation (one shadow ray) + cosine sampling.
 template <bool MULTI>
 __global__ void __launch_bounds__(kBlk) k_ext_shade_lambert(ExtSceneDev S0, ExtFrame F0, ExtBatch B, ExtWave Wv,
                                                             int cur, int bounce) {
@@ -1876,106 +2073,26 @@ __global__ void __launch_bounds__(kBlk) k_ext_shade_lambert(ExtSceneDev S0, ExtF
         int p = 0;
         bool cont = false, shadow = false;
         float4 ro = make_float4(0.0f, 0.0f, 0.0f, 0.0f), rd = ro;  // the next ray, for its queue entry
-        f3 sP = mk3(0, 0, 0), sD = sP, sC = sP;
-        float smax = 0.0f;
+        ShadowRay sh{};
         uint32_t rid = 0u;
         if (active) {
             const MatEntry me = Wv.mq[Q_LAMBERT][idx];
             p = me.p;
-            uint4 aux = Wv.pr[p].aux;
+            const uint4 aux = Wv.pr[p].aux;
             rid = aux.w;
             const ExtSceneDev& S = scene_of<MULTI>(S0, B, rid);
             const int maxDepth = MULTI ? B.frames[rid].maxDepth : F0.maxDepth;
-            float4 org, dir;  // org.w: hero wavelength
-            path_ray(Wv, p, org, dir);
-            f3 o = xyz(org), d = xyz(dir);
-            Surf sf = surface(S, me.ref, o, d, me.t);
-            f3 N = dot(sf.n, d) < 0.0f ? sf.n : -sf.n;
-            const ExtMat& M = S.mat[sf.mat];
-            float l[4];
-            wavelengths(S, org.w, l);
-            const bool multi = S.n_lambda > 1;
-            f4 rho = f4{reflectance(M, l[0]), 0.0f, 0.0f, 0.0f};
-            if (multi) rho = f4{rho.x, reflectance(M, l[1]), reflectance(M, l[2]), reflectance(M, l[3])};
-            f4 T = f4of(Wv.pr[p].T);
-            uint32_t key = aux.x;
-            f3 P = sf.p + N * offset_scale(sf.p);
-            if (S.nlight_nee > 0) {
-                float ul = rnd(key, (uint32_t)bounce, 3);
-                int li = min((int)(ul * (float)S.nlight_nee), S.nlight_nee - 1);
-                const ExtLight& L = S.light[li];
-                float u4 = rnd(key, (uint32_t)bounce, 4), u5 = rnd(key, (uint32_t)bounce, 5);
-                f3 wi;
-                float dist, pl;
-                bool ok = true;
-                if (L.type == REF_QUAD) {
-                    f3 y = L.p + L.e1 * u4 + L.e2 * u5;
-                    f3 v = y - P;
-                    float d2 = dot(v, v);
-                    dist = sqrtf(d2);
-                    wi = v * (1.0f / dist);
-                    float cl = fabsf(dot(L.n, wi));
-                    ok = cl > 1e-7f;
-                    pl = d2 / fmaxf(cl * L.area, 1e-30f);
-                } else {
-                    f3 dc = L.p - P;
-                    float dc2 = dot(dc, dc);
-                    float sin2 = (L.radius * L.radius) / dc2;
-                    ok = sin2 < 1.0f;
-                    float cmax = sqrtf(fmaxf(1.0f - sin2, 0.0f));
-                    float ct = 1.0f - u4 * (1.0f - cmax);
-                    float st = sqrtf(fmaxf(1.0f - ct * ct, 0.0f));
-                    float phi = 2.0f * kPiF * u5;
-                    f3 ax = dc * rsqrtf(dc2), tb, bb;
-                    onb(ax, tb, bb);
-                    wi = tb * (st * __cosf(phi)) + bb * (st * __sinf(phi)) + ax * ct;
-                    float th = 0.0f;
-                    ok = ok && isect_sphere(make_float4(L.p.x, L.p.y, L.p.z, L.radius), P, wi, 1e30f, th);
-                    dist = th;
-                    pl = 1.0f / (2.0f * kPiF * fmaxf(1.0f - cmax, 1e-12f));
-                }
-                pl *= 1.0f / (float)S.nlight_nee;
-                float cs = dot(N, wi);
-                if (ok && cs > 0.0f) {
-                    float pb = cs * (1.0f / kPiF);
-                    float w = pl * pl / (pl * pl + pb * pb);
-                    f4 Le = f4{planck_norm(l[0], L.T, L.lum), 0.0f, 0.0f, 0.0f};
-                    if (multi)
-                        Le = f4{Le.x, planck_norm(l[1], L.T, L.lum), planck_norm(l[2], L.T, L.lum),
-                                planck_norm(l[3], L.T, L.lum)};
-                    float g = cs * (1.0f / kPiF) / pl * w;
-                    sC = to_xyz(S, l, T * rho * Le * g);
-                    sP = P;
-                    sD = wi;
-                    smax = dist * (1.0f - 1e-4f);
-                    shadow = true;
-                }
-            }
-            // cosine-weighted hemisphere (Malley's method)
-            float u0 = rnd(key, (uint32_t)bounce, 0), u1 = rnd(key, (uint32_t)bounce, 1);
-            float rr = sqrtf(u0), phi = 2.0f * kPiF * u1;
-            float z = sqrtf(fmaxf(1.0f - u0, 0.0f));
-            f3 tb, bb;
-            onb(N, tb, bb);
-            f3 wo = tb * (rr * __cosf(phi)) + bb * (rr * __sinf(phi)) + N * z;
-            T = T * rho;
-            if (bounce + 1 < maxDepth && z > 0.0f && roulette(S, key, bounce, T)) {
-                cont = true;
-                ro = make_float4(P.x, P.y, P.z, org.w);
-                rd = make_float4(wo.x, wo.y, wo.z, 0.0f);
-                Wv.pr[p].org = ro;
-                Wv.pr[p].dir = rd;
-                Wv.pr[p].T = make_float4(T.x, T.y, T.z, T.w);
-                Wv.pr[p].aux = make_uint4(key, aux.y & ~2u, __float_as_uint(z * (1.0f / kPiF)), aux.w);
-            }
+            Vertex v = load_vertex(Wv, p, aux);
+            cont = shade_lambert(S, v, me.ref, me.t, bounce, maxDepth, shadow, sh);
+            if (cont) store_vertex(Wv, p, v, rid, ro, rd);
         }
         int* const ctr[2] = {qlen(Wv, shadow_cnt(bounce)), qlen(Wv, nxt)};
         int slot[2];
         block_append<kBlk, 2>(ctr, (shadow ? 1u : 0u) | (cont ? 2u : 0u), slot);
         if (shadow) {
-            Wv.s_org[slot[0]] = make_float4(sP.x, sP.y, sP.z, smax);
-            Wv.s_dir[slot[0]] = make_float4(sD.x, sD.y, sD.z, __int_as_float(p));
-            Wv.s_xyz[slot[0]] = make_float4(sC.x, sC.y, sC.z, __uint_as_float(rid));
+            Wv.s_org[slot[0]] = make_float4(sh.o.x, sh.o.y, sh.o.z, sh.tmax);
+            Wv.s_dir[slot[0]] = make_float4(sh.d.x, sh.d.y, sh.d.z, __int_as_float(p));
+            Wv.s_xyz[slot[0]] = make_float4(sh.c.x, sh.c.y, sh.c.z, __uint_as_float(rid));
         }
         if (cont) {
             Wv.q[nxt][slot[1]] = p;
@@ -1985,14 +2102,14 @@ __global__ void __launch_bounds__(kBlk) k_ext_shade_lambert(ExtSceneDev S0, ExtF
     }
 }
 
-// Smooth dielectric: Fresnel-weighted choice of reflection or refraction at the
-// hero wavelength; a dispersive interface keeps only the hero.
-template <bool MULTI>
-__global__ void __launch_bounds__(kBlk) k_ext_shade_dielectric(ExtSceneDev S0, ExtFrame F0, ExtBatch B, ExtWave Wv,
-                                                               int cur, int bounce) {
+// Dielectric (GLASS) or conductor vertices.
+template <bool MULTI, bool GLASS>
+__global__ void __launch_bounds__(kBlk) k_ext_shade_specular(ExtSceneDev S0, ExtFrame F0, ExtBatch B, ExtWave Wv,
+                                                             int cur, int bounce) {
+    constexpr int Q = GLASS ? Q_DIELECTRIC : Q_CONDUCTOR;
     const int nxt = cur ^ 1;
-    const int n = *qlen(Wv, CNT_MAT + Q_DIELECTRIC);
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&Wv.stats[6 + Q_DIELECTRIC], (unsigned long long)n);
+    const int n = *qlen(Wv, CNT_MAT + Q);
+    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&Wv.stats[6 + Q], (unsigned long long)n);
     const int stride = gridDim.x * blockDim.x;
     const int rounds = (n + stride - 1) / stride;
     for (int r = 0; r < rounds; ++r) {
@@ -2002,108 +2119,15 @@ __global__ void __launch_bounds__(kBlk) k_ext_shade_dielectric(ExtSceneDev S0, E
         bool cont = false;
         float4 ro = make_float4(0.0f, 0.0f, 0.0f, 0.0f), rd = ro;  // the next ray, for its queue entry
         if (active) {
-            const MatEntry me = Wv.mq[Q_DIELECTRIC][idx];
+            const MatEntry me = Wv.mq[Q][idx];
             p = me.p;
-            uint4 aux = Wv.pr[p].aux;
+            const uint4 aux = Wv.pr[p].aux;
             const ExtSceneDev& S = scene_of<MULTI>(S0, B, aux.w);
             const int maxDepth = MULTI ? B.frames[aux.w].maxDepth : F0.maxDepth;
-            float4 org, dir;  // org.w: hero wavelength
-            path_ray(Wv, p, org, dir);
-            f3 o = xyz(org), d = xyz(dir);
-            Surf sf = surface(S, me.ref, o, d, me.t);
-            const ExtMat& M = S.mat[sf.mat];
-            uint32_t key = aux.x;
-            float l0 = org.w;
-            f3 N = sf.n;
-            float ci = -dot(d, N);
-            bool entering = ci > 0.0f;
-            if (!entering) { N = -N; ci = -ci; }
-            float eta = ior(M, l0);
-            float ei = entering ? 1.0f : eta, et = entering ? eta : 1.0f;
-            float er = ei / et;
-            float s2t = er * er * fmaxf(1.0f - ci * ci, 0.0f);
-            float Fr = 1.0f, ct = 0.0f;
-            if (s2t < 1.0f) {
-                ct = sqrtf(1.0f - s2t);
-                Fr = fresnel_dielectric(ci, ct, ei, et);
-            }
-            f3 wo, P;
-            float os = offset_scale(sf.p);
-            if (rnd(key, (uint32_t)bounce, 2) < Fr) {
-                wo = d + N * (2.0f * ci);
-                P = sf.p + N * os;
-            } else {
-                wo = normalize(d * er + N * (er * ci - ct));
-                P = sf.p - N * os;
-            }
-            f4 T = f4of(Wv.pr[p].T);
-            uint32_t fl = aux.y;
-            if (M.dispersive && S.n_lambda > 1 && !(fl & 1u)) {
-                T = f4{T.x * (float)S.n_lambda, 0.0f, 0.0f, 0.0f};
-                fl |= 1u;
-            }
-            if (bounce + 1 < maxDepth && roulette(S, key, bounce, T)) {
-                cont = true;
-                ro = make_float4(P.x, P.y, P.z, l0);
-                rd = make_float4(wo.x, wo.y, wo.z, 0.0f);
-                Wv.pr[p].org = ro;
-                Wv.pr[p].dir = rd;
-                Wv.pr[p].T = make_float4(T.x, T.y, T.z, T.w);
-                Wv.pr[p].aux = make_uint4(key, fl | 2u, aux.z, aux.w);
-            }
-        }
-        int* const ctr[1] = {qlen(Wv, nxt)};
-        int slot[1];
-        block_append<kBlk, 1>(ctr, cont ? 1u : 0u, slot);
-        if (cont) {
-            Wv.q[nxt][slot[0]] = p;
-            Wv.rq_org[nxt][slot[0]] = ro;
-            Wv.rq_dir[nxt][slot[0]] = rd;
-        }
-    }
-}
-
-// Smooth conductor: mirror reflection weighted by the complex-index Fresnel term.
-template <bool MULTI>
-__global__ void __launch_bounds__(kBlk) k_ext_shade_conductor(ExtSceneDev S0, ExtFrame F0, ExtBatch B, ExtWave Wv,
-                                                              int cur, int bounce) {
-    const int nxt = cur ^ 1;
-    const int n = *qlen(Wv, CNT_MAT + Q_CONDUCTOR);
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&Wv.stats[6 + Q_CONDUCTOR], (unsigned long long)n);
-    const int stride = gridDim.x * blockDim.x;
-    const int rounds = (n + stride - 1) / stride;
-    for (int r = 0; r < rounds; ++r) {
-        int idx = r * stride + blockIdx.x * blockDim.x + threadIdx.x;
-        bool active = idx < n;
-        int p = 0;
-        bool cont = false;
-        float4 ro = make_float4(0.0f, 0.0f, 0.0f, 0.0f), rd = ro;  // the next ray, for its queue entry
-        if (active) {
-            const MatEntry me = Wv.mq[Q_CONDUCTOR][idx];
-            p = me.p;
-            uint4 aux = Wv.pr[p].aux;
-            const ExtSceneDev& S = scene_of<MULTI>(S0, B, aux.w);
-            const int maxDepth = MULTI ? B.frames[aux.w].maxDepth : F0.maxDepth;
-            float4 org, dir;  // org.w: hero wavelength
-            path_ray(Wv, p, org, dir);
-            f3 o = xyz(org), d = xyz(dir);
-            Surf sf = surface(S, me.ref, o, d, me.t);
-            const ExtMat& M = S.mat[sf.mat];
-            f3 N = dot(sf.n, d) < 0.0f ? sf.n : -sf.n;
-            float ci = -dot(d, N);
-            float Fr = fresnel_conductor(ci, M.p[0], M.p[1]);
-            f4 T = f4of(Wv.pr[p].T) * Fr;
-            f3 wo = d + N * (2.0f * ci);
-            f3 P = sf.p + N * offset_scale(sf.p);
-            if (bounce + 1 < maxDepth && roulette(S, aux.x, bounce, T)) {
-                cont = true;
-                ro = make_float4(P.x, P.y, P.z, org.w);
-                rd = make_float4(wo.x, wo.y, wo.z, 0.0f);
-                Wv.pr[p].org = ro;
-                Wv.pr[p].dir = rd;
-                Wv.pr[p].T = make_float4(T.x, T.y, T.z, T.w);
-                Wv.pr[p].aux = make_uint4(aux.x, aux.y | 2u, aux.z, aux.w);
-            }
+            Vertex v = load_vertex(Wv, p, aux);
+            cont = GLASS ? shade_dielectric(S, v, me.ref, me.t, bounce, maxDepth)
+                         : shade_conductor(S, v, me.ref, me.t, bounce, maxDepth);
+            if (cont) store_vertex(Wv, p, v, aux.w, ro, rd);
         }
         int* const ctr[1] = {qlen(Wv, nxt)};
         int slot[1];
@@ -2262,8 +2286,303 @@ __global__ void __launch_bounds__(kBlk) k_ext_extras_shadow(ExtSceneDev S0, ExtB
     }
 }
 
-// Per pixel, in sample order: add each path's XYZ to the running sum.
-__global__ void __launch_bounds__(kBlk) k_ext_accum(ExtFrame F, ExtWave Wv) {
+// ---------------------------------------------------------------------------------
+// Whole paths in one persistent kernel.
+//
+// Visits one node of a binary sphere BVH (bvh_step with W = 2), for an extension
+// ray or, with `any`, a shadow ray: the same tests, the same next node and the
+// same visits as bvh_step's two forms, chosen by lane. Returns true at a shadow
+// ray's hit. `stack` is this lane's column, LANES entries apart.
+template <int LANES>
+__device__ __forceinline__ bool bvh_step2(const BvhDev& B, f3 o, f3 d, f3 inv, f3 oi, float& tbest, int& hit, int& node,
+                                          int& sp, uint16_t* stack, bool any) {
+    const float big = 1e30f;
+    const float4* nd = reinterpret_cast<const float4*>(B.nodes + (size_t)node * 16);
+    const float4 r0 = nd[0], r1 = nd[1], r2 = nd[2], r3 = nd[3];
+    const float lo_x[2] = {r0.x, r0.y}, lo_y[2] = {r0.z, r0.w}, lo_z[2] = {r1.x, r1.y};
+    const float hi_x[2] = {r1.z, r1.w}, hi_y[2] = {r2.x, r2.y}, hi_z[2] = {r2.z, r2.w};
+    const int kid[2] = {__float_as_int(r3.x), __float_as_int(r3.y)}, cnt[2] = {__float_as_int(r3.z), __float_as_int(r3.w)};
+    float tn[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        float tx0 = fmaf(lo_x[j], inv.x, -oi.x), tx1 = fmaf(hi_x[j], inv.x, -oi.x);
+        float ty0 = fmaf(lo_y[j], inv.y, -oi.y), ty1 = fmaf(hi_y[j], inv.y, -oi.y);
+        float tz0 = fmaf(lo_z[j], inv.z, -oi.z), tz1 = fmaf(hi_z[j], inv.z, -oi.z);
+        float lo = fmaxf(fmaxf(fminf(tx0, tx1), fminf(ty0, ty1)), fmaxf(fminf(tz0, tz1), 0.0f));
+        float hi = fminf(fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1)), fminf(fmaxf(tz0, tz1), tbest));
+        tn[j] = (lo <= hi && cnt[j] >= 0) ? lo : big;
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        if (cnt[j] == kInlineSphere) {
+            float t;
+            if (isect_sphere(make_float4(lo_x[j], lo_y[j], lo_z[j], hi_x[j]), o, d, tbest, t)) {
+                tbest = t;
+                hit = kid[j];
+                if (any) return true;
+            }
+        } else if (tn[j] < big && cnt[j] > 0) {
+            for (int k = kid[j]; k < kid[j] + cnt[j]; ++k) {
+                float t;
+                if (isect_sphere(B.prims[k], o, d, tbest, t)) {
+                    tbest = t;
+                    hit = k;
+                    if (any) return true;
+                }
+            }
+            tn[j] = big;
+        }
+    }
+    const bool in0 = tn[0] < tbest && cnt[0] == 0, in1 = tn[1] < tbest && cnt[1] == 0;
+    int next = -1;
+    if (in0 && in1) {
+        // extension rays take the nearer child first (the second on a tie), shadow rays node order
+        const bool first = any || tn[0] < tn[1];
+        next = first ? kid[0] : kid[1];
+        stack[(sp++) * LANES] = (uint16_t)(first ? kid[1] : kid[0]);
+    } else if (in0 || in1) {
+        next = in0 ? kid[0] : kid[1];
+    } else if (sp > 0) {
+        next = (int)stack[(--sp) * LANES];
+    }
+    node = next;
+    return false;
+}
+
+// What a dispatch does with its paths' XYZ once the last sample is in.
+struct ExtFinish {
+    int spf, currentSamples, frame, ISO;
+    float apSize, FPS, persistence;
+};
+__device__ __forceinline__ float4 finish_texel(const ExtFinish& F, f3 sum, float4 tx) {
+    float e = F.apSize * F.apSize * (float)F.ISO / (float)F.spf;
+    f3 out = sum * e;
+    f3 in = mk3(tx.x, tx.y, tx.z);
+    if (F.currentSamples == F.spf && F.frame > F.spf) {
+        float wgt = ptm_pow(2.0f, -8.0f / (F.FPS * F.persistence));
+        out = (1.0f - wgt) * out + wgt * in;
+    } else {
+        int u = F.currentSamples / F.spf;
+        out = ((float)(u - 1) * in + out) / (float)u;
+    }
+    return make_float4(out.x, out.y, out.z, 1.0f);
+}
+
+// A lane's state in k_ext_path, what it does next.
+enum : int {
+    LS_IDLE,    // takes a path from the queue
+    LS_HIT,     // its extension ray's nearest sphere is known
+    LS_SHADOW,  // its shadow ray's visibility is known
+    LS_DONE,    // its path has ended and is to be stored
+    LS_EXT,     // traversal, extension ray
+    LS_ANY,     // traversal, shadow ray
+};
+constexpr int kPathLanes = 64;  // threads per block: one wave, so that few paths spread over all compute units
+constexpr int kPathStack = 32;
+// Lanes waiting for scene work before a wave does it, or as many as traverse (24: 13 %
+// slower on the 4096-sphere scene, 40 and 48 the same: half the wave then decides), and
+// ended lanes before they are stored and refilled (8 / 16 / 32: Cornell box 3.03 / 2.89 /
+// 2.94 ms, 1000-sphere features 4.57 / 4.70 / 5.93 ms).
+constexpr int kPathScene = 32, kPathRefill = 16;
+
+// Whole paths: scenes of spheres (binary BVH, 16-bit nodes), at most kQuadBrute
+// parallelograms and planes. A lane keeps its path in registers from the camera to its
+// end, with the device functions of the per-bounce kernels in the order in which they
+// would take it, so its XYZ is theirs bit for bit. Every iteration visits one BVH node
+// of each traversing lane (extension and shadow rays alike); the others wait for the
+// scene work (hits, shading, new rays and paths).
+// It is bound by VALU issue with 19 of 64 lanes active (rocprofv3, 4096 spheres: the
+// scene work runs each material's code for the few of the waiting lanes that need it),
+// against the persistent traversal kernels' 35; but it has one launch where they have
+// nine a bounce, each as long as its slowest ray, and no path state in memory. Rule
+// (ext_run): dispatches of at most kWholePaths, or any size with at most kWholeSpheres
+// spheres. Depth 12, 1 to 4096 spheres, wavefront against whole, with the read-back of
+// the display image: 160x90x1 646-1835 against 204-602 us, 640x360x1 787-2270 against
+// 240-829 us, 1920x1080x1 1.4-3.7 against 0.9-2.0 ms, x4 2.5-6.0 against 1.8-4.9 ms; at
+// x16 the whole-path kernel is slower from 30 spheres on (7.6-14.7 against 8.9-16.4 ms)
+// and faster with 3 (6.5 against 5.5 ms). Cornell box, 512x512x64: 4.4 against 2.9 ms.
+// Splitting the waiting lanes by material so that each material's code runs at 16 lanes
+// or more took 152 registers and was 20 % slower.
+// `direct`: the dispatch has one sample per pixel, all in this wave, and the paths'
+// texels are finished here instead of by k_ext_fold.
+constexpr int kWholePaths = 1 << 23, kWholeSpheres = 8;
+__global__ void __launch_bounds__(kPathLanes, 4) k_ext_path(ExtSceneDev S, ExtFrame F, ExtWave Wv, ExtFinish Fin,
+                                                          float4* texels, int direct, int aov, int count_dispatch) {
+    __shared__ uint16_t stack_mem[kPathStack * kPathLanes];
+    __shared__ float4 s_quad[4 * kQuadBrute];
+    uint16_t* stack = stack_mem + threadIdx.x;
+    const int nq = min(S.nquad, kQuadBrute);
+    for (int i = (int)threadIdx.x; i < 4 * nq; i += kPathLanes) s_quad[i] = S.quad[i];
+    __syncthreads();
+    const int n = F.pc * F.m;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        atomicAdd(&Wv.stats[3], (unsigned long long)n);
+        if (count_dispatch) atomicAdd(&Wv.stats[5], 1ull);
+    }
+    unsigned nseg = 0, nshadow = 0, nvis = 0, nsvis = 0, ncls[N_MATQ] = {}, nbad = 0, nnan = 0;  // wave totals
+    int st = LS_IDLE, p = 0, bounce = 0;
+    Vertex v{};
+    ShadowRay sh{};
+    f3 acc = mk3(0.0f, 0.0f, 0.0f), inv = acc, oi = acc;
+    bool cont = false, blocked = false;
+    float t = 0.0f;
+    uint32_t ref = kMiss;
+    int node = -1, sp = 0, best = -1;
+    // blocks of 64 consecutive paths are dealt to the queue's segments in turn, so that
+    // each segment, which only its own waves drain, holds a share of the whole image;
+    // entries past the last path are dropped
+    const int nsegm = min(kSeg, (int)gridDim.x);
+    const int seg_blocks = ((n + 63) / 64 + nsegm - 1) / nsegm;
+    int* const cursor = Wv.cursor + CUR_PATH * kSeg * kCntStride;
+    WaveChunk chunk = wave_chunk_init(cursor, seg_blocks * nsegm * 64);
+    while (true) {
+        const int trav = (int)__popcll(__ballot(st >= LS_EXT));
+        const int wait = (int)__popcll(__ballot(st < LS_EXT && !(st == LS_IDLE && chunk.drained())));
+        if (trav == 0 || wait >= min(kPathScene, trav)) {
+            bool ext = false;  // an extension ray starts
+            if (st == LS_SHADOW) {
+                for (int k = 0; !blocked && k < S.nplane; ++k) {
+                    float tp = (ld_ro(S.plane_y + k) - sh.o.y) / sh.d.y;
+                    blocked = tp > kEps && tp < t;
+                }
+                if (!blocked) acc = mk3(acc.x + sh.c.x, acc.y + sh.c.y, acc.z + sh.c.z);
+                ext = cont;
+                if (!cont) st = LS_DONE;
+            }
+            int cls = -1;
+            bool shadow = false;
+            if (st == LS_HIT) {
+                if (best >= 0) ref = (REF_SPHERE << kRefShift) | (uint32_t)S.sbvh.ids[best];
+                for (int i = 0; i < S.nplane; ++i) {
+                    float tp = (ld_ro(S.plane_y + i) - v.o.y) / v.d.y;
+                    if (tp > kEps && tp < t) {
+                        t = tp;
+                        ref = (REF_PLANE << kRefShift) | (uint32_t)i;
+                    }
+                }
+                cls = hit_class(S, ref);
+                if (bounce == 0 && aov) store_aov(S, Wv, p, ref, v.o, v.d, t);
+                cont = false;
+                if (cls == Q_MISS) {
+                    if (S.has_env) {
+                        const f3 c = shade_miss(S, v);
+                        acc = mk3(acc.x + c.x, acc.y + c.y, acc.z + c.z);
+                    }
+                } else if (cls == Q_EMIT) {
+                    const f3 c = shade_emit(S, v, ref, t);
+                    acc = mk3(acc.x + c.x, acc.y + c.y, acc.z + c.z);
+                } else if (cls == Q_LAMBERT) {
+                    cont = shade_lambert(S, v, ref, t, bounce, F.maxDepth, shadow, sh);
+                } else if (cls == Q_DIELECTRIC) {
+                    cont = shade_dielectric(S, v, ref, t, bounce, F.maxDepth);
+                } else {
+                    cont = shade_conductor(S, v, ref, t, bounce, F.maxDepth);
+                }
+                ++bounce;
+                st = LS_DONE;
+                ext = cont && !shadow;
+            }
+            nbad += (unsigned)__popcll(__ballot(cls >= 0 && ref_is_bad(S, ref)));
+#pragma unroll
+            for (int q = 0; q < N_MATQ; ++q) ncls[q] += (unsigned)__popcll(__ballot(cls == q));
+            nshadow += (unsigned)__popcll(__ballot(shadow));
+            // ended paths are stored, idle lanes refilled
+            const bool free_lane = st == LS_IDLE || (st == LS_DONE && !ext && !shadow);
+            const uint64_t idle = __ballot(free_lane);
+            if (__popcll(idle) >= kPathRefill || __ballot(st >= LS_EXT || ext || shadow) == 0ull) {
+                const bool ended = st == LS_DONE && free_lane;
+                if (direct) {
+                    const bool nan = acc.x != acc.x || acc.y != acc.y || acc.z != acc.z;
+                    nnan += (unsigned)__popcll(__ballot(ended && nan));
+                    if (ended) {
+                        // the sum over samples starts from zero and drops NaN samples
+                        const f3 sum = nan ? mk3(0.0f, 0.0f, 0.0f) : mk3(0.0f, 0.0f, 0.0f) + acc;
+                        texels[F.p0 + p] = finish_texel(Fin, sum, texels[F.p0 + p]);
+                    }
+                } else if (ended) {
+                    Wv.acc[p] = make_float4(acc.x, acc.y, acc.z, 0.0f);
+                }
+                if (ended) st = LS_IDLE;
+                if (!chunk.drained()) {
+                    const int e = wave_refill(idle, chunk);
+                    const int b = e >> 6;
+                    const int path = ((b % seg_blocks) * nsegm + b / seg_blocks) * 64 + (e & 63);
+                    if (e >= 0 && path < n) {
+                        p = path;
+                        camera_ray(S, F, F.p0 + p % F.pc, F.k0 + p / F.pc, v.o, v.d, v.l0, v.key);
+                        v.T = mk4(1.0f);
+                        v.flags = 2u;  // the camera ray counts as specular for emitter MIS
+                        v.pdf = 0.0f;
+                        acc = mk3(0.0f, 0.0f, 0.0f);
+                        bounce = 0;
+                        st = LS_DONE;
+                        ext = F.maxDepth > 0;
+                    }
+                }
+                if (chunk.drained() && __ballot(st != LS_IDLE) == 0ull) break;
+            }
+            nseg += (unsigned)__popcll(__ballot(ext));
+            // the new rays: the parallelograms, then the BVH
+            if (ext || shadow) {
+                const f3 ro = shadow ? sh.o : v.o, rd = shadow ? sh.d : v.d;
+                t = shadow ? sh.tmax : 1e30f;
+                ref = kMiss;
+                best = -1;
+                blocked = false;
+                for (int i = 0; i < nq; ++i) {
+                    float tq;
+                    if (!blocked && isect_quad(s_quad + 4 * i, ro, rd, t, tq)) {
+                        t = shadow ? t : tq;
+                        blocked = shadow;
+                        ref = (REF_QUAD << kRefShift) | (uint32_t)i;
+                    }
+                }
+                ray_inv(ro, rd, inv, oi);
+                sp = 0;
+                node = 0;
+                st = shadow ? LS_ANY : LS_EXT;
+                if (blocked || S.nsph == 0) st = shadow ? LS_SHADOW : LS_HIT;
+            }
+        }
+        const bool any = st == LS_ANY;
+        nvis += (unsigned)__popcll(__ballot(st == LS_EXT));
+        nsvis += (unsigned)__popcll(__ballot(any));
+        if (st >= LS_EXT) {
+            const f3 ro = any ? sh.o : v.o, rd = any ? sh.d : v.d;
+            if (bvh_step2<kPathLanes>(S.sbvh, ro, rd, inv, oi, t, best, node, sp, stack, any)) {
+                blocked = true;
+                node = -1;
+            }
+            if (node < 0) st = any ? LS_SHADOW : LS_HIT;
+        }
+    }
+    if (threadIdx.x == 0) {
+        auto add = [&](int slot, unsigned x) {
+            if (x) atomicAdd(stat_slot(Wv.stats, slot), (unsigned long long)x);
+        };
+        add(0, nseg);
+        add(1, nshadow);
+        for (int q = 0; q < N_MATQ; ++q) add(6 + q, ncls[q]);
+        add(11, nvis);
+        add(12, nsvis);
+        add(4, nnan);
+        add(kStatBadRefs, nbad);
+    }
+    // the last wave to end clears the cursors and the count for the next launch:
+    // every other wave has taken its entries before it counted itself
+    int last = 0;
+    if (threadIdx.x == 0) {
+        __threadfence();
+        last = atomicAdd(cursor + kSeg * kCntStride, 1) == (int)gridDim.x - 1;
+    }
+    if (__builtin_amdgcn_readfirstlane(last)) {
+        for (int j = (int)threadIdx.x; j < kPathCursors; j += kPathLanes) cursor[j * kCntStride] = 0;
+    }
+}
+
+// Per pixel, in sample order: each path's XYZ added to the running sum; after the
+// dispatch's last samples, the texel.
+__global__ void __launch_bounds__(kBlk) k_ext_fold(ExtFrame F, ExtWave Wv, ExtFinish Fin, float4* texels, int last) {
     int j = blockIdx.x * blockDim.x + threadIdx.x;
     unsigned nans = 0;
     if (j < F.pc) {
@@ -2274,30 +2593,13 @@ __global__ void __launch_bounds__(kBlk) k_ext_accum(ExtFrame F, ExtWave Wv) {
             if (a.x != a.x || a.y != a.y || a.z != a.z) { ++nans; continue; }
             ax += a.x; ay += a.y; az += a.z;
         }
-        Wv.sum[j] = ax; Wv.sum[F.pc + j] = ay; Wv.sum[2 * F.pc + j] = az;
+        if (last) {
+            texels[F.p0 + j] = finish_texel(Fin, mk3(ax, ay, az), texels[F.p0 + j]);
+        } else {
+            Wv.sum[j] = ax; Wv.sum[F.pc + j] = ay; Wv.sum[2 * F.pc + j] = az;
+        }
     }
     wave_add_u64(stat_slot(Wv.stats, 4), nans);
-}
-
-struct ExtFinish {
-    int p0, pc, spf, currentSamples, frame, ISO;
-    float apSize, FPS, persistence;
-};
-__global__ void __launch_bounds__(kBlk) k_ext_finish(ExtFinish F, const float* sum, float4* texels) {
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= F.pc) return;
-    float e = F.apSize * F.apSize * (float)F.ISO / (float)F.spf;
-    f3 out = mk3(sum[j], sum[F.pc + j], sum[2 * F.pc + j]) * e;
-    float4 tx = texels[F.p0 + j];
-    f3 in = mk3(tx.x, tx.y, tx.z);
-    if (F.currentSamples == F.spf && F.frame > F.spf) {
-        float wgt = ptm_pow(2.0f, -8.0f / (F.FPS * F.persistence));
-        out = (1.0f - wgt) * out + wgt * in;
-    } else {
-        int u = F.currentSamples / F.spf;
-        out = ((float)(u - 1) * in + out) / (float)u;
-    }
-    texels[F.p0 + j] = make_float4(out.x, out.y, out.z, 1.0f);
 }
 
 // Serving sink: per pixel, in sample order, the first and second moments of
@@ -2429,6 +2731,10 @@ struct ExtSceneHost {
 struct ExtCtxState {
     DevAlloc mem;
     ExtWave wave{};
+    // the wave of the whole-path kernel (acc, first-hit features, sums and its cursors
+    // only), for contexts that have no full wave of its size
+    DevAlloc lean_mem;
+    ExtWave lean{};
     int cu = 0;  // compute units of the context's device (grid sizing)
     DevAlloc batch_mem;  // batched waves: header + scene, frame, segment and sink tables of up to kMaxBatch requests
     // pinned host copy of those tables: one asynchronous upload per wave, and
@@ -2777,22 +3083,60 @@ static T* carve_e(char*& p, size_t n) {
     return r;
 }
 
-static int ensure_ext_wave(pt_ctx* ctx, int cap) {
-    ExtCtxState* st = static_cast<ExtCtxState*>(ctx->ext_state);
-    if (st && st->wave.cap >= cap) return PT_OK;
-    if (!st) {
-        st = new ExtCtxState();
-        ctx->ext_state = st;
+static ExtCtxState* ext_state(pt_ctx* ctx) {
+    if (!ctx->ext_state) ctx->ext_state = new ExtCtxState();
+    return static_cast<ExtCtxState*>(ctx->ext_state);
+}
+
+constexpr size_t kCursorBytes = (size_t)(N_CUR * kSeg + kPathCursors) * kCntStride * 4;
+
+static int clear_path_cursors(pt_ctx* ctx, const ExtWave& W) {
+    launch(ctx, "k_ext_clear", k_ext_clear, dim3(1), dim3(64), W.cursor);
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? PT_OK : hip_fail(ctx, e, "extended wave");
+}
+
+// A wave for the whole-path kernel (*W): the full one when it is large enough, else the
+// lean one, made for `cap` paths.
+static int ensure_lean_wave(pt_ctx* ctx, int cap, ExtWave** W) {
+    ExtCtxState* st = ext_state(ctx);
+    if (st->wave.cap >= cap) {
+        *W = &st->wave;
+        return PT_OK;
     }
+    *W = &st->lean;
+    if (st->lean.cap >= cap) return PT_OK;
+    st->lean = ExtWave{};
+    dev_free(ctx, st->lean_mem);
+    const size_t n = (size_t)cap;
+    int rc = dev_alloc(ctx, st->lean_mem, n * (16 + 32 + 12) + 5 * 256 + kCursorBytes);
+    if (rc != PT_OK) return rc;
+    char* p = static_cast<char*>(st->lean_mem.p);
+    ExtWave& L = st->lean;
+    L.acc = carve_e<float4>(p, n);
+    L.aov0 = carve_e<float4>(p, n); L.aov1 = carve_e<float4>(p, n);
+    L.sum = carve_e<float>(p, 3 * n);
+    L.cursor = carve_e<int>(p, kCursorBytes / 4);
+    L.stats = ctx->d_stats;
+    L.cap = cap;
+    return clear_path_cursors(ctx, L);
+}
+
+static int ensure_ext_wave(pt_ctx* ctx, int cap) {
+    ExtCtxState* st = ext_state(ctx);
+    if (st->wave.cap >= cap) return PT_OK;
     drop_graphs(st);  // they hold the old wave's addresses
+    st->wave = ExtWave{};
     dev_free(ctx, st->mem);
+    st->lean = ExtWave{};  // a full wave serves the whole-path kernel too
+    dev_free(ctx, st->lean_mem);
     size_t n = (size_t)cap;
     // per path: record (org, dir, T, aux) 64, acc 16, hit 8, extension queues 4 * 2,
     // material-queue entries 16 * N_MATQ, shadow org/dir/xyz 48, first-hit
     // features 32, SDF mask 4, sums 12, queue-ordered rays 64
     size_t per_path = 64 + 16 + 8 + 4 * 2 + 16 * N_MATQ + 48 + 32 + 4 + 12 + 64;
     // + 256-byte rounding of 26 arrays + the counters and cursors, one line each
-    int rc = dev_alloc(ctx, st->mem, n * per_path + 28 * 256 + (size_t)(N_CNT + N_CUR * kSeg) * kCntStride * 4);
+    int rc = dev_alloc(ctx, st->mem, n * per_path + 28 * 256 + (size_t)N_CNT * kCntStride * 4 + kCursorBytes);
     if (rc != PT_OK) return rc;
     char* p = static_cast<char*>(st->mem.p);
     ExtWave& W = st->wave;
@@ -2810,10 +3154,10 @@ static int ensure_ext_wave(pt_ctx* ctx, int cap) {
     W.smask = carve_e<uint32_t>(p, n);
     W.sum = carve_e<float>(p, 3 * n);
     W.counts = carve_e<int>(p, (size_t)N_CNT * kCntStride);
-    W.cursor = carve_e<int>(p, (size_t)N_CUR * kSeg * kCntStride);
+    W.cursor = carve_e<int>(p, kCursorBytes / 4);
     W.stats = ctx->d_stats;
     W.cap = cap;
-    return PT_OK;
+    return clear_path_cursors(ctx, W);
 }
 
 void ext_wave_release(pt_ctx* ctx) {
@@ -2824,6 +3168,7 @@ void ext_wave_release(pt_ctx* ctx) {
     if (st->batch_done) (void)hipEventDestroy(st->batch_done);
     if (st->batch_host) (void)hipHostFree(st->batch_host);
     dev_free(ctx, st->batch_mem);
+    dev_free(ctx, st->lean_mem);
     dev_free(ctx, st->mem);
     delete st;
     ctx->ext_state = nullptr;
@@ -2914,9 +3259,9 @@ static void launch_bounce(pt_ctx* ctx, const ExtPlan& P, ExtWave& Wv, int cur, i
     launch(ctx, "k_ext_shade_miss", k_ext_shade_terminal<MULTI>, dim3(grid), dim3(kBlk), S, P.B, Wv, (int)Q_MISS);
     launch(ctx, "k_ext_shade_emit", k_ext_shade_terminal<MULTI>, dim3(grid), dim3(kBlk), S, P.B, Wv, (int)Q_EMIT);
     launch(ctx, "k_ext_shade_lambert", k_ext_shade_lambert<MULTI>, dim3(grid), dim3(kBlk), S, P.F0, P.B, Wv, cur, b);
-    launch(ctx, "k_ext_shade_dielectric", k_ext_shade_dielectric<MULTI>, dim3(grid), dim3(kBlk), S, P.F0, P.B, Wv, cur,
+    launch(ctx, "k_ext_shade_dielectric", k_ext_shade_specular<MULTI, true>, dim3(grid), dim3(kBlk), S, P.F0, P.B, Wv, cur,
            b);
-    launch(ctx, "k_ext_shade_conductor", k_ext_shade_conductor<MULTI>, dim3(grid), dim3(kBlk), S, P.F0, P.B, Wv, cur,
+    launch(ctx, "k_ext_shade_conductor", k_ext_shade_specular<MULTI, false>, dim3(grid), dim3(kBlk), S, P.F0, P.B, Wv, cur,
            b);
     // Shadow rays push children unordered: near-first ordering measured slower
     // on the 4096-sphere scene (most shadow rays are occluded early anyway).
@@ -3020,6 +3365,7 @@ struct ExtSink {
     int* nsamp = nullptr;
     float* feat = nullptr;  // features sink: sums of XYZ, first-hit features and Y^2, 12 per pixel
     ExtFeatEnd feat_end{};
+    bool count = false;  // counts as a dispatch (pt_counters.dispatches)
 };
 
 // Default paths per wave of a single-scene dispatch: 2^27 paths, 28 GB of wave
@@ -3040,9 +3386,23 @@ static int ext_run(pt_ctx* ctx, const pt_scene* s, const pt_push_constants* pc, 
     // allocated for what this dispatch needs, up to that capacity.
     int64_t cap = ctx->cfg.wave_paths > 0 ? ctx->cfg.wave_paths : kDispatchWave;
     cap = std::max<int64_t>(1024, std::min<int64_t>(cap, (int64_t)P * std::max(1, pc->samplesPerFrame)));
-    st = ensure_ext_wave(ctx, (int)cap);
+    // whole paths in one kernel, or a kernel per stage and bounce (k_ext_path has the rule's reasons)
+    const bool whole = H.dev.nsdf == 0 && !H.dev.quad_bvh && H.dev.nlens + H.dev.ncyc == 0 && H.width == 2 &&
+                       H.small_nodes && H.stack_need <= kPathStack && ctx->cfg.traversal == 0 &&
+                       (cap <= kWholePaths || H.dev.nsph <= kWholeSpheres);
+    ExtWave* wave = nullptr;
+    if (whole) {
+        st = ensure_lean_wave(ctx, (int)cap, &wave);
+    } else {
+        st = ensure_ext_wave(ctx, (int)cap);
+        wave = &ext_state(ctx)->wave;
+    }
     if (st != PT_OK) return st;
-    ExtWave& Wv = static_cast<ExtCtxState*>(ctx->ext_state)->wave;
+    ExtWave& Wv = *wave;
+    if (whole && ctx->path_waves == 0 &&
+        (hipOccupancyMaxActiveBlocksPerMultiprocessor(&ctx->path_waves, k_ext_path, kPathLanes, 0) != hipSuccess ||
+         ctx->path_waves < 1))
+        ctx->path_waves = 8;
 
     ExtFrame F = frame_of(*pc);
     const int grid_cap = ctx_cus(ctx) * blocks_per_cu(ctx);
@@ -3057,6 +3417,11 @@ static int ext_run(pt_ctx* ctx, const pt_scene* s, const pt_push_constants* pc, 
     plan.stack_need = H.stack_need;
     plan.small_nodes = H.small_nodes;
     plan.aov = sink.feat != nullptr;
+    ExtFinish Fin{};
+    Fin.spf = pc->samplesPerFrame; Fin.currentSamples = pc->currentSamples; Fin.frame = pc->frame; Fin.ISO = pc->ISO;
+    Fin.apSize = pc->apertureSize; Fin.FPS = pc->FPS; Fin.persistence = pc->persistence;
+    // one sample per pixel: the whole-path kernel finishes the texels
+    const int direct = whole && sink.acc && pc->samplesPerFrame == 1;
     const int pcmax = (int)std::min<int64_t>(P, cap);
     for (int p0 = 0; p0 < P; p0 += pcmax) {
         const int pcur = std::min(pcmax, P - p0);
@@ -3065,25 +3430,26 @@ static int ext_run(pt_ctx* ctx, const pt_scene* s, const pt_push_constants* pc, 
             F.p0 = p0; F.pc = pcur; F.k0 = k0; F.m = std::min(m, pc->samplesPerFrame - k0);
             const int npaths = F.pc * F.m;
             const int grid = std::min((npaths + kBlk - 1) / kBlk, grid_cap);
-            launch(ctx, "k_ext_counts", k_ext_counts, dim3(1), dim3(64), Wv.counts, npaths);
-            launch(ctx, "k_ext_raygen", k_ext_raygen, dim3(grid), dim3(kBlk), H.dev, F, Wv);
-            plan.F0 = F;
-            launch_bounces(ctx, plan, Wv, pc->pathLength, grid);
+            const int count = sink.count && p0 == 0 && k0 == 0;
+            if (whole) {
+                const int waves = std::max(1, std::min((npaths + kPathLanes - 1) / kPathLanes, ctx->cus * ctx->path_waves));
+                launch(ctx, "k_ext_path", k_ext_path, dim3(waves), dim3(kPathLanes), H.dev, F, Wv, Fin,
+                       sink.acc ? reinterpret_cast<float4*>(sink.acc->d_texels) : nullptr, direct, (int)plan.aov, count);
+                if (direct) continue;
+            } else {
+                launch(ctx, "k_ext_counts", k_ext_counts, dim3(1), dim3(64), Wv.counts, npaths, Wv.stats, count);
+                launch(ctx, "k_ext_raygen", k_ext_raygen, dim3(grid), dim3(kBlk), H.dev, F, Wv);
+                plan.F0 = F;
+                launch_bounces(ctx, plan, Wv, pc->pathLength, grid);
+            }
             const dim3 pg((F.pc + kBlk - 1) / kBlk);
             if (sink.acc)
-                launch(ctx, "k_ext_accum", k_ext_accum, pg, dim3(kBlk), F, Wv);
+                launch(ctx, "k_ext_fold", k_ext_fold, pg, dim3(kBlk), F, Wv, Fin,
+                       reinterpret_cast<float4*>(sink.acc->d_texels), (int)(k0 + m >= pc->samplesPerFrame));
             else if (sink.feat)
                 launch(ctx, "k_ext_features", k_ext_features, pg, dim3(kBlk), F, Wv, sink.feat, sink.nsamp, sink.feat_end);
             else
                 launch(ctx, "k_ext_moments", k_ext_moments, pg, dim3(kBlk), F, Wv, P, sink.sum, sink.sumsq, sink.nsamp);
-        }
-        if (sink.acc) {
-            ExtFinish Fin{};
-            Fin.p0 = p0; Fin.pc = pcur; Fin.spf = pc->samplesPerFrame; Fin.currentSamples = pc->currentSamples;
-            Fin.frame = pc->frame; Fin.ISO = pc->ISO; Fin.apSize = pc->apertureSize; Fin.FPS = pc->FPS;
-            Fin.persistence = pc->persistence;
-            launch(ctx, "k_ext_finish", k_ext_finish, dim3((pcur + kBlk - 1) / kBlk), dim3(kBlk), Fin,
-                   (const float*)Wv.sum, reinterpret_cast<float4*>(sink.acc->d_texels));
         }
     }
     hipError_t e = hipGetLastError();
@@ -3094,6 +3460,7 @@ static int ext_run(pt_ctx* ctx, const pt_scene* s, const pt_push_constants* pc, 
 int ext_dispatch(pt_ctx* ctx, const pt_scene* s, pt_accum* acc, const pt_push_constants* pc) {
     ExtSink sink;
     sink.acc = acc;
+    sink.count = true;
     sink.pc = pc;
     return ext_run(ctx, s, pc, sink);
 }
@@ -3257,6 +3624,7 @@ int ext_dispatch_features(pt_ctx* ctx, const pt_scene* s, const pt_push_constant
     sink.pc = pc;
     sink.feat = feat;
     sink.nsamp = nsamp;
+    sink.count = means;
     sink.feat_end = ExtFeatEnd{means ? 1 : 0, pc->apertureSize * pc->apertureSize * (float)pc->ISO};
     return ext_run(ctx, s, pc, sink);
 }

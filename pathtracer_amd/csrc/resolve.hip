@@ -162,8 +162,6 @@ int peak_probe(pt_ctx* ctx, int what, size_t n, int reps, double* units) {
     return PT_OK;
 }
 
-__global__ void k_bump_dispatch(unsigned long long* stats) { stats[5] += 1ull; }
-
 int prof_kernel_id(pt_ctx* ctx, const char* name) {
     for (size_t i = 0; i < ctx->prof_totals.size(); ++i)
         if (ctx->prof_totals[i].name == name) return (int)i;
@@ -182,13 +180,6 @@ hipEvent_t prof_event(pt_ctx* ctx) {
     hipEvent_t e = nullptr;
     (void)hipEventCreate(&e);
     return e;
-}
-
-int count_dispatch(pt_ctx* ctx) {
-    launch(ctx, "k_bump_dispatch", k_bump_dispatch, dim3(1), dim3(1), ctx->d_stats);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return hip_fail(ctx, e, "dispatch counter");
-    return PT_OK;
 }
 
 }  // namespace ptk

@@ -123,6 +123,7 @@ struct pt_ctx {
     DevAlloc ref_mem;
     ptk::RefWave ref_wave{};
     int ref_waves[6] = {};  // resident waves per compute unit of k_ref_path, by its KIND + 1
+    int path_waves = 0;  // resident waves per compute unit of k_ext_path (0: not asked yet)
     // extended-mode wave (owned by ext_tracer.hip)
     void* ext_state = nullptr;
 };
@@ -260,7 +261,6 @@ void ext_wave_release(pt_ctx* ctx);
 int resolve_srgb8(pt_ctx* ctx, pt_accum* acc, int tonemap, uint8_t* host_rgb);
 int math_eval_device(pt_ctx* ctx, int fn, const float* x, const float* y, float* out, size_t n);
 int peak_probe(pt_ctx* ctx, int what, size_t n, int reps, double* units);
-int count_dispatch(pt_ctx* ctx);
 
 // Kernel launch on the context's stream; with profiling on, bracketed by two
 // HIP events whose elapsed time is added to the kernel's total on read.

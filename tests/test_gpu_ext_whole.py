@@ -1,0 +1,103 @@
+"""The extended mode's whole-path kernel (small dispatches and scenes) against the
+kernels per stage and bounce (traversal = 1), bit for bit with equal counters: the
+two are the same device functions in the same order per path. Image edges around
+a wave, one sample (finished in the kernel) and several, waves smaller than the
+image, path lengths 0 and 1, scenes with and without spheres, planes, sky and
+sphere lights, and the features sink."""
+import json
+
+import numpy as np
+import pytest
+
+import pathtracer_amd as pt
+from pathtracer_amd import scenes
+
+
+def plane_and_sky(spheres=3, light=True):
+    """Spheres of the three materials over a ground plane under a sky, one of them a light."""
+    s = scenes.random_spheres_dict(n=spheres, scene_seed=4, wavelengths=4, seed=9)
+    s["quad"] = []
+    s["plane"] = [{"position": [0.0, -0.2, 0.0], "materialID": 1, "lightID": 0}]
+    s["environment"] = {"radiance": 0.7}
+    if light:
+        s["sphere"].append({"position": [0.5, 1.6, 0.3], "radius": 0.2, "materialID": 6, "lightID": 1})
+    else:
+        s["light"] = []
+    return json.dumps(s)
+
+
+SCENES = {
+    "spheres": lambda: scenes.random_spheres(n=500, scene_seed=2, wavelengths=4, seed=7),
+    "cornell1": lambda: scenes.cornell(1, seed=7),
+    "plane_sky": plane_and_sky,
+    "no_light": lambda: plane_and_sky(light=False),
+    "quads_only": lambda: json.dumps(dict(scenes.cornell_dict(4, seed=7), sphere=[])),
+}
+COUNTERS = ("segments", "shadow_segments", "paths", "nan_samples", "dispatches", "escaped", "emitter_hits", "lambert_hits",
+            "dielectric_hits", "conductor_hits", "bvh_nodes", "shadow_bvh_nodes", "bad_refs")
+
+
+def render(traversal, text, w, h, spp, depth, frames=2, wave_paths=0):
+    with pt.Context(0, traversal=traversal, wave_paths=wave_paths) as ctx:
+        r = pt.Renderer(ctx, ctx.scene_from_json(text), w, h, spf=spp, path_length=depth, mode=pt.MODE_EXT)
+        for _ in range(frames):
+            r.render_frame()
+        ctx.profile(True)
+        r.render_frame()
+        names = set(ctx.profile_read())
+        return r.acc.read(), ctx.counters(), names
+
+
+def check(text, w, h, spp, depth, **k):
+    a, ca, na = render(0, text, w, h, spp, depth, **k)
+    b, cb, nb = render(1, text, w, h, spp, depth, **k)
+    assert "k_ext_path" in na and "k_ext_path" not in nb
+    np.testing.assert_array_equal(a.view(np.uint32), b.view(np.uint32))
+    assert {c: ca[c] for c in COUNTERS} == {c: cb[c] for c in COUNTERS}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", SCENES)
+@pytest.mark.parametrize("spp", [1, 3])
+def test_scenes(name, spp):
+    check(SCENES[name](), 61, 37, spp, 7)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("w,h", [(1, 1), (63, 1), (65, 1)])
+@pytest.mark.parametrize("spp", [1, 2])
+def test_image_edges(w, h, spp):
+    check(SCENES["spheres"](), w, h, spp, 5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("depth", [0, 1])
+def test_short_paths(depth):
+    check(SCENES["plane_sky"](), 40, 30, 2, depth)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("spp", [1, 4])
+def test_waves_smaller_than_the_image(spp):
+    check(SCENES["spheres"](), 53, 41, spp, 4, wave_paths=1024)
+
+
+@pytest.mark.gpu
+def test_features_and_a_full_wave_in_between():
+    """First-hit features of both forms; and a context whose full wave (a scene the
+    whole-path kernel does not take) serves the whole-path kernel afterwards."""
+    text = SCENES["spheres"]()
+    out = []
+    for tr in (0, 1):
+        with pt.Context(0, traversal=tr) as ctx:
+            sc = ctx.scene_from_json(text)
+            pc = pt.push_constants(45, 31, 3, 5)
+            sc.camera(1, pc)
+            pc.frame = pc.currentSamples = 3
+            first = ctx.features(sc, pc)
+            sdf = ctx.scene_from_json(scenes.sdf_scene(seed=3))
+            pt.Renderer(ctx, sdf, 64, 48, spf=4, path_length=3, mode=pt.MODE_EXT).render_frame()
+            for _ in range(2):
+                np.testing.assert_array_equal(ctx.features(sc, pc).view(np.uint32), first.view(np.uint32))
+            out.append(first)
+    np.testing.assert_array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
