@@ -364,8 +364,7 @@ pt_status pt_accum_read_xyz(pt_accum* a, float* host, size_t n) {
     if (!a || !host) return set_global(PT_ERR_INVALID_ARG, "pt_accum_read_xyz: NULL argument");
     if (n != (size_t)a->w * a->h * 4) return set_err(a->ctx, PT_ERR_INVALID_ARG, "pt_accum_read_xyz: size mismatch");
     (void)hipSetDevice(a->ctx->device);
-    hipError_t e = hipMemcpyAsync(host, a->d_texels, n * 4, hipMemcpyDeviceToHost, a->ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(a->ctx->stream);
+    hipError_t e = a->ctx->copies.to_host(host, a->d_texels, n * 4, a->ctx->stream);
     if (e != hipSuccess) return ptk::hip_fail(a->ctx, e, "pt_accum_read_xyz");
     return PT_OK;
 }
@@ -374,7 +373,7 @@ pt_status pt_accum_write_xyz(pt_accum* a, const float* host, size_t n) {
     if (!a || !host) return set_global(PT_ERR_INVALID_ARG, "pt_accum_write_xyz: NULL argument");
     if (n != (size_t)a->w * a->h * 4) return set_err(a->ctx, PT_ERR_INVALID_ARG, "pt_accum_write_xyz: size mismatch");
     (void)hipSetDevice(a->ctx->device);
-    hipError_t e = hipMemcpyAsync(a->d_texels, host, n * 4, hipMemcpyHostToDevice, a->ctx->stream);
+    hipError_t e = a->ctx->copies.to_device(a->d_texels, host, n * 4, a->ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(a->ctx->stream);
     if (e != hipSuccess) return ptk::hip_fail(a->ctx, e, "pt_accum_write_xyz");
     return PT_OK;
@@ -556,9 +555,8 @@ pt_status pt_render_features(pt_ctx* ctx, const pt_scene* s, const pt_push_const
         int* d_n = (int*)((char*)mem.p + feat_bytes);
         st = ptk::ext_dispatch_features(ctx, s, pc, d_feat, d_n, true);
         hipError_t e = hipSuccess;
-        if (st == PT_OK) e = hipMemcpyAsync(host, d_feat, P * 48, hipMemcpyDeviceToHost, ctx->stream);
-        const hipError_t es = hipStreamSynchronize(ctx->stream);
-        if (e == hipSuccess) e = es;
+        if (st == PT_OK) e = ctx->copies.to_host(host, d_feat, P * 48, ctx->stream);
+        else (void)hipStreamSynchronize(ctx->stream);  // the scratch memory is free for others after the call
         if (st == PT_OK && e != hipSuccess) st = ptk::hip_fail(ctx, e, "pt_render_features");
         return st;
     } catch (const std::exception& ex) {

@@ -796,7 +796,7 @@ void refresh_bf16(pt_denoiser* d) {
 }
 
 int upload(pt_denoiser* d, float* dst, const float* src, size_t n) {
-    hipError_t e = hipMemcpyAsync(dst, src, n * 4, hipMemcpyHostToDevice, d->ctx->stream);
+    hipError_t e = d->ctx->copies.to_device(dst, src, n * 4, d->ctx->stream);
     if (e != hipSuccess) return dn_fail(d, ptk::hip_fail(d->ctx, e, "denoiser upload"), d->ctx->err);
     return PT_OK;
 }
@@ -1027,8 +1027,7 @@ pt_status pt_dn_set_loss(pt_denoiser* d, int kind) {
 
 pt_status pt_dn_get_params(pt_denoiser* d, float* host, size_t n) {
     if (!d || !host || n != d->nparam) return PT_ERR_INVALID_ARG;
-    hipError_t e = hipMemcpyAsync(host, d->w, n * 4, hipMemcpyDeviceToHost, d->ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(d->ctx->stream);
+    hipError_t e = d->ctx->copies.to_host(host, d->w, n * 4, d->ctx->stream);
     return e == hipSuccess ? PT_OK : dn_fail(d, ptk::hip_fail(d->ctx, e, "pt_dn_get_params"), d->ctx->err);
 }
 
@@ -1052,8 +1051,7 @@ pt_status pt_dn_denoise(pt_denoiser* d, const float* features, int N, int H, int
     forward(d, N, H, W);
     ptk::launch(d->ctx, "k_dn_head", k_head, ew_grid(P), dim3(256), (const float*)d->feat, (const u16*)d->out,
                 (const float*)nullptr, d->den, (u16*)nullptr, (float*)nullptr, P, 0);
-    hipError_t e = hipMemcpyAsync(denoised, d->den, P * 3 * 4, hipMemcpyDeviceToHost, d->ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(d->ctx->stream);
+    hipError_t e = d->ctx->copies.to_host(denoised, d->den, P * 3 * 4, d->ctx->stream);
     return e == hipSuccess ? PT_OK : dn_fail(d, ptk::hip_fail(d->ctx, e, "pt_dn_denoise"), d->ctx->err);
 }
 
@@ -1077,7 +1075,7 @@ pt_status pt_dn_gradients(pt_denoiser* d, const float* features, const float* ta
                 (const float*)d->tgt, (float*)nullptr, d->gc, d->loss, P, d->loss_kind);
     backward(d, N, H, W);
     if (loss) e = hipMemcpyAsync(loss, d->loss, 4, hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess && host_grads) e = hipMemcpyAsync(host_grads, d->g, n_grads * 4, hipMemcpyDeviceToHost, ctx->stream);
+    if (e == hipSuccess && host_grads) e = ctx->copies.to_host(host_grads, d->g, n_grads * 4, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     return e == hipSuccess ? PT_OK : dn_fail(d, ptk::hip_fail(ctx, e, "pt_dn_gradients"), ctx->err);
 }

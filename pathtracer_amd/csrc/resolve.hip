@@ -51,9 +51,7 @@ int resolve_srgb8(pt_ctx* ctx, pt_accum* acc, int tonemap, uint8_t* host_rgb) {
     if (st != PT_OK) return st;
     launch(ctx, "k_resolve", k_resolve, dim3((n + 255) / 256), dim3(256), reinterpret_cast<const float4*>(acc->d_texels),
            n, tonemap, static_cast<uint8_t*>(buf.p));
-    hipError_t e = hipMemcpyAsync(host_rgb, buf.p, (size_t)n * 3, hipMemcpyDeviceToHost, ctx->stream);
-    const hipError_t es = hipStreamSynchronize(ctx->stream);
-    if (e == hipSuccess) e = es;
+    hipError_t e = ctx->copies.to_host(host_rgb, buf.p, (size_t)n * 3, ctx->stream);
     if (e != hipSuccess) return hip_fail(ctx, e, "pt_resolve_srgb8");
     return PT_OK;
 }

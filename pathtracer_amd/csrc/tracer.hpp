@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "../../include/pathtracer.h"
+#include "hostcopy.hpp"
 #include "ptdev.h"
 #include "scene.hpp"
 
@@ -113,6 +114,7 @@ struct pt_ctx {
     int64_t allocated = 0;
     DevAlloc scratch;  // ptk::ScratchUse
     bool scratch_used = false;
+    ptk::HostCopy copies;  // between the caller's buffers and the device, on `stream`
     unsigned long long* d_stats = nullptr;  // pt_counters fields, 16 slots
     // kernel timing (pt_profile_enable)
     bool prof = false;
