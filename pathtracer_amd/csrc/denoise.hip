@@ -95,7 +95,18 @@ struct ConvArgs {
     int flip;
     int tiles_per_block;  // consecutive pixel tiles a block computes in turn
     int up1;              // X1 is at half resolution, upsampled 2x (nearest) as it is read
+    const u16* mask;      // null, or the activation (as Y1) whose ReLU the output goes back through
 };
+
+// The 8 BF16 values v where those of y are positive, else 0: the gradient through
+// the ReLU that produced y.
+__device__ __forceinline__ uint32_t relu_mask(uint32_t v, uint32_t y) {
+    const uint32_t lo = (y & 0xffffu) - 1u < 0x7f80u ? 0xffffu : 0u, hi = (y >> 16) - 1u < 0x7f80u ? 0xffff0000u : 0u;
+    return v & (lo | hi);
+}
+__device__ __forceinline__ uint4 relu_mask(uint4 v, uint4 y) {
+    return make_uint4(relu_mask(v.x, y.x), relu_mask(v.y, y.y), relu_mask(v.z, y.z), relu_mask(v.w, y.w));
+}
 
 // ---------------------------------------------------------------------------------
 // Conv forward (also backward-data), tiled: a block computes tiles of TH rows x
@@ -259,8 +270,9 @@ __global__ void __launch_bounds__(kThreads, NC == 2 ? 2 : 3) k_conv_t(ConvArgs a
             const int g = i % VPP, pix = i / VPP;
             const int y = y0 + pix / TW, x = x0 + pix % TW, c = co0 + J0 * 32 + g * 8;
             if (y >= a.H || x >= a.W || c >= a.Cout) continue;
-            const uint4 val = *reinterpret_cast<const uint4*>(&s_o[pix * OP + g * 8]);
+            uint4 val = *reinterpret_cast<const uint4*>(&s_o[pix * OP + g * 8]);
             const size_t p = ((size_t)n * a.H + y) * a.W + x;
+            if (a.mask) val = relu_mask(val, *reinterpret_cast<const uint4*>(a.mask + p * a.Co1 + c));
             u16* dst = c < a.Co1 ? a.Y1 + p * a.Co1 + c : a.Y2 + p * (a.Cout - a.Co1) + (c - a.Co1);
             *reinterpret_cast<uint4*>(dst) = val;
         }
@@ -434,110 +446,150 @@ __global__ void k_pool2(const u16* x, u16* y, int N, int H, int W, int C) {  // 
         yv[i] = sum4(xv[q * C8 + g], xv[(q + 1) * C8 + g], xv[(q + W) * C8 + g], xv[(q + W + 1) * C8 + g], 0.25f);
     }
 }
-// gradient of the 2x2 average: dX[q] = 0.25 dY (dX written, not accumulated)
-__global__ void k_pool2_bwd(const u16* dy, u16* dx, int N, int H, int W, int C) {
+__device__ __forceinline__ uint32_t add2(uint32_t a, uint32_t b) {
+    return bf_pack(bf_lo(a) + bf_lo(b), bf_hi(a) + bf_hi(b));
+}
+// dZ of an encoder level's output y: the gradient of its 2x2 average (0.25 dY) plus
+// the skip connection's `add`, through the ReLU that produced y (in one pass; they
+// were two kernels with the sum's first term stored in between, rounded as here).
+__global__ void k_pool2_bwd(const u16* dy, const u16* add, const u16* y, u16* dz, int N, int H, int W, int C) {
     const uint32_t C8 = C >> 3;
     const uint32_t n = (uint32_t)N * H * W * C8;
     const uint4* dyv = reinterpret_cast<const uint4*>(dy);
-    uint4* dxv = reinterpret_cast<uint4*>(dx);
+    const uint4* addv = reinterpret_cast<const uint4*>(add);
+    const uint4* yv = reinterpret_cast<const uint4*>(y);
+    uint4* dzv = reinterpret_cast<uint4*>(dz);
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const uint32_t g = i % C8, r = i / C8;
         const uint32_t x = r % W, r2 = r / W;
-        const uint32_t y = r2 % H, b = r2 / H;
-        const uint4 v = dyv[((b * (uint32_t)(H / 2) + y / 2) * (uint32_t)(W / 2) + x / 2) * C8 + g];
-        dxv[i] = make_uint4(scale2(v.x, 0.25f), scale2(v.y, 0.25f), scale2(v.z, 0.25f), scale2(v.w, 0.25f));
+        const uint32_t yy = r2 % H, b = r2 / H;
+        const uint4 v = dyv[((b * (uint32_t)(H / 2) + yy / 2) * (uint32_t)(W / 2) + x / 2) * C8 + g], s = addv[i];
+        const uint4 sum = make_uint4(add2(scale2(v.x, 0.25f), s.x), add2(scale2(v.y, 0.25f), s.y),
+                                     add2(scale2(v.z, 0.25f), s.z), add2(scale2(v.w, 0.25f), s.w));
+        dzv[i] = relu_mask(sum, yv[i]);
     }
 }
-// gradient of the nearest 2x upsample the skip layers apply to their first
-// input as they read it (up_index): dX = sum of the 4 dY it fed
-__global__ void k_up2_bwd(const u16* dy, u16* dx, int N, int H, int W, int C) {
+// dZ of a decoder level's output y: the gradient of the nearest 2x upsample the skip
+// layers apply to it as they read it (up_index; the sum of the 4 dY it fed), through
+// the ReLU that produced y.
+__global__ void k_up2_bwd(const u16* dy, const u16* y, u16* dz, int N, int H, int W, int C) {
     const uint32_t C8 = C >> 3;
     const uint32_t n = (uint32_t)N * H * W * C8;
     const uint4* dyv = reinterpret_cast<const uint4*>(dy);
-    uint4* dxv = reinterpret_cast<uint4*>(dx);
+    const uint4* yv = reinterpret_cast<const uint4*>(y);
+    uint4* dzv = reinterpret_cast<uint4*>(dz);
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const uint32_t g = i % C8, r = i / C8;
         const uint32_t x = r % W, r2 = r / W;
-        const uint32_t y = r2 % H, b = r2 / H;
-        const uint32_t q = (b * 2 * (uint32_t)H + 2 * y) * 2 * (uint32_t)W + 2 * x;
-        dxv[i] = sum4(dyv[q * C8 + g], dyv[(q + 1) * C8 + g], dyv[(q + 2 * W) * C8 + g],
-                      dyv[(q + 2 * W + 1) * C8 + g], 1.0f);
+        const uint32_t yy = r2 % H, b = r2 / H;
+        const uint32_t q = (b * 2 * (uint32_t)H + 2 * yy) * 2 * (uint32_t)W + 2 * x;
+        dzv[i] = relu_mask(sum4(dyv[q * C8 + g], dyv[(q + 1) * C8 + g], dyv[(q + 2 * W) * C8 + g],
+                                dyv[(q + 2 * W + 1) * C8 + g], 1.0f), yv[i]);
     }
 }
-// dZ = dY * (Y > 0): gradient through the ReLU that produced Y; a second
-// gradient `add` (skip connection) is summed in when given
-__global__ void k_relu_bwd(const u16* dy, const u16* add, const u16* y, u16* dz, size_t n) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        float g = bf2f(dy[i]) + (add ? bf2f(add[i]) : 0.0f);
-        dz[i] = f2bf(bf2f(y[i]) > 0.0f ? g : 0.0f);
-    }
-}
-// features (N, H, W, 10) FP32 -> input tensor (16 channels BF16)
-__global__ void k_prep(const float* f, u16* x, size_t P) {
+// features (N, H, W, 12) FP32 -> input tensor (16 channels BF16), a pixel per thread in
+// 16-byte vectors; before a backward pass also clears the nz floats at `zero` (the
+// gradients and, after them, the loss).
+__global__ void k_prep(const float* f, u16* x, size_t P, float* zero, size_t nz) {
     for (size_t p = blockIdx.x * (size_t)blockDim.x + threadIdx.x; p < P; p += (size_t)gridDim.x * blockDim.x) {
-        const float* s = f + p * kFeat;
-        u16* d = x + p * kIn;
-        for (int c = 0; c < 3; ++c) d[c] = f2bf(log1pf(fmaxf(s[c], 0.0f)));
-        for (int c = 3; c < 9; ++c) d[c] = f2bf(s[c]);
-        d[9] = f2bf(1.0f / (1.0f + fmaxf(s[9], 0.0f)));
-        d[10] = f2bf(log1pf(fmaxf(s[10], 0.0f)));
-        d[11] = f2bf(rsqrtf(fmaxf(s[11], 1.0f)));
-        for (int c = 12; c < kIn; ++c) d[c] = 0;
+        const float4* s = reinterpret_cast<const float4*>(f + p * kFeat);
+        const float4 a = s[0], b = s[1], c = s[2];
+        auto log_in = [](float v) { return f2bf(log1pf(fmaxf(v, 0.0f))); };
+        auto pair = [](u16 lo, u16 hi) { return (uint32_t)lo | ((uint32_t)hi << 16); };
+        uint4* d = reinterpret_cast<uint4*>(x + p * kIn);
+        d[0] = make_uint4(pair(log_in(a.x), log_in(a.y)), pair(log_in(a.z), f2bf(a.w)), bf_pack(b.x, b.y),
+                          bf_pack(b.z, b.w));
+        d[1] = make_uint4(pair(f2bf(c.x), f2bf(1.0f / (1.0f + fmaxf(c.y, 0.0f)))),
+                          pair(log_in(c.z), f2bf(rsqrtf(fmaxf(c.w, 1.0f)))), 0u, 0u);
     }
+    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < nz; i += (size_t)gridDim.x * blockDim.x)
+        zero[i] = 0.0f;
 }
 // prediction z = log1p(denoised) = log1p(in) + out[0..2]; loss and its
 // gradient with respect to z, mean over 3P values: |z - log1p(target)|
 // (l2 == 0) or (expm1(z) - target)^2 (l2 == 1); also the denoised image
-// max(expm1(z), 0).
-__global__ void k_head(const float* f, const u16* out, const float* target, float* denoised, u16* dout,
-                       float* loss, size_t P, int l2) {
+// max(expm1(z), 0). The loss takes one atomic per block: one per wave (1152 on one
+// address for 8 crops of 96 x 96, 12 ns each) was most of the kernel's 24 us.
+__global__ void __launch_bounds__(kThreads) k_head(const float* f, const u16* out, const float* target, float* denoised,
+                                                   u16* dout, float* loss, size_t P, int l2) {
+    __shared__ float s_l[kThreads / 64];
     float l = 0.0f;
     const float inv = 1.0f / (3.0f * (float)P);
     for (size_t p = blockIdx.x * (size_t)blockDim.x + threadIdx.x; p < P; p += (size_t)gridDim.x * blockDim.x) {
-        for (int c = 0; c < kOutC; ++c) {
-            if (c >= 3) {
-                if (dout) dout[p * kOutC + c] = 0;
-                continue;
-            }
-            const float z = log1pf(fmaxf(f[p * kFeat + c], 0.0f)) + bf2f(out[p * kOutC + c]);
+        const float4 in = *reinterpret_cast<const float4*>(f + p * kFeat);
+        const uint2 o = *reinterpret_cast<const uint2*>(out + p * kOutC);
+        const float xin[3] = {in.x, in.y, in.z}, res[3] = {bf_lo(o.x), bf_hi(o.x), bf_lo(o.y)};
+        u16 dz[3] = {0, 0, 0};
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const float z = log1pf(fmaxf(xin[c], 0.0f)) + res[c];
             if (denoised) denoised[p * 3 + c] = fmaxf(expm1f(z), 0.0f);
             if (target && l2) {
                 const float y = expm1f(z), d = y - fmaxf(target[p * 3 + c], 0.0f);
                 l += d * d;
-                if (dout) dout[p * kOutC + c] = f2bf(2.0f * d * (y + 1.0f) * inv);
+                dz[c] = f2bf(2.0f * d * (y + 1.0f) * inv);
             } else if (target) {
                 const float d = z - log1pf(fmaxf(target[p * 3 + c], 0.0f));
                 l += fabsf(d);
-                if (dout) dout[p * kOutC + c] = f2bf(d > 0.0f ? inv : (d < 0.0f ? -inv : 0.0f));
+                dz[c] = f2bf(d > 0.0f ? inv : (d < 0.0f ? -inv : 0.0f));
             }
+        }
+        if (dout) {
+            uint4* dv = reinterpret_cast<uint4*>(dout + p * kOutC);
+            dv[0] = make_uint4((uint32_t)dz[0] | ((uint32_t)dz[1] << 16), (uint32_t)dz[2], 0u, 0u);
+            dv[1] = make_uint4(0u, 0u, 0u, 0u);
         }
     }
     if (loss) {
         for (int off = 32; off > 0; off >>= 1) l += __shfl_down(l, off);
-        if ((threadIdx.x & 63) == 0 && l != 0.0f) atomicAdd(loss, l * inv);
+        if ((threadIdx.x & 63) == 0) s_l[threadIdx.x >> 6] = l;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            float t = 0.0f;
+            for (int w = 0; w < kThreads / 64; ++w) t += s_l[w];
+            if (t != 0.0f) atomicAdd(loss, t * inv);
+        }
     }
 }
-// Adam on FP32 masters; then the BF16 forward copy Wf[t][co][ci] and the
-// backward-data copy Wb[t][ci][co] (k_conv_t with `flip` reads tap 8 - t: the
-// gradient of tap t's offset o is gathered from offset -o, which is tap 8 - t).
-__global__ void k_adam(float* w, const float* g, float* m, float* v, size_t n, float lr, float b1, float b2, float eps,
-                       float c1, float c2) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const float gi = g[i];
-        const float mi = b1 * m[i] + (1.0f - b1) * gi;
-        const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-        m[i] = mi;
-        v[i] = vi;
-        w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-    }
-}
-__global__ void k_wcopy(const float* w, u16* wf, u16* wb, int Cout, int Cin) {
-    const int n = 9 * Cout * Cin;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const int ci = i % Cin, co = (i / Cin) % Cout, t = i / (Cin * Cout);
-        const u16 h = f2bf(w[i]);
-        wf[i] = h;
-        wb[((size_t)t * Cin + ci) * Cout + co] = h;
+// A layer's parameters: FP32 masters at w (weights [9][Cout][Cin], then Cout biases),
+// and their BF16 copies: forward Wf[t][co][ci] and backward-data Wb[t][ci][co]
+// (k_conv_t with `flip` reads tap 8 - t: the gradient of tap t's offset o is gathered
+// from offset -o, which is tap 8 - t).
+struct LayerParams {
+    uint32_t off, cout, cin;
+    u16 *wf, *wb;
+};
+constexpr int kLayers = 11;
+struct AllParams {
+    LayerParams l[kLayers];
+};
+struct AdamArgs {
+    float lr, b1, b2, eps, c1, c2;
+};
+// Adam on the FP32 masters (ADAM), then their BF16 copies; blockIdx.y is the layer. One
+// launch for the network, where Adam and a copy kernel per layer were twelve of 6 us.
+template <bool ADAM>
+__global__ void k_params(AllParams A, float* w, const float* g, float* m, float* v, AdamArgs h) {
+    const LayerParams l = A.l[blockIdx.y];
+    const uint32_t nw = 9 * l.cout * l.cin, n = nw + l.cout;
+    for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
+        const uint32_t i = l.off + j;
+        float x = w[i];
+        if (ADAM) {
+            const float gi = g[i];
+            const float mi = h.b1 * m[i] + (1.0f - h.b1) * gi;
+            const float vi = h.b2 * v[i] + (1.0f - h.b2) * gi * gi;
+            m[i] = mi;
+            v[i] = vi;
+            x -= h.lr * (mi / h.c1) / (sqrtf(vi / h.c2) + h.eps);
+            w[i] = x;
+        }
+        if (j < nw) {
+            const uint32_t ci = j % l.cin, r = j / l.cin, co = r % l.cout, t = r / l.cout;
+            const u16 b = f2bf(x);
+            l.wf[j] = b;
+            l.wb[(t * l.cin + ci) * l.cout + co] = b;
+        }
     }
 }
 
@@ -664,7 +716,7 @@ int dn_fail(pt_denoiser* d, int st, const std::string& msg) {
 }
 
 void conv(pt_denoiser* d, const Layer& l, const u16* x1, const u16* x2, u16* y, int N, int H, int W, bool bwd_data,
-          u16* y2 = nullptr, int co1 = 0) {
+          u16* y2 = nullptr, int co1 = 0, const u16* mask = nullptr) {
     ConvArgs a{};
     a.N = N;
     a.H = H;
@@ -679,7 +731,7 @@ void conv(pt_denoiser* d, const Layer& l, const u16* x1, const u16* x2, u16* y, 
         a.X1 = x1; a.X2 = nullptr; a.C1 = l.cout; a.C2 = 0;
         a.Wt = l.wb; a.bias = nullptr;
         a.Y1 = y; a.Y2 = y2; a.Co1 = co1 ? co1 : l.cin1 + l.cin2; a.Cout = l.cin1 + l.cin2;
-        a.relu = 0; a.flip = 1;
+        a.relu = 0; a.flip = 1; a.mask = mask;
     }
     // tiles of 8 x 32 pixels x 64 output channels (32 below 64 channels); each
     // block takes consecutive tiles so that the grid is about two rounds of the
@@ -719,11 +771,13 @@ void wgrad(pt_denoiser* d, const Layer& l, const u16* dz, const u16* x1, const u
 dim3 ew_grid(size_t n) { return dim3((unsigned)std::min<size_t>((n + 255) / 256, 8192)); }
 
 // Forward pass of features already in d->feat (N images H x W).
-void forward(pt_denoiser* d, int N, int H, int W) {
+// With `grads` the gradients and the loss are cleared for a backward pass.
+void forward(pt_denoiser* d, int N, int H, int W, bool grads = false) {
     pt_ctx* ctx = d->ctx;
     const int P = N * H * W, P1 = P / 4, P2 = P / 16;
     const int H1 = H / 2, W1 = W / 2, H2 = H / 4, W2 = W / 4;
-    ptk::launch(ctx, "k_dn_prep", k_prep, ew_grid(P), dim3(256), (const float*)d->feat, d->x0, (size_t)P);
+    ptk::launch(ctx, "k_dn_prep", k_prep, ew_grid(P), dim3(256), (const float*)d->feat, d->x0, (size_t)P, d->g,
+                grads ? d->nparam + 1 : (size_t)0);
     conv(d, d->L[0], d->x0, nullptr, d->e0a, N, H, W, false);
     conv(d, d->L[1], d->e0a, nullptr, d->e0, N, H, W, false);
     ptk::launch(ctx, "k_dn_pool", k_pool2, ew_grid((size_t)P1 * 32 / 8), dim3(256), (const u16*)d->e0, d->p1, N, H, W, 32);
@@ -744,55 +798,56 @@ void backward(pt_denoiser* d, int N, int H, int W) {
     pt_ctx* ctx = d->ctx;
     const int P = N * H * W, P1 = P / 4, P2 = P / 16;
     const int H1 = H / 2, W1 = W / 2, H2 = H / 4, W2 = W / 4;
-    auto relu_bwd = [&](const u16* dy, const u16* add, const u16* y, u16* dz, size_t n) {
-        ptk::launch(ctx, "k_dn_relu_bwd", k_relu_bwd, ew_grid(n), dim3(256), dy, add, y, dz, n);
-    };
+    // Each conv's gradient with respect to its input goes through the ReLU that
+    // produced that input as it is stored (the mask), into the other of ga / gb.
     // out = conv10(d0): no activation
     wgrad(d, d->L[10], d->gc, d->d0, nullptr, N, H, W);
-    conv(d, d->L[10], d->gc, nullptr, d->ga, N, H, W, true);          // dL/d d0 (32)
-    relu_bwd(d->ga, nullptr, d->d0, d->gb, (size_t)P * 32);            // dZ9
+    conv(d, d->L[10], d->gc, nullptr, d->gb, N, H, W, true, nullptr, 0, d->d0);    // dZ9
     wgrad(d, d->L[9], d->gb, d->d0a, nullptr, N, H, W);
-    conv(d, d->L[9], d->gb, nullptr, d->ga, N, H, W, true);           // dL/d d0a (32)
-    relu_bwd(d->ga, nullptr, d->d0a, d->gb, (size_t)P * 32);           // dZ8
-    wgrad(d, d->L[8], d->gb, d->d1, d->e0, N, H, W);
-    conv(d, d->L[8], d->gb, nullptr, d->gc, N, H, W, true, d->gs0, 64);  // dL/d up(d1) (64) | dL/d e0 via skip (32)
-    ptk::launch(ctx, "k_dn_up_bwd", k_up2_bwd, ew_grid((size_t)P1 * 64 / 8), dim3(256), (const u16*)d->gc, d->ga, N, H1, W1,
-                64);                                                   // dL/d d1 (64)
-    relu_bwd(d->ga, nullptr, d->d1, d->gb, (size_t)P1 * 64);           // dZ7
+    conv(d, d->L[9], d->gb, nullptr, d->ga, N, H, W, true, nullptr, 0, d->d0a);    // dZ8
+    wgrad(d, d->L[8], d->ga, d->d1, d->e0, N, H, W);
+    conv(d, d->L[8], d->ga, nullptr, d->gc, N, H, W, true, d->gs0, 64);  // dL/d up(d1) (64) | dL/d e0 via skip (32)
+    ptk::launch(ctx, "k_dn_up_bwd", k_up2_bwd, ew_grid((size_t)P1 * 64 / 8), dim3(256), (const u16*)d->gc,
+                (const u16*)d->d1, d->gb, N, H1, W1, 64);                // dZ7
     wgrad(d, d->L[7], d->gb, d->d1a, nullptr, N, H1, W1);
-    conv(d, d->L[7], d->gb, nullptr, d->ga, N, H1, W1, true);         // dL/d d1a (64)
-    relu_bwd(d->ga, nullptr, d->d1a, d->gb, (size_t)P1 * 64);          // dZ6
-    wgrad(d, d->L[6], d->gb, d->bb, d->e1, N, H1, W1);
-    conv(d, d->L[6], d->gb, nullptr, d->gc, N, H1, W1, true, d->gs1, 128);  // dL/d up(bb) (128) | dL/d e1 via skip (64)
-    ptk::launch(ctx, "k_dn_up_bwd", k_up2_bwd, ew_grid((size_t)P2 * 128 / 8), dim3(256), (const u16*)d->gc, d->ga, N, H2,
-                W2, 128);                                              // dL/d bb (128)
-    relu_bwd(d->ga, nullptr, d->bb, d->gb, (size_t)P2 * 128);          // dZ5
+    conv(d, d->L[7], d->gb, nullptr, d->ga, N, H1, W1, true, nullptr, 0, d->d1a);  // dZ6
+    wgrad(d, d->L[6], d->ga, d->bb, d->e1, N, H1, W1);
+    conv(d, d->L[6], d->ga, nullptr, d->gc, N, H1, W1, true, d->gs1, 128);  // dL/d up(bb) (128) | dL/d e1 via skip (64)
+    ptk::launch(ctx, "k_dn_up_bwd", k_up2_bwd, ew_grid((size_t)P2 * 128 / 8), dim3(256), (const u16*)d->gc,
+                (const u16*)d->bb, d->gb, N, H2, W2, 128);               // dZ5
     wgrad(d, d->L[5], d->gb, d->ba, nullptr, N, H2, W2);
-    conv(d, d->L[5], d->gb, nullptr, d->ga, N, H2, W2, true);         // dL/d ba
-    relu_bwd(d->ga, nullptr, d->ba, d->gb, (size_t)P2 * 128);          // dZ4
-    wgrad(d, d->L[4], d->gb, d->p2, nullptr, N, H2, W2);
-    conv(d, d->L[4], d->gb, nullptr, d->ga, N, H2, W2, true);         // dL/d p2 (64)
-    ptk::launch(ctx, "k_dn_pool_bwd", k_pool2_bwd, ew_grid((size_t)P1 * 64 / 8), dim3(256), (const u16*)d->ga, d->gc, N, H1,
-                W1, 64);                                               // dL/d e1 via pool (64)
-    relu_bwd(d->gc, d->gs1, d->e1, d->gb, (size_t)P1 * 64);            // dZ3 (pool + skip)
+    conv(d, d->L[5], d->gb, nullptr, d->ga, N, H2, W2, true, nullptr, 0, d->ba);   // dZ4
+    wgrad(d, d->L[4], d->ga, d->p2, nullptr, N, H2, W2);
+    conv(d, d->L[4], d->ga, nullptr, d->gc, N, H2, W2, true);            // dL/d p2 (64)
+    ptk::launch(ctx, "k_dn_pool_bwd", k_pool2_bwd, ew_grid((size_t)P1 * 64 / 8), dim3(256), (const u16*)d->gc,
+                (const u16*)d->gs1, (const u16*)d->e1, d->gb, N, H1, W1, 64);  // dZ3 (pool + skip)
     wgrad(d, d->L[3], d->gb, d->e1a, nullptr, N, H1, W1);
-    conv(d, d->L[3], d->gb, nullptr, d->ga, N, H1, W1, true);         // dL/d e1a
-    relu_bwd(d->ga, nullptr, d->e1a, d->gb, (size_t)P1 * 64);          // dZ2
-    wgrad(d, d->L[2], d->gb, d->p1, nullptr, N, H1, W1);
-    conv(d, d->L[2], d->gb, nullptr, d->ga, N, H1, W1, true);         // dL/d p1 (32)
-    ptk::launch(ctx, "k_dn_pool_bwd", k_pool2_bwd, ew_grid((size_t)P * 32 / 8), dim3(256), (const u16*)d->ga, d->gc, N, H, W,
-                32);                                                   // dL/d e0 via pool (32)
-    relu_bwd(d->gc, d->gs0, d->e0, d->gb, (size_t)P * 32);             // dZ1 (pool + skip)
+    conv(d, d->L[3], d->gb, nullptr, d->ga, N, H1, W1, true, nullptr, 0, d->e1a);  // dZ2
+    wgrad(d, d->L[2], d->ga, d->p1, nullptr, N, H1, W1);
+    conv(d, d->L[2], d->ga, nullptr, d->gc, N, H1, W1, true);            // dL/d p1 (32)
+    ptk::launch(ctx, "k_dn_pool_bwd", k_pool2_bwd, ew_grid((size_t)P * 32 / 8), dim3(256), (const u16*)d->gc,
+                (const u16*)d->gs0, (const u16*)d->e0, d->gb, N, H, W, 32);    // dZ1 (pool + skip)
     wgrad(d, d->L[1], d->gb, d->e0a, nullptr, N, H, W);
-    conv(d, d->L[1], d->gb, nullptr, d->ga, N, H, W, true);           // dL/d e0a
-    relu_bwd(d->ga, nullptr, d->e0a, d->gb, (size_t)P * 32);           // dZ0
-    wgrad(d, d->L[0], d->gb, d->x0, nullptr, N, H, W);
+    conv(d, d->L[1], d->gb, nullptr, d->ga, N, H, W, true, nullptr, 0, d->e0a);    // dZ0
+    wgrad(d, d->L[0], d->ga, d->x0, nullptr, N, H, W);
 }
 
-void refresh_bf16(pt_denoiser* d) {
-    for (const Layer& l : d->L)
-        ptk::launch(d->ctx, "k_dn_wcopy", k_wcopy, ew_grid((size_t)9 * l.cout * (l.cin1 + l.cin2)), dim3(256),
-                    (const float*)(d->w + l.w_off), l.wf, l.wb, l.cout, l.cin1 + l.cin2);
+// The BF16 copies of the masters, after one Adam step on them when `adam` is given.
+void update_params(pt_denoiser* d, const AdamArgs* adam) {
+    AllParams A{};
+    size_t most = 0;
+    for (int i = 0; i < kLayers; ++i) {
+        const Layer& l = d->L[(size_t)i];
+        const int cin = l.cin1 + l.cin2;
+        A.l[i] = LayerParams{(uint32_t)l.w_off, (uint32_t)l.cout, (uint32_t)cin, l.wf, l.wb};
+        most = std::max(most, (size_t)9 * l.cout * cin + (size_t)l.cout);
+    }
+    const dim3 grid((unsigned)((most + 255) / 256), kLayers);
+    if (adam)
+        ptk::launch(d->ctx, "k_dn_adam", k_params<true>, grid, dim3(256), A, d->w, (const float*)d->g, d->m, d->v, *adam);
+    else
+        ptk::launch(d->ctx, "k_dn_wcopy", k_params<false>, grid, dim3(256), A, d->w, (const float*)d->g, d->m, d->v,
+                    AdamArgs{});
 }
 
 int upload(pt_denoiser* d, float* dst, const float* src, size_t n) {
@@ -963,7 +1018,8 @@ pt_status pt_dn_create(pt_ctx* ctx, int max_batch, int max_height, int max_width
         return q;
     };
     d->w = reinterpret_cast<float*>(carve(off * 4));
-    d->g = reinterpret_cast<float*>(carve(off * 4));
+    d->g = reinterpret_cast<float*>(carve(off * 4 + 4));
+    d->loss = d->g + off;  // cleared with the gradients
     d->m = reinterpret_cast<float*>(carve(off * 4));
     d->v = reinterpret_cast<float*>(carve(off * 4));
     d->wbf = reinterpret_cast<u16*>(carve(off * 4));
@@ -974,7 +1030,6 @@ pt_status pt_dn_create(pt_ctx* ctx, int max_batch, int max_height, int max_width
     d->feat = reinterpret_cast<float*>(carve(P * kFeat * 4));
     d->tgt = reinterpret_cast<float*>(carve(P * 3 * 4));
     d->den = reinterpret_cast<float*>(carve(P * 3 * 4));
-    d->loss = reinterpret_cast<float*>(carve(64 * 4));
     u16* wb = d->wbf;
     for (Layer& l : d->L) {
         const size_t n = (size_t)9 * l.cout * (l.cin1 + l.cin2);
@@ -995,14 +1050,15 @@ pt_status pt_dn_create(pt_ctx* ctx, int max_batch, int max_height, int max_width
             for (int ci = 0; ci < 32; ++ci) h[d->L[10].w_off + ((size_t)t * kOutC + co) * 32 + ci] *= 0.1f;
     (void)hipSetDevice(ctx->device);
     hipError_t e = hipMemcpyAsync(d->w, h.data(), off * 4, hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(d->m, 0, off * 8, ctx->stream);  // m and v are adjacent
+    if (e == hipSuccess) e = hipMemsetAsync(d->m, 0, off * 4, ctx->stream);
+    if (e == hipSuccess) e = hipMemsetAsync(d->v, 0, off * 4, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) {
         ptk::dev_free(ctx, d->mem);
         delete d;
         return ptk::hip_fail(ctx, e, "pt_dn_create");
     }
-    refresh_bf16(d);
+    update_params(d, nullptr);
     *out = d;
     return PT_OK;
 }
@@ -1035,7 +1091,7 @@ pt_status pt_dn_set_params(pt_denoiser* d, const float* host, size_t n) {
     if (!d || !host || n != d->nparam) return PT_ERR_INVALID_ARG;
     int st = upload(d, d->w, host, n);
     if (st != PT_OK) return st;
-    refresh_bf16(d);
+    update_params(d, nullptr);
     hipError_t e = hipStreamSynchronize(d->ctx->stream);
     return e == hipSuccess ? PT_OK : dn_fail(d, ptk::hip_fail(d->ctx, e, "pt_dn_set_params"), d->ctx->err);
 }
@@ -1067,10 +1123,8 @@ pt_status pt_dn_gradients(pt_denoiser* d, const float* features, const float* ta
     st = upload(d, d->feat, features, P * kFeat);
     if (st == PT_OK) st = upload(d, d->tgt, target, P * 3);
     if (st != PT_OK) return st;
-    hipError_t e = hipMemsetAsync(d->g, 0, d->nparam * 4, ctx->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(d->loss, 0, 4, ctx->stream);
-    if (e != hipSuccess) return dn_fail(d, ptk::hip_fail(ctx, e, "pt_dn_gradients"), ctx->err);
-    forward(d, N, H, W);
+    hipError_t e = hipSuccess;
+    forward(d, N, H, W, true);
     ptk::launch(ctx, "k_dn_head", k_head, ew_grid(P), dim3(256), (const float*)d->feat, (const u16*)d->out,
                 (const float*)d->tgt, (float*)nullptr, d->gc, d->loss, P, d->loss_kind);
     backward(d, N, H, W);
@@ -1087,9 +1141,8 @@ pt_status pt_dn_train_step(pt_denoiser* d, const float* features, const float* t
     d->step += 1;
     const float b1 = 0.9f, b2 = 0.999f;
     const float c1 = 1.0f - std::pow(b1, (float)d->step), c2 = 1.0f - std::pow(b2, (float)d->step);
-    ptk::launch(d->ctx, "k_dn_adam", k_adam, ew_grid(d->nparam), dim3(256), d->w, (const float*)d->g, d->m, d->v,
-                d->nparam, lr, b1, b2, 1e-8f, c1, c2);
-    refresh_bf16(d);
+    const AdamArgs adam{lr, b1, b2, 1e-8f, c1, c2};
+    update_params(d, &adam);
     hipError_t e = hipStreamSynchronize(d->ctx->stream);
     return e == hipSuccess ? PT_OK : dn_fail(d, ptk::hip_fail(d->ctx, e, "pt_dn_train_step"), d->ctx->err);
 }
