@@ -336,78 +336,147 @@ __global__ void __launch_bounds__(kThreads, NC == 2 ? 2 : 3) k_conv_t(ConvArgs a
 }
 
 // ---------------------------------------------------------------------------------
-// Conv backward-weights: dW[t][co][ci] += sum over pixels of dZ[p][co] * X[p + tap t][ci]
-// (FP32 atomics), dbias[co] += sum of dZ[p][co] (tap 4 blocks). Grid: x = pixel
-// chunks, y = co tiles of 32, z = 9 taps x ci tiles of 32.
+// Conv backward-weights: dW[t][co][ci] = sum over pixels of dZ[p][co] * X[p + tap t][ci],
+// dbias[co] = sum of dZ[p][co]. Grid: x = pixel tiles of kWR rows x 32 columns, taken
+// in turn by a block, y = co tiles of 32, z = ci tiles of 32. The blocks of one x write
+// their sums to partial x (k_grad_sum adds the partials in order, so a gradient does
+// not depend on the order in which blocks end), or add them to the cleared gradient
+// with FP32 atomics when there is no memory for partials.
 struct WgradArgs {
     const u16* dZ;
     int Cout;
     const u16* X1;
     const u16* X2;
     int C1, C2;
-    float* dW;   // [9][Cout][C1 + C2]
-    float* dB;   // [Cout]
+    float* g;     // the layer's gradient: [9][Cout][C1 + C2], then [Cout]
+    float* part;  // gridDim.x copies of it, or null
     int N, H, W;
-    int chunk;   // pixels per block (multiple of 64)
-    int up1;     // X1 at half resolution, as in ConvArgs
+    int up1;      // X1 at half resolution, as in ConvArgs
 };
+constexpr int kWR = 4;          // pixel rows of a tile
+constexpr int kWThreads = 192;  // three waves, one per row of taps
 
-__global__ void __launch_bounds__(kThreads) k_conv_wgrad(WgradArgs a) {
-    __shared__ u16 s_dz[4][16][32 + 8];
-    __shared__ u16 s_x[4][16][32 + 8];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int P = a.N * a.H * a.W;
+// Pixels are the K dimension, so both MFMA operands are read transposed: a tile's dZ
+// and X (with its halo) go into LDS channel-major, pairs of neighbouring pixels per
+// 4-byte write, and all 9 taps run from the staged tile, each wave one row of taps: per
+// 16 pixels one 16-byte read of dZ and one of X with the pixel pairs beside it, from
+// which the left and right taps' 8 pixels are funnel-shifted, for 3 MFMAs. (The kernel
+// before staged both operands again for each tap and gathered them element by element;
+// X staged once per column offset instead of shifted took 398 us for the 11 layers.)
+// The next tile's loads are in flight under the MFMAs. LDS rows are 4 modulo 16 dwords
+// apart, so that 16 rows read in turn hit different banks. All 11 layers of a step, us
+// before and after with the partials' sum: 8 crops of 96 x 96 315 -> 215, 16 of 128 x 128
+// 651 -> 390, one of 32 x 32 77 -> 115 (its launches' latency; the step is shorter all the
+// same). Bound by the chain of a tile: loads, transposing writes, 24 MFMAs per wave.
+__global__ void __launch_bounds__(kWThreads) k_conv_wgrad(WgradArgs a) {
+    constexpr int ZP = kWR * 32 + 8;                    // row: kWR x 32 pixels
+    constexpr int XR = 48, XP = (kWR + 2) * XR + 8;     // row: kWR + 2 lines of pixels -8 .. 39 (-2 .. 33 used)
+    constexpr int NZ = kWR * 16 * 4, NX = (kWR + 2) * 18 * 4;  // staging tasks: line, pixel pair, 8 channels
+    constexpr int NZT = (NZ + kWThreads - 1) / kWThreads, NXT = (NX + kWThreads - 1) / kWThreads;
+    __shared__ __align__(16) u16 s_z[32 * ZP];
+    __shared__ __align__(16) u16 s_x[32 * XP];
+    const int lane = threadIdx.x & 63, dy = threadIdx.x >> 6;
     const int Cin = a.C1 + a.C2;
-    const int nci = (Cin + 31) / 32;
-    const int t = blockIdx.z / nci, ci0 = (blockIdx.z % nci) * 32;
-    const int co0 = blockIdx.y * 32;
-    const int dy = t / 3 - 1, dx = t % 3 - 1;
-    const int pbeg = blockIdx.x * a.chunk, pend = min(P, pbeg + a.chunk);
-    f16v acc = f16v{};
-    float bsum = 0.0f;  // lanes 0..31: this co's sum of dZ (tap 4 only)
-    const int lr = lane >> 2, lc = (lane & 3) * 8;  // staging: pixel row, 8-channel group
-    // each wave takes every 4th group of 16 pixels of the block's chunk
-    for (int g = pbeg + wave * 16; g < pend; g += 64) {
-        const int p = g + lr;
-        Frag dz, xv;
-        dz.u = make_uint4(0, 0, 0, 0);
-        xv.u = make_uint4(0, 0, 0, 0);
-        if (p < pend) {
-            if (co0 + lc < a.Cout) dz.u = *reinterpret_cast<const uint4*>(a.dZ + (size_t)p * a.Cout + co0 + lc);
-            const int n = p / (a.H * a.W), rem = p % (a.H * a.W);
-            const int y = rem / a.W + dy, x = rem % a.W + dx;
-            const int c = ci0 + lc;
-            if (y >= 0 && y < a.H && x >= 0 && x < a.W && c < Cin) {
-                const size_t q = ((size_t)n * a.H + y) * a.W + x;
-                const u16* src = c < a.C1 ? a.X1 + up_index(a.up1, q, n, y, x, a.H, a.W) * a.C1 + c
-                                          : a.X2 + q * a.C2 + (c - a.C1);
-                xv.u = *reinterpret_cast<const uint4*>(src);
+    const int co0 = blockIdx.y * 32, ci0 = blockIdx.z * 32;
+    const int tiles_x = (a.W + 31) / 32, tiles_y = (a.H + kWR - 1) / kWR, ntiles = a.N * tiles_y * tiles_x;
+    const bool bias = ci0 == 0 && dy == 1;
+    f16v acc[3] = {f16v{}, f16v{}, f16v{}}, accb = f16v{};
+    Frag one;
+    one.u = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);  // BF16 ones
+    uint4 zr[NZT][2], xr[NXT][2];
+    auto fetch = [&](int tile) {
+        const int x0 = (tile % tiles_x) * 32, rest = tile / tiles_x;
+        const int y0 = (rest % tiles_y) * kWR, n = rest / tiles_y;
+#pragma unroll
+        for (int u = 0; u < NZT; ++u) {
+            const int i = threadIdx.x + u * kWThreads;
+            const int g = i & 3, px = (i >> 2) & 15, y = y0 + (i >> 6), x = x0 + 2 * px, c = co0 + g * 8;
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+                zr[u][k] = i < NZ && y < a.H && x + k < a.W && c < a.Cout
+                               ? *reinterpret_cast<const uint4*>(a.dZ + (((size_t)n * a.H + y) * a.W + x + k) * a.Cout + c)
+                               : make_uint4(0, 0, 0, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < NXT; ++u) {
+            const int i = threadIdx.x + u * kWThreads;
+            const int g = i & 3, px = (i >> 2) % 18, y = y0 + (i >> 2) / 18 - 1, c = ci0 + g * 8;
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const int x = x0 + 2 * px - 2 + k;
+                uint4 val = make_uint4(0, 0, 0, 0);
+                if (i < NX && y >= 0 && y < a.H && x >= 0 && x < a.W && c < Cin) {
+                    const size_t q = ((size_t)n * a.H + y) * a.W + x;
+                    const u16* src = c < a.C1 ? a.X1 + up_index(a.up1, q, n, y, x, a.H, a.W) * a.C1 + c
+                                              : a.X2 + q * a.C2 + (c - a.C1);
+                    val = *reinterpret_cast<const uint4*>(src);
+                }
+                xr[u][k] = val;
             }
         }
-        *reinterpret_cast<uint4*>(&s_dz[wave][lr][lc]) = dz.u;
-        *reinterpret_cast<uint4*>(&s_x[wave][lr][lc]) = xv.u;
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
-        Frag A, B;
-        const int kq = (lane >> 5) * 8, col = lane & 31;
+    };
+    // channels 8 g .. 8 g + 7 of a pixel pair into rows 8 g .. of dst at `at`
+    auto put = [](u16* dst, int pitch, int g, int at, uint4 p0, uint4 p1) {
+        const uint32_t u[4] = {p0.x, p0.y, p0.z, p0.w}, v[4] = {p1.x, p1.y, p1.z, p1.w};
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            reinterpret_cast<u16*>(&A.u)[i] = s_dz[wave][kq + i][col];
-            reinterpret_cast<u16*>(&B.u)[i] = s_x[wave][kq + i][col];
+        for (int k = 0; k < 4; ++k) {
+            *reinterpret_cast<uint32_t*>(&dst[(g * 8 + 2 * k) * pitch + at]) = (u[k] & 0xffffu) | (v[k] << 16);
+            *reinterpret_cast<uint32_t*>(&dst[(g * 8 + 2 * k + 1) * pitch + at]) = (u[k] >> 16) | (v[k] & 0xffff0000u);
         }
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.v, B.v, acc, 0, 0, 0);
-        if (t == 4 && blockIdx.z % nci == 0 && lane < 32)
-            for (int i = 0; i < 16; ++i) bsum += bf2f(s_dz[wave][i][lane]);
-        __builtin_amdgcn_wave_barrier();
+    };
+    const int row = lane & 31, kq = (lane >> 5) * 8;
+    if ((int)blockIdx.x < ntiles) fetch(blockIdx.x);
+    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        __syncthreads();  // every wave is done with the previous tile
+#pragma unroll
+        for (int u = 0; u < NZT; ++u) {
+            const int i = threadIdx.x + u * kWThreads;
+            if (i < NZ) put(s_z, ZP, i & 3, (i >> 6) * 32 + 2 * ((i >> 2) & 15), zr[u][0], zr[u][1]);
+        }
+#pragma unroll
+        for (int u = 0; u < NXT; ++u) {
+            const int i = threadIdx.x + u * kWThreads;
+            if (i < NX) put(s_x, XP, i & 3, (i >> 2) / 18 * XR + 2 * ((i >> 2) % 18) + 6, xr[u][0], xr[u][1]);
+        }
+        __syncthreads();
+        if (tile + (int)gridDim.x < ntiles) fetch(tile + gridDim.x);
+#pragma unroll
+        for (int r = 0; r < kWR; ++r) {
+#pragma unroll
+            for (int k = 0; k < 32; k += 16) {
+                Frag A, L, C, R;
+                A.u = *reinterpret_cast<const uint4*>(&s_z[row * ZP + r * 32 + k + kq]);
+                const u16* xp = &s_x[row * XP + (r + dy) * XR + 8 + k + kq];
+                C.u = *reinterpret_cast<const uint4*>(xp);
+                const uint32_t before = *reinterpret_cast<const uint32_t*>(xp - 2);
+                const uint32_t after = *reinterpret_cast<const uint32_t*>(xp + 8);
+                // 8 pixels from one to the left and one to the right
+                auto shift = [](uint32_t lo, uint32_t hi) { return __builtin_amdgcn_alignbit(hi, lo, 16); };
+                L.u = make_uint4(shift(before, C.u.x), shift(C.u.x, C.u.y), shift(C.u.y, C.u.z), shift(C.u.z, C.u.w));
+                R.u = make_uint4(shift(C.u.x, C.u.y), shift(C.u.y, C.u.z), shift(C.u.z, C.u.w), shift(C.u.w, after));
+                acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.v, L.v, acc[0], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.v, C.v, acc[1], 0, 0, 0);
+                acc[2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.v, R.v, acc[2], 0, 0, 0);
+                if (bias) accb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.v, one.v, accb, 0, 0, 0);
+            }
+        }
     }
+    const int nw = 9 * a.Cout * Cin;
+    float* part = a.part ? a.part + (size_t)blockIdx.x * (nw + a.Cout) : nullptr;
+    auto sink = [&](int j, float v) {
+        if (part) part[j] = v;
+        else if (v != 0.0f) atomicAdd(&a.g[j], v);
+    };
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
         const int co = co0 + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3), ci = ci0 + (lane & 31);
-        if (co < a.Cout && ci < Cin && acc[v] != 0.0f) atomicAdd(&a.dW[((size_t)t * a.Cout + co) * Cin + ci], acc[v]);
+        if (co >= a.Cout) continue;
+        if (ci < Cin) {
+#pragma unroll
+            for (int s = 0; s < 3; ++s) sink(((dy * 3 + s) * a.Cout + co) * Cin + ci, acc[s][v]);
+        }
+        if (bias && (lane & 31) == 0) sink(nw + co, accb[v]);
     }
-    if (t == 4 && blockIdx.z % nci == 0 && lane < 32 && co0 + lane < a.Cout && bsum != 0.0f)
-        atomicAdd(&a.dB[co0 + lane], bsum);
 }
 
 // ---------------------------------------------------------------------------------
@@ -563,6 +632,33 @@ constexpr int kLayers = 11;
 struct AllParams {
     LayerParams l[kLayers];
 };
+// The gradients from k_conv_wgrad's partials, one launch for the network: blockIdx.y is
+// the layer, a block adds 32 parameters' partials in 8 slices and the slices in order.
+struct PartialSums {
+    struct {
+        const float* part;
+        uint32_t off, n, count;  // first parameter, parameters, partials
+    } l[kLayers];
+};
+__global__ void __launch_bounds__(kThreads) k_grad_sum(PartialSums A, float* g) {
+    __shared__ float s_p[8][32];
+    const auto l = A.l[blockIdx.y];
+    const uint32_t j = blockIdx.x * 32 + (threadIdx.x & 31), slice = threadIdx.x >> 5;
+    if (blockIdx.x * 32 >= l.n) return;  // the whole block
+    float t = 0.0f;
+    if (j < l.n) {
+        const uint32_t per = (l.count + 7) / 8, b0 = slice * per, b1 = min(b0 + per, l.count);
+#pragma unroll 8
+        for (uint32_t b = b0; b < b1; ++b) t += l.part[(size_t)b * l.n + j];
+    }
+    s_p[slice][threadIdx.x & 31] = t;
+    __syncthreads();
+    if (slice == 0 && j < l.n) {
+        for (int k = 1; k < 8; ++k) t += s_p[k][threadIdx.x];
+        g[l.off + j] = t;
+    }
+}
+
 struct AdamArgs {
     float lr, b1, b2, eps, c1, c2;
 };
@@ -754,18 +850,32 @@ void conv(pt_denoiser* d, const Layer& l, const u16* x1, const u16* x2, u16* y, 
     }
 }
 
-void wgrad(pt_denoiser* d, const Layer& l, const u16* dz, const u16* x1, const u16* x2, int N, int H, int W) {
+// Blocks of a layer's k_conv_wgrad over all its channel tiles, and so the memory of its
+// partials (36 KB a block): 256, and 512 where those take more than 8 tiles each. A tile
+// costs a block about 3 us, a partial the sum's reading of it: 8 crops of 96 x 96 with
+// 128 / 256 / 512 blocks a layer 270 / 193 / 168 us and 18 / 24 / 35 us for the sum.
+dim3 wgrad_grid(const Layer& l, int N, int H, int W) {
+    const int cot = (l.cout + 31) / 32, cit = (l.cin1 + l.cin2 + 31) / 32;
+    const int tiles = N * ((H + kWR - 1) / kWR) * ((W + 31) / 32);
+    const int blocks = (int64_t)tiles * cot * cit >= 2048 ? 512 : 256;
+    return dim3((unsigned)std::min(tiles, std::max(1, blocks / (cot * cit))), cot, cit);
+}
+// The level of a layer: its resolution is the image's over 1, 2 or 4.
+constexpr int kLevel[kLayers] = {0, 0, 1, 1, 2, 2, 1, 1, 0, 0, 0};
+size_t layer_params(const Layer& l) { return (size_t)9 * l.cout * (l.cin1 + l.cin2) + l.cout; }
+
+// `part`: the partials of all layers, one after the other (null: atomics).
+void wgrad(pt_denoiser* d, int layer, const u16* dz, const u16* x1, const u16* x2, int N, int H, int W, float*& part) {
+    const Layer& l = d->L[(size_t)layer];
     WgradArgs a{};
     a.dZ = dz; a.Cout = l.cout; a.X1 = x1; a.X2 = x2; a.C1 = l.cin1; a.C2 = l.cin2;
     a.up1 = l.up1 ? 1 : 0;
-    a.dW = d->g + l.w_off; a.dB = d->g + l.b_off;
+    a.g = d->g + l.w_off;
+    a.part = part;
     a.N = N; a.H = H; a.W = W;
-    const int P = N * H * W;
-    const int cin = l.cin1 + l.cin2;
-    // about 2048 pixels per block, at least 16 blocks per (tap, tile)
-    a.chunk = std::max(64, std::min(2048, (P / 16 + 63) / 64 * 64));
-    dim3 grid((P + a.chunk - 1) / a.chunk, (l.cout + 31) / 32, 9 * ((cin + 31) / 32));
-    ptk::launch(d->ctx, "k_dn_wgrad", k_conv_wgrad, grid, dim3(kThreads), a);
+    const dim3 grid = wgrad_grid(l, N, H, W);
+    if (part) part += grid.x * layer_params(l);
+    ptk::launch(d->ctx, "k_dn_wgrad", k_conv_wgrad, grid, dim3(kWThreads), a);
 }
 
 dim3 ew_grid(size_t n) { return dim3((unsigned)std::min<size_t>((n + 255) / 256, 8192)); }
@@ -796,40 +906,68 @@ void forward(pt_denoiser* d, int N, int H, int W, bool grads = false) {
 // Backward pass: d->gc holds dL/d(out) (kOutC channels); gradients summed into d->g.
 void backward(pt_denoiser* d, int N, int H, int W) {
     pt_ctx* ctx = d->ctx;
+    // the weight gradients' partials, in the context's scratch memory until they are summed;
+    // without it (a budget) the layers add to the gradients with atomics
+    PartialSums sums{};
+    size_t floats = 0;
+    for (int i = 0; i < kLayers; ++i)
+        floats += wgrad_grid(d->L[(size_t)i], N, H >> kLevel[i], W >> kLevel[i]).x * layer_params(d->L[(size_t)i]);
+    ptk::ScratchUse scratch(ctx);
+    const std::string err = ctx->err;
+    const bool partials = scratch.take(floats * sizeof(float)) == PT_OK;
+    if (!partials) {
+        (void)hipGetLastError();
+        ctx->err = err;
+    }
+    float* part = partials ? static_cast<float*>(scratch.p) : nullptr;
+    uint32_t most = 0;
+    const float* at = part;
+    for (const int i : {10, 9, 8, 7, 6, 5, 4, 3, 2, 1, 0}) {  // the order of the layers below
+        const Layer& l = d->L[(size_t)i];
+        const uint32_t n = (uint32_t)layer_params(l), count = wgrad_grid(l, N, H >> kLevel[i], W >> kLevel[i]).x;
+        sums.l[i].part = at;
+        sums.l[i].off = (uint32_t)l.w_off;
+        sums.l[i].n = n;
+        sums.l[i].count = count;
+        if (at) at += (size_t)n * count;
+        most = std::max(most, n);
+    }
     const int P = N * H * W, P1 = P / 4, P2 = P / 16;
     const int H1 = H / 2, W1 = W / 2, H2 = H / 4, W2 = W / 4;
     // Each conv's gradient with respect to its input goes through the ReLU that
     // produced that input as it is stored (the mask), into the other of ga / gb.
     // out = conv10(d0): no activation
-    wgrad(d, d->L[10], d->gc, d->d0, nullptr, N, H, W);
+    wgrad(d, 10, d->gc, d->d0, nullptr, N, H, W, part);
     conv(d, d->L[10], d->gc, nullptr, d->gb, N, H, W, true, nullptr, 0, d->d0);    // dZ9
-    wgrad(d, d->L[9], d->gb, d->d0a, nullptr, N, H, W);
+    wgrad(d, 9, d->gb, d->d0a, nullptr, N, H, W, part);
     conv(d, d->L[9], d->gb, nullptr, d->ga, N, H, W, true, nullptr, 0, d->d0a);    // dZ8
-    wgrad(d, d->L[8], d->ga, d->d1, d->e0, N, H, W);
+    wgrad(d, 8, d->ga, d->d1, d->e0, N, H, W, part);
     conv(d, d->L[8], d->ga, nullptr, d->gc, N, H, W, true, d->gs0, 64);  // dL/d up(d1) (64) | dL/d e0 via skip (32)
     ptk::launch(ctx, "k_dn_up_bwd", k_up2_bwd, ew_grid((size_t)P1 * 64 / 8), dim3(256), (const u16*)d->gc,
                 (const u16*)d->d1, d->gb, N, H1, W1, 64);                // dZ7
-    wgrad(d, d->L[7], d->gb, d->d1a, nullptr, N, H1, W1);
+    wgrad(d, 7, d->gb, d->d1a, nullptr, N, H1, W1, part);
     conv(d, d->L[7], d->gb, nullptr, d->ga, N, H1, W1, true, nullptr, 0, d->d1a);  // dZ6
-    wgrad(d, d->L[6], d->ga, d->bb, d->e1, N, H1, W1);
+    wgrad(d, 6, d->ga, d->bb, d->e1, N, H1, W1, part);
     conv(d, d->L[6], d->ga, nullptr, d->gc, N, H1, W1, true, d->gs1, 128);  // dL/d up(bb) (128) | dL/d e1 via skip (64)
     ptk::launch(ctx, "k_dn_up_bwd", k_up2_bwd, ew_grid((size_t)P2 * 128 / 8), dim3(256), (const u16*)d->gc,
                 (const u16*)d->bb, d->gb, N, H2, W2, 128);               // dZ5
-    wgrad(d, d->L[5], d->gb, d->ba, nullptr, N, H2, W2);
+    wgrad(d, 5, d->gb, d->ba, nullptr, N, H2, W2, part);
     conv(d, d->L[5], d->gb, nullptr, d->ga, N, H2, W2, true, nullptr, 0, d->ba);   // dZ4
-    wgrad(d, d->L[4], d->ga, d->p2, nullptr, N, H2, W2);
+    wgrad(d, 4, d->ga, d->p2, nullptr, N, H2, W2, part);
     conv(d, d->L[4], d->ga, nullptr, d->gc, N, H2, W2, true);            // dL/d p2 (64)
     ptk::launch(ctx, "k_dn_pool_bwd", k_pool2_bwd, ew_grid((size_t)P1 * 64 / 8), dim3(256), (const u16*)d->gc,
                 (const u16*)d->gs1, (const u16*)d->e1, d->gb, N, H1, W1, 64);  // dZ3 (pool + skip)
-    wgrad(d, d->L[3], d->gb, d->e1a, nullptr, N, H1, W1);
+    wgrad(d, 3, d->gb, d->e1a, nullptr, N, H1, W1, part);
     conv(d, d->L[3], d->gb, nullptr, d->ga, N, H1, W1, true, nullptr, 0, d->e1a);  // dZ2
-    wgrad(d, d->L[2], d->ga, d->p1, nullptr, N, H1, W1);
+    wgrad(d, 2, d->ga, d->p1, nullptr, N, H1, W1, part);
     conv(d, d->L[2], d->ga, nullptr, d->gc, N, H1, W1, true);            // dL/d p1 (32)
     ptk::launch(ctx, "k_dn_pool_bwd", k_pool2_bwd, ew_grid((size_t)P * 32 / 8), dim3(256), (const u16*)d->gc,
                 (const u16*)d->gs0, (const u16*)d->e0, d->gb, N, H, W, 32);    // dZ1 (pool + skip)
-    wgrad(d, d->L[1], d->gb, d->e0a, nullptr, N, H, W);
+    wgrad(d, 1, d->gb, d->e0a, nullptr, N, H, W, part);
     conv(d, d->L[1], d->gb, nullptr, d->ga, N, H, W, true, nullptr, 0, d->e0a);    // dZ0
-    wgrad(d, d->L[0], d->ga, d->x0, nullptr, N, H, W);
+    wgrad(d, 0, d->ga, d->x0, nullptr, N, H, W, part);
+    if (partials)
+        ptk::launch(ctx, "k_dn_grad_sum", k_grad_sum, dim3((most + 31) / 32, kLayers), dim3(kThreads), sums, d->g);
 }
 
 // The BF16 copies of the masters, after one Adam step on them when `adam` is given.

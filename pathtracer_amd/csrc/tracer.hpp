@@ -163,10 +163,11 @@ namespace ptk {
 // PT_ERR_BUDGET or PT_ERR_HIP (message in ctx->err).
 int dev_alloc(pt_ctx* ctx, DevAlloc& a, size_t bytes);
 void dev_free(pt_ctx* ctx, DevAlloc& a);
-// The context's scratch memory for the length of a call, which has waited for its
-// work on the stream when it ends: kept between calls up to kScratchKeep (an
-// allocation and a free cost more than a small call's kernels), and given back
-// when another allocation needs the room.
+// The context's scratch memory for the length of a call, whose last use of it is
+// enqueued on the context's stream when it ends (the next user comes after it on that
+// stream, and hipFree waits for the device): kept between calls up to kScratchKeep (an
+// allocation and a free cost more than a small call's kernels), and given back when
+// another allocation needs the room.
 constexpr size_t kScratchKeep = (size_t)512 << 20;
 struct ScratchUse {
     pt_ctx* ctx;
