@@ -829,25 +829,31 @@ void conv(pt_denoiser* d, const Layer& l, const u16* x1, const u16* x2, u16* y, 
         a.Y1 = y; a.Y2 = y2; a.Co1 = co1 ? co1 : l.cin1 + l.cin2; a.Cout = l.cin1 + l.cin2;
         a.relu = 0; a.flip = 1; a.mask = mask;
     }
-    // tiles of 8 x 32 pixels x 64 output channels (32 below 64 channels); each
-    // block takes consecutive tiles so that the grid is about two rounds of the
-    // blocks the CUs hold at once (2 per CU at 64 channels, 3 at 32), at most 16
-    constexpr int kTH = 8;
-    const int nc = a.Cout >= 64 ? 2 : 1;
-    const int ntiles = N * ((H + kTH - 1) / kTH) * ((W + 31) / 32);
-    const int cotiles = (a.Cout + 32 * nc - 1) / (32 * nc);
-    const int64_t resident = (int64_t)d->cus * (nc == 2 ? 2 : 3);
-    const int64_t want = ((int64_t)ntiles * cotiles + 2 * resident - 1) / (2 * resident);
+    // Tiles of 8 x 32 pixels x 64 output channels (32 below 64 channels). A grid of those
+    // that leaves compute units idle (training crops: 48 blocks on the quarter-resolution
+    // layers of 8 crops of 96 x 96) takes 32 channels a block, then 4 rows: the same sums
+    // in the same order, more blocks and shorter chains in each. All layers of a forward
+    // pass (of a training step for the crops), us before and after: 64x64 149 -> 96,
+    // 256x256 155 -> 105, 512x512 206 -> 186, 1024x768 403 -> 396, 1920x1080 the same;
+    // 8 crops of 96x96 312 -> 233, 16 of 128x128 407 -> 383. Splitting from fewer blocks on
+    // (1 and 1 per compute unit) left 249 for the 8 crops.
     const bool one = a.C1 + a.C2 <= 32;  // one input chunk: the weights stay in LDS for all the block's tiles
+    auto ntiles = [&](int th) { return N * ((H + th - 1) / th) * ((W + 31) / 32); };
+    auto cotiles = [&](int nc) { return (a.Cout + 32 * nc - 1) / (32 * nc); };
+    int nc = a.Cout >= 64 ? 2 : 1, th = 8;
+    if (nc == 2 && ntiles(8) * cotiles(2) < 2 * d->cus) nc = 1;
+    if (nc == 1 && ntiles(8) * cotiles(1) < 2 * d->cus) th = 4;
+    // each block takes consecutive tiles so that the grid is about two rounds of the
+    // blocks the CUs hold at once (2 per CU at 64 channels, 3 at 32), at most 16
+    const int tiles = ntiles(th);
+    const int64_t resident = (int64_t)d->cus * (nc == 2 ? 2 : 3);
+    const int64_t want = ((int64_t)tiles * cotiles(nc) + 2 * resident - 1) / (2 * resident);
     a.tiles_per_block = one ? (int)std::max<int64_t>(1, std::min<int64_t>(16, want)) : 1;
-    dim3 grid((unsigned)((ntiles + a.tiles_per_block - 1) / a.tiles_per_block), cotiles);
-    if (nc == 2) {
-        if (one) ptk::launch(d->ctx, "k_dn_conv", k_conv_t<2, kTH, true>, grid, dim3(kThreads), a);
-        else ptk::launch(d->ctx, "k_dn_conv", k_conv_t<2, kTH, false>, grid, dim3(kThreads), a);
-    } else {
-        if (one) ptk::launch(d->ctx, "k_dn_conv", k_conv_t<1, kTH, true>, grid, dim3(kThreads), a);
-        else ptk::launch(d->ctx, "k_dn_conv", k_conv_t<1, kTH, false>, grid, dim3(kThreads), a);
-    }
+    dim3 grid((unsigned)((tiles + a.tiles_per_block - 1) / a.tiles_per_block), cotiles(nc));
+    auto run = [&](auto kernel) { ptk::launch(d->ctx, "k_dn_conv", kernel, grid, dim3(kThreads), a); };
+    if (nc == 2) run(one ? k_conv_t<2, 8, true> : k_conv_t<2, 8, false>);
+    else if (th == 8) run(one ? k_conv_t<1, 8, true> : k_conv_t<1, 8, false>);
+    else run(one ? k_conv_t<1, 4, true> : k_conv_t<1, 4, false>);
 }
 
 // Blocks of a layer's k_conv_wgrad over all its channel tiles, and so the memory of its

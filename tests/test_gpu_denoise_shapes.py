@@ -1,6 +1,7 @@
-"""The denoiser's weight-gradient kernel at ragged sizes: images smaller than a tile,
-one more than a tile, several images; gradients against the FP64 oracle, bit-equal
-from run to run, and the atomics they fall back to without memory for partial sums."""
+"""The denoiser's weight-gradient and convolution kernels at ragged sizes: images
+smaller than a tile, one more than a tile, several images; gradients against the
+FP64 oracle, bit-equal from run to run, the atomics they fall back to without memory
+for partial sums, and images computed alone (small tiles) and in a batch (large ones)."""
 import numpy as np
 import pytest
 
@@ -49,3 +50,14 @@ def test_atomics_without_memory_for_partials():
     with pt.Context(0, hbm_budget=20 << 20) as ctx:  # the denoiser takes 17 MB, the partials more than the rest
         _, a = gradients(ctx, n, h, w, p, feat, target)
     assert np.linalg.norm(a - g) <= 4080 * 2.0 ** -24 * np.linalg.norm(g)
+
+
+@pytest.mark.gpu
+def test_a_batch_equals_its_images(gpu_ctx):
+    rng = np.random.default_rng(5)
+    feat = random_features(rng, 24, 96, 160)
+    with pt.Denoiser(gpu_ctx, 24, 96, 160) as dn:
+        dn.set_params(random_params(rng).astype(np.float32))
+        batch = dn.denoise(feat)
+        for i in (0, 7, 23):
+            np.testing.assert_array_equal(dn.denoise(feat[i:i + 1])[0].view(np.uint32), batch[i].view(np.uint32))
