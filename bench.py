@@ -74,6 +74,8 @@ BYTES_PER_UNIT = {
     # reference mode: a path stays in its lane's registers and leaves its XYZ, 16 B, which the
     # fold reads (the kernel is bound by VALU issue, the shader's transcendentals restated)
     "k_ref_path": [(16, "paths")],
+    # extended mode's whole paths: the same
+    "k_ext_path": [(16, "paths")],
     "k_ref_fold": [(16, "paths")],
 }
 

@@ -78,7 +78,8 @@ struct ExtLight {
     float area, radius;
 };
 struct ExtSdf {
-    int kind, iters, mat, pad;
+    int kind, iters, mat;
+    int next;  // the SDF marched after this one by an extension ray (kind by kind), -1 none
     float bailout;
     f3 lo, hi, c;
 };
@@ -126,6 +127,7 @@ struct ExtSceneDev {
     BvhDev sbvh, qbvh;
     int nsph, nquad, nplane, nsdf, nmat, nlight;
     int nlens, ncyc;
+    int sdf_first;  // the SDF an extension ray marches first, -1 none
     int nlight_nee;     // lights [0, nlight_nee) are sampled by next-event estimation
     int quad_bvh;       // parallelograms go through qbvh
     int has_env;
@@ -1107,8 +1109,8 @@ __global__ void k_ext_counts(int* counts, int n0, unsigned long long* stats, int
     if (i == 0 && count_dispatch) atomicAdd(&stats[5], 1ull);
 }
 // Zeroes the whole-path kernel's cursors in new wave memory (a kernel, not a memset).
-__global__ void k_ext_clear(int* cursor) {
-    for (int j = (int)threadIdx.x; j < kPathCursors; j += blockDim.x) cursor[(CUR_PATH * kSeg + j) * kCntStride] = 0;
+__global__ void k_ext_clear(int* cursor, int n) {
+    for (int j = (int)threadIdx.x; j < n; j += blockDim.x) cursor[j * kCntStride] = 0;
 }
 // Start of bounce b: empty the next extension queue, the material queues, the
 // shadow queue bounce b appends to (read by bounce b - 1 at the latest), and
@@ -2354,12 +2356,15 @@ struct ExtFinish {
     int spf, currentSamples, frame, ISO;
     float apSize, FPS, persistence;
 };
-__device__ __forceinline__ float4 finish_texel(const ExtFinish& F, f3 sum, float4 tx) {
+// The persistence blend's weight of the texel that is there; the same for all texels.
+__device__ __forceinline__ float blend_weight(const ExtFinish& F) {
+    return F.currentSamples == F.spf && F.frame > F.spf ? ptm_pow(2.0f, -8.0f / (F.FPS * F.persistence)) : 0.0f;
+}
+__device__ __forceinline__ float4 finish_texel(const ExtFinish& F, f3 sum, float4 tx, float wgt) {
     float e = F.apSize * F.apSize * (float)F.ISO / (float)F.spf;
     f3 out = sum * e;
     f3 in = mk3(tx.x, tx.y, tx.z);
     if (F.currentSamples == F.spf && F.frame > F.spf) {
-        float wgt = ptm_pow(2.0f, -8.0f / (F.FPS * F.persistence));
         out = (1.0f - wgt) * out + wgt * in;
     } else {
         int u = F.currentSamples / F.spf;
@@ -2370,190 +2375,305 @@ __device__ __forceinline__ float4 finish_texel(const ExtFinish& F, f3 sum, float
 
 // A lane's state in k_ext_path, what it does next.
 enum : int {
-    LS_IDLE,    // takes a path from the queue
-    LS_HIT,     // its extension ray's nearest sphere is known
-    LS_SHADOW,  // its shadow ray's visibility is known
-    LS_DONE,    // its path has ended and is to be stored
-    LS_EXT,     // traversal, extension ray
-    LS_ANY,     // traversal, shadow ray
+    LS_IDLE,   // takes a path from the queue
+    LS_SEEK,   // its ray leaves the BVH or an SDF: planes, then the next SDF's box
+    LS_END,    // its ray's nearest hit or visibility is known
+    LS_DONE,   // its path has ended and is to be stored
+    LS_BVH,    // traversal
+    LS_MARCH,  // an SDF's march
 };
 constexpr int kPathLanes = 64;  // threads per block: one wave, so that few paths spread over all compute units
 constexpr int kPathStack = 32;
-// Lanes waiting for scene work before a wave does it, or as many as traverse (24: 13 %
-// slower on the 4096-sphere scene, 40 and 48 the same: half the wave then decides), and
-// ended lanes before they are stored and refilled (8 / 16 / 32: Cornell box 3.03 / 2.89 /
-// 2.94 ms, 1000-sphere features 4.57 / 4.70 / 5.93 ms).
-constexpr int kPathScene = 32, kPathRefill = 16;
+// A wave does its scene work when three lanes wait for it for each one that traverses
+// or marches (from 24 / 32 / 43 / 48 / 53 of 64 waiting: 1080p SDFs, 16 samples, 15.5 /
+// 14.2 / 13.2 / 13.3 / 13.9 ms), and stores and refills from 12 ended lanes on (8 / 12 /
+// 16: Cornell box 2.66 / 2.61 / 2.54 ms, 1080p 4096 spheres 46.2 / 46.7 / 47.4 ms).
+// Between those looks it takes 4 BVH visits (1 / 2 / 4 / 6: 51.5 / 48.6 / 47.3 / 46.9 ms,
+// Cornell box 2.54 / 2.59 / 2.62 / 2.66) and 2 march steps.
+constexpr int kPathScene = 3, kPathRefill = 12;
+constexpr int kPathSteps = 2, kPathVisits = 4;
 
 // Whole paths: scenes of spheres (binary BVH, 16-bit nodes), at most kQuadBrute
-// parallelograms and planes. A lane keeps its path in registers from the camera to its
-// end, with the device functions of the per-bounce kernels in the order in which they
-// would take it, so its XYZ is theirs bit for bit. Every iteration visits one BVH node
-// of each traversing lane (extension and shadow rays alike); the others wait for the
-// scene work (hits, shading, new rays and paths).
-// It is bound by VALU issue with 19 of 64 lanes active (rocprofv3, 4096 spheres: the
-// scene work runs each material's code for the few of the waiting lanes that need it),
-// against the persistent traversal kernels' 35; but it has one launch where they have
-// nine a bounce, each as long as its slowest ray, and no path state in memory. Rule
-// (ext_run): dispatches of at most kWholePaths, or any size with at most kWholeSpheres
-// spheres. Depth 12, 1 to 4096 spheres, wavefront against whole, with the read-back of
-// the display image: 160x90x1 646-1835 against 204-602 us, 640x360x1 787-2270 against
-// 240-829 us, 1920x1080x1 1.4-3.7 against 0.9-2.0 ms, x4 2.5-6.0 against 1.8-4.9 ms; at
-// x16 the whole-path kernel is slower from 30 spheres on (7.6-14.7 against 8.9-16.4 ms)
-// and faster with 3 (6.5 against 5.5 ms). Cornell box, 512x512x64: 4.4 against 2.9 ms.
-// Splitting the waiting lanes by material so that each material's code runs at 16 lanes
-// or more took 152 registers and was 20 % slower.
+// parallelograms, planes and SDFs. A lane keeps its path in registers from the camera to
+// its end, with the device functions of the per-bounce kernels in the order in which they
+// would take it, so its XYZ is theirs bit for bit. Every iteration visits BVH nodes for
+// the traversing lanes and steps the marching ones (extension and shadow rays alike); the
+// others wait for the scene work (hits, shading, new rays and paths). It is bound by VALU
+// issue, with the lanes of a wave in different states and materials, where the kernels per
+// stage keep more lanes busy; but it has one launch where they have nine a bounce, each as
+// long as its slowest ray (about 0.3 ms for a march of 256 steps), and no path state in
+// memory. The scene and frame come through scalar loads where they are used, not as
+// by-value arguments loaded at the start, which filled the scalar registers and spilled
+// into vector ones (120 against 96 VGPRs, 4 against 5 waves per SIMD).
+// Rule (whole_takes, ext_run): scenes without SDFs at any size, with SDFs dispatches of at
+// most kWholeSdfPaths: a large wave hides the marches' tails, and the march kernels keep
+// their lanes on one estimator. Kernels per stage against this one, ms, 1920 x 1080 at
+// depth 12 with 4 / 16 / 64 samples: 30 spheres 2.81 / 7.38 / 25.6 against 1.64 / 5.63 /
+// 21.8, 300 4.03 / 10.9 / 37.4 against 2.69 / 9.25 / 35.9, 1000 5.07 / 13.3 / 46.2 against
+// 3.44 / 11.9 / 46.0, 4096 5.95 / 14.5 / 49.2 against 3.65 / 12.2 / 46.7; mandelbulb and
+// menger at depth 8 with 1 / 4 / 16 / 32 / 64 samples 5.3 / 7.4 / 15.2 / 24.9 / 44.1 against
+// 1.5 / 3.8 / 12.7 / 24.6 / 48.5. Batched waves of a served burst 32.1 against 10.5 ms.
 // `direct`: the dispatch has one sample per pixel, all in this wave, and the paths'
 // texels are finished here instead of by k_ext_fold.
-constexpr int kWholePaths = 1 << 23, kWholeSpheres = 8;
-__global__ void __launch_bounds__(kPathLanes, 4) k_ext_path(ExtSceneDev S, ExtFrame F, ExtWave Wv, ExtFinish Fin,
-                                                          float4* texels, int direct, int aov, int count_dispatch) {
+constexpr int kWholeSdfPaths = 1 << 25;
+// A batched wave's tables (in constant memory for the kernel's length, so that a
+// request's scene comes through scalar loads), and its cursors: kSeg a request, then the
+// count of ended waves.
+#define PT_RO const __attribute__((address_space(4)))
+struct ExtPathBatch {
+    PT_RO ExtSceneDev* scenes;
+    PT_RO ExtFrame* frames;
+    PT_RO ExtSeg* segs;
+    PT_RO ExtBatchHdr* hdr;
+    int* cursor;
+};
+constexpr int kBatchCursors = kMaxBatch * kSeg + 1;
+template <bool MULTI, bool SDF>
+__global__ void __launch_bounds__(kPathLanes, 5) k_ext_path(ExtFrame F0, ExtWave Wv, ExtFinish Fin,
+                                                            float4* texels, int direct, int aov, int count_dispatch,
+                                                            ExtPathBatch PB) {
     __shared__ uint16_t stack_mem[kPathStack * kPathLanes];
     __shared__ float4 s_quad[4 * kQuadBrute];
+    // a lane's march operations: per kind for extension rays, then shadow rays
+    __shared__ unsigned long long s_flops[SDF ? 5 : 1][kPathLanes];
     uint16_t* stack = stack_mem + threadIdx.x;
-    const int nq = min(S.nquad, kQuadBrute);
-    for (int i = (int)threadIdx.x; i < 4 * nq; i += kPathLanes) s_quad[i] = S.quad[i];
-    __syncthreads();
-    const int n = F.pc * F.m;
+    const int nreq = MULTI ? PB.hdr->nseg : 1;
+    const int npaths = MULTI ? PB.hdr->npaths : F0.pc * F0.m;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        atomicAdd(&Wv.stats[3], (unsigned long long)n);
+        atomicAdd(&Wv.stats[3], (unsigned long long)npaths);
         if (count_dispatch) atomicAdd(&Wv.stats[5], 1ull);
     }
-    unsigned nseg = 0, nshadow = 0, nvis = 0, nsvis = 0, ncls[N_MATQ] = {}, nbad = 0, nnan = 0;  // wave totals
-    int st = LS_IDLE, p = 0, bounce = 0;
-    Vertex v{};
-    ShadowRay sh{};
-    f3 acc = mk3(0.0f, 0.0f, 0.0f), inv = acc, oi = acc;
-    bool cont = false, blocked = false;
-    float t = 0.0f;
-    uint32_t ref = kMiss;
-    int node = -1, sp = 0, best = -1;
-    // blocks of 64 consecutive paths are dealt to the queue's segments in turn, so that
-    // each segment, which only its own waves drain, holds a share of the whole image;
-    // entries past the last path are dropped
+    if (SDF)
+        for (int i = 0; i < 5; ++i) s_flops[i][threadIdx.x] = 0ull;
+    float wgt = 0.0f;
+    if (!MULTI && direct) wgt = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(blend_weight(Fin))));
+    // wave totals
+    unsigned nseg = 0, nshadow = 0, nvis = 0, nsvis = 0, ncls[N_MATQ] = {}, nbad = 0, nnan = 0, nsteps = 0, nexhausted = 0;
     const int nsegm = min(kSeg, (int)gridDim.x);
-    const int seg_blocks = ((n + 63) / 64 + nsegm - 1) / nsegm;
-    int* const cursor = Wv.cursor + CUR_PATH * kSeg * kCntStride;
-    WaveChunk chunk = wave_chunk_init(cursor, seg_blocks * nsegm * 64);
-    while (true) {
-        const int trav = (int)__popcll(__ballot(st >= LS_EXT));
-        const int wait = (int)__popcll(__ballot(st < LS_EXT && !(st == LS_IDLE && chunk.drained())));
-        if (trav == 0 || wait >= min(kPathScene, trav)) {
-            bool ext = false;  // an extension ray starts
-            if (st == LS_SHADOW) {
-                for (int k = 0; !blocked && k < S.nplane; ++k) {
-                    float tp = (ld_ro(S.plane_y + k) - sh.o.y) / sh.d.y;
-                    blocked = tp > kEps && tp < t;
-                }
-                if (!blocked) acc = mk3(acc.x + sh.c.x, acc.y + sh.c.y, acc.z + sh.c.z);
-                ext = cont;
-                if (!cont) st = LS_DONE;
-            }
-            int cls = -1;
-            bool shadow = false;
-            if (st == LS_HIT) {
-                if (best >= 0) ref = (REF_SPHERE << kRefShift) | (uint32_t)S.sbvh.ids[best];
-                for (int i = 0; i < S.nplane; ++i) {
-                    float tp = (ld_ro(S.plane_y + i) - v.o.y) / v.d.y;
-                    if (tp > kEps && tp < t) {
-                        t = tp;
-                        ref = (REF_PLANE << kRefShift) | (uint32_t)i;
+    int* const cursor = MULTI ? PB.cursor : Wv.cursor + CUR_PATH * kSeg * kCntStride;
+    // A wave takes one request's paths at a time, so that its scene is the wave's, and goes
+    // on to the next request when that one's queue has no more; the waves of a segment
+    // start spread over the requests by their paths.
+    int first = 0;
+    if (MULTI) {
+        const int rounds = ((int)gridDim.x + nsegm - 1) / nsegm;
+        const int at = (int)((int64_t)(blockIdx.x / nsegm) * npaths / rounds);
+        first = seg_find(nreq, at, [&](int k) { return PB.segs[k].base; });
+    }
+    for (int rq = 0; rq < nreq; ++rq) {
+        const int req = MULTI ? __builtin_amdgcn_readfirstlane(first + rq < nreq ? first + rq : first + rq - nreq) : 0;
+        const ExtSceneDev& S = *(const ExtSceneDev*)(PB.scenes + req);
+        const ExtFrame& F = *(const ExtFrame*)(MULTI ? PB.frames + req : (PT_RO ExtFrame*)__builtin_amdgcn_kernarg_segment_ptr());
+        const int pc = MULTI ? PB.segs[req].pc : F0.pc, k0 = MULTI ? PB.segs[req].k0 : F0.k0;
+        const int n = pc * (MULTI ? PB.segs[req].m : F0.m), base = MULTI ? PB.segs[req].base : 0;
+        const int p0 = MULTI ? PB.segs[req].p0 : F0.p0;
+        const int nq = min(S.nquad, kQuadBrute);
+        __syncthreads();
+        for (int i = (int)threadIdx.x; i < 4 * nq; i += kPathLanes) s_quad[i] = S.quad[i];
+        __syncthreads();
+        int st = LS_IDLE, p = 0, bounce = 0;
+        Vertex v{};
+        ShadowRay sh{};
+        f3 acc = mk3(0.0f, 0.0f, 0.0f);
+        bool cont = false, blocked = false, any = false;  // any: the ray is a shadow ray
+        float t = 0.0f;
+        uint32_t ref = kMiss;
+        // In the BVH: the ray's 1 / d and o / d, node, stack height and nearest sphere. In a
+        // march: the SDF's centre, (position, exit, bailout), index, steps and iterations * 16
+        // + kind.
+        f3 inv = acc, oi = acc;
+        int node = -1, sp = 0, best = -1;
+        unsigned it = 0;  // a march's estimator iterations
+        // blocks of 64 consecutive paths are dealt to the queue's segments in turn, so that
+        // each segment, which only its own waves drain, holds a share of the whole image;
+        // entries past the last path are dropped
+        const int seg_blocks = ((n + 63) / 64 + nsegm - 1) / nsegm;
+        WaveChunk chunk = wave_chunk_init(cursor + req * kSeg * kCntStride, seg_blocks * nsegm * 64);
+        while (true) {
+            const int trav = (int)__popcll(__ballot(st >= LS_BVH));
+            const int wait = (int)__popcll(__ballot(st < LS_BVH && !(st == LS_IDLE && chunk.drained())));
+            if (trav == 0 || wait >= kPathScene * trav) {
+                bool ended_all = false;
+                // with SDFs a second pass looks for the new rays' boxes when there is no BVH
+#pragma clang loop unroll(disable)
+                for (int pass = 0; pass < (SDF ? 2 : 1); ++pass) {
+                    if (st == LS_SEEK) {
+                        if (!SDF || node < 0) {
+                            if (any) {
+                                for (int k = 0; !blocked && k < S.nplane; ++k) {
+                                    float tp = (ld_ro(S.plane_y + k) - sh.o.y) / sh.d.y;
+                                    blocked = tp > kEps && tp < t;
+                                }
+                            } else {
+                                if (best >= 0) ref = (REF_SPHERE << kRefShift) | (uint32_t)S.sbvh.ids[best];
+                                for (int i = 0; i < S.nplane; ++i) {
+                                    float tp = (ld_ro(S.plane_y + i) - v.o.y) / v.d.y;
+                                    if (tp > kEps && tp < t) {
+                                        t = tp;
+                                        ref = (REF_PLANE << kRefShift) | (uint32_t)i;
+                                    }
+                                }
+                            }
+                        } else {
+                            s_flops[any ? 4 : (best & 15) - 1][threadIdx.x] +=
+                                (unsigned long long)(unsigned)sp * de_step_flops(best & 15, best >> 4) +
+                                (unsigned long long)it * de_iter_flops(best & 15);
+                        }
+                        st = LS_END;
+                        if (SDF && !(any && blocked)) {
+                            // shadow rays in scene order, extension rays kind by kind
+                            const f3 ro = any ? sh.o : v.o, rd = any ? sh.d : v.d;
+                            int s = any ? node + 1 : node < 0 ? S.sdf_first : S.sdf[node].next;
+                            while (s >= 0 && s < S.nsdf) {
+                                const ExtSdf& e = S.sdf[s];
+                                float tin, tout;
+                                if (sdf_box(e, ro, rd, t, tin, tout)) {
+                                    inv = e.c;
+                                    oi = mk3(tin, tout, e.bailout);
+                                    node = s;
+                                    sp = 0;
+                                    it = 0;
+                                    best = e.iters * 16 + e.kind;
+                                    st = LS_MARCH;
+                                    break;
+                                }
+                                s = any ? s + 1 : e.next;
+                            }
+                        }
                     }
-                }
-                cls = hit_class(S, ref);
-                if (bounce == 0 && aov) store_aov(S, Wv, p, ref, v.o, v.d, t);
-                cont = false;
-                if (cls == Q_MISS) {
-                    if (S.has_env) {
-                        const f3 c = shade_miss(S, v);
-                        acc = mk3(acc.x + c.x, acc.y + c.y, acc.z + c.z);
-                    }
-                } else if (cls == Q_EMIT) {
-                    const f3 c = shade_emit(S, v, ref, t);
-                    acc = mk3(acc.x + c.x, acc.y + c.y, acc.z + c.z);
-                } else if (cls == Q_LAMBERT) {
-                    cont = shade_lambert(S, v, ref, t, bounce, F.maxDepth, shadow, sh);
-                } else if (cls == Q_DIELECTRIC) {
-                    cont = shade_dielectric(S, v, ref, t, bounce, F.maxDepth);
-                } else {
-                    cont = shade_conductor(S, v, ref, t, bounce, F.maxDepth);
-                }
-                ++bounce;
-                st = LS_DONE;
-                ext = cont && !shadow;
-            }
-            nbad += (unsigned)__popcll(__ballot(cls >= 0 && ref_is_bad(S, ref)));
-#pragma unroll
-            for (int q = 0; q < N_MATQ; ++q) ncls[q] += (unsigned)__popcll(__ballot(cls == q));
-            nshadow += (unsigned)__popcll(__ballot(shadow));
-            // ended paths are stored, idle lanes refilled
-            const bool free_lane = st == LS_IDLE || (st == LS_DONE && !ext && !shadow);
-            const uint64_t idle = __ballot(free_lane);
-            if (__popcll(idle) >= kPathRefill || __ballot(st >= LS_EXT || ext || shadow) == 0ull) {
-                const bool ended = st == LS_DONE && free_lane;
-                if (direct) {
-                    const bool nan = acc.x != acc.x || acc.y != acc.y || acc.z != acc.z;
-                    nnan += (unsigned)__popcll(__ballot(ended && nan));
-                    if (ended) {
-                        // the sum over samples starts from zero and drops NaN samples
-                        const f3 sum = nan ? mk3(0.0f, 0.0f, 0.0f) : mk3(0.0f, 0.0f, 0.0f) + acc;
-                        texels[F.p0 + p] = finish_texel(Fin, sum, texels[F.p0 + p]);
-                    }
-                } else if (ended) {
-                    Wv.acc[p] = make_float4(acc.x, acc.y, acc.z, 0.0f);
-                }
-                if (ended) st = LS_IDLE;
-                if (!chunk.drained()) {
-                    const int e = wave_refill(idle, chunk);
-                    const int b = e >> 6;
-                    const int path = ((b % seg_blocks) * nsegm + b / seg_blocks) * 64 + (e & 63);
-                    if (e >= 0 && path < n) {
-                        p = path;
-                        camera_ray(S, F, F.p0 + p % F.pc, F.k0 + p / F.pc, v.o, v.d, v.l0, v.key);
-                        v.T = mk4(1.0f);
-                        v.flags = 2u;  // the camera ray counts as specular for emitter MIS
-                        v.pdf = 0.0f;
-                        acc = mk3(0.0f, 0.0f, 0.0f);
-                        bounce = 0;
+                    if (SDF && pass == 1) break;
+                    bool ext = false;  // an extension ray starts
+                    if (st == LS_END && any) {
+                        if (!blocked) acc = mk3(acc.x + sh.c.x, acc.y + sh.c.y, acc.z + sh.c.z);
+                        ext = cont;
                         st = LS_DONE;
-                        ext = F.maxDepth > 0;
+                    }
+                    int cls = -1;
+                    bool shadow = false;
+                    if (st == LS_END) {
+                        cls = hit_class(S, ref);
+                        if (bounce == 0 && aov) store_aov(S, Wv, p, ref, v.o, v.d, t);
+                        cont = false;
+                        if (cls == Q_MISS) {
+                            if (S.has_env) {
+                                const f3 c = shade_miss(S, v);
+                                acc = mk3(acc.x + c.x, acc.y + c.y, acc.z + c.z);
+                            }
+                        } else if (cls == Q_EMIT) {
+                            const f3 c = shade_emit(S, v, ref, t);
+                            acc = mk3(acc.x + c.x, acc.y + c.y, acc.z + c.z);
+                        } else if (cls == Q_LAMBERT) {
+                            cont = shade_lambert(S, v, ref, t, bounce, F.maxDepth, shadow, sh);
+                        } else if (cls == Q_DIELECTRIC) {
+                            cont = shade_dielectric(S, v, ref, t, bounce, F.maxDepth);
+                        } else {
+                            cont = shade_conductor(S, v, ref, t, bounce, F.maxDepth);
+                        }
+                        ++bounce;
+                        st = LS_DONE;
+                        ext = cont && !shadow;
+                    }
+                    nbad += (unsigned)__popcll(__ballot(cls >= 0 && ref_is_bad(S, ref)));
+#pragma unroll
+                    for (int q = 0; q < N_MATQ; ++q) ncls[q] += (unsigned)__popcll(__ballot(cls == q));
+                    nshadow += (unsigned)__popcll(__ballot(shadow));
+                    // ended paths are stored, idle lanes refilled
+                    const bool free_lane = st == LS_IDLE || (st == LS_DONE && !ext && !shadow);
+                    const uint64_t idle = __ballot(free_lane);
+                    if (__popcll(idle) >= kPathRefill || __ballot(st >= LS_BVH || ext || shadow) == 0ull) {
+                        const bool ended = st == LS_DONE && free_lane;
+                        if (!MULTI && direct) {
+                            const bool nan = acc.x != acc.x || acc.y != acc.y || acc.z != acc.z;
+                            nnan += (unsigned)__popcll(__ballot(ended && nan));
+                            if (ended) {
+                                // the sum over samples starts from zero and drops NaN samples
+                                const f3 sum = nan ? mk3(0.0f, 0.0f, 0.0f) : mk3(0.0f, 0.0f, 0.0f) + acc;
+                                texels[p0 + p] = finish_texel(Fin, sum, texels[p0 + p], wgt);
+                            }
+                        } else if (ended) {
+                            Wv.acc[base + p] = make_float4(acc.x, acc.y, acc.z, 0.0f);
+                        }
+                        if (ended) st = LS_IDLE;
+                        if (!chunk.drained()) {
+                            const int e = wave_refill(idle, chunk);
+                            const int b = e >> 6;
+                            const int path = ((b % seg_blocks) * nsegm + b / seg_blocks) * 64 + (e & 63);
+                            if (e >= 0 && path < n) {
+                                p = path;
+                                camera_ray(S, F, p0 + p % pc, k0 + p / pc, v.o, v.d, v.l0, v.key);
+                                v.T = mk4(1.0f);
+                                v.flags = 2u;  // the camera ray counts as specular for emitter MIS
+                                v.pdf = 0.0f;
+                                acc = mk3(0.0f, 0.0f, 0.0f);
+                                bounce = 0;
+                                st = LS_DONE;
+                                ext = F.maxDepth > 0;
+                            }
+                        }
+                        ended_all = chunk.drained() && __ballot(st != LS_IDLE) == 0ull;
+                    }
+                    nseg += (unsigned)__popcll(__ballot(ext));
+                    // the new rays: the parallelograms, then the BVH
+                    if (ext || shadow) {
+                        const f3 ro = shadow ? sh.o : v.o, rd = shadow ? sh.d : v.d;
+                        t = shadow ? sh.tmax : 1e30f;
+                        ref = kMiss;
+                        best = -1;
+                        blocked = false;
+                        any = shadow;
+                        for (int i = 0; i < nq; ++i) {
+                            float tq;
+                            if (!blocked && isect_quad(s_quad + 4 * i, ro, rd, t, tq)) {
+                                t = shadow ? t : tq;
+                                blocked = shadow;
+                                ref = (REF_QUAD << kRefShift) | (uint32_t)i;
+                            }
+                        }
+                        ray_inv(ro, rd, inv, oi);
+                        sp = 0;
+                        const bool skip = blocked || S.nsph == 0;
+                        node = skip ? -1 : 0;
+                        st = skip ? LS_SEEK : LS_BVH;
                     }
                 }
-                if (chunk.drained() && __ballot(st != LS_IDLE) == 0ull) break;
+                if (ended_all) break;
             }
-            nseg += (unsigned)__popcll(__ballot(ext));
-            // the new rays: the parallelograms, then the BVH
-            if (ext || shadow) {
-                const f3 ro = shadow ? sh.o : v.o, rd = shadow ? sh.d : v.d;
-                t = shadow ? sh.tmax : 1e30f;
-                ref = kMiss;
-                best = -1;
-                blocked = false;
-                for (int i = 0; i < nq; ++i) {
-                    float tq;
-                    if (!blocked && isect_quad(s_quad + 4 * i, ro, rd, t, tq)) {
-                        t = shadow ? t : tq;
-                        blocked = shadow;
-                        ref = (REF_QUAD << kRefShift) | (uint32_t)i;
+#pragma unroll
+            for (int u = 0; u < kPathVisits; ++u) {
+                nvis += (unsigned)__popcll(__ballot(st == LS_BVH && !any));
+                nsvis += (unsigned)__popcll(__ballot(st == LS_BVH && any));
+                if (st == LS_BVH) {
+                    const f3 ro = any ? sh.o : v.o, rd = any ? sh.d : v.d;
+                    if (bvh_step2<kPathLanes>(S.sbvh, ro, rd, inv, oi, t, best, node, sp, stack, any)) {
+                        blocked = true;
+                        node = -1;
+                    }
+                    if (node < 0) st = LS_SEEK;
+                }
+            }
+            for (int u = 0; u < (SDF ? kPathSteps : 0); ++u) {
+                const bool march = st == LS_MARCH;
+                const bool step = march && sp < S.sdf_steps_max;
+                nsteps += (unsigned)__popcll(__ballot(step));
+                nexhausted += (unsigned)__popcll(__ballot(march && !step));
+                if (march && !step) st = LS_SEEK;  // a miss
+                if (step) {
+                    const float dist = ext_de_at(best & 15, inv, best >> 4, oi.z,
+                                                 ray_at(any ? sh.o : v.o, any ? sh.d : v.d, oi.x), it);
+                    ++sp;
+                    if (dist < 1e-4f) {
+                        blocked = any;
+                        if (!any && oi.x < t) {
+                            t = oi.x;
+                            ref = (REF_SDF << kRefShift) | (uint32_t)node;
+                        }
+                        st = LS_SEEK;
+                    } else {
+                        oi.x += dist;
+                        if (oi.x > oi.y) st = LS_SEEK;
                     }
                 }
-                ray_inv(ro, rd, inv, oi);
-                sp = 0;
-                node = 0;
-                st = shadow ? LS_ANY : LS_EXT;
-                if (blocked || S.nsph == 0) st = shadow ? LS_SHADOW : LS_HIT;
             }
-        }
-        const bool any = st == LS_ANY;
-        nvis += (unsigned)__popcll(__ballot(st == LS_EXT));
-        nsvis += (unsigned)__popcll(__ballot(any));
-        if (st >= LS_EXT) {
-            const f3 ro = any ? sh.o : v.o, rd = any ? sh.d : v.d;
-            if (bvh_step2<kPathLanes>(S.sbvh, ro, rd, inv, oi, t, best, node, sp, stack, any)) {
-                blocked = true;
-                node = -1;
-            }
-            if (node < 0) st = any ? LS_SHADOW : LS_HIT;
         }
     }
     if (threadIdx.x == 0) {
@@ -2566,17 +2686,24 @@ __global__ void __launch_bounds__(kPathLanes, 4) k_ext_path(ExtSceneDev S, ExtFr
         add(11, nvis);
         add(12, nsvis);
         add(4, nnan);
+        add(2, nsteps);
+        add(13, nexhausted);
         add(kStatBadRefs, nbad);
     }
+    if (SDF)
+        for (int i = 0; i < 5; ++i)
+            wave_add_u64(stat_slot(Wv.stats, i < 4 ? kStatMarchFlops + i : kStatShadowMarchFlops), s_flops[i][threadIdx.x]);
     // the last wave to end clears the cursors and the count for the next launch:
     // every other wave has taken its entries before it counted itself
+    const int ncur = MULTI ? kMaxBatch * kSeg : kSeg;
     int last = 0;
     if (threadIdx.x == 0) {
         __threadfence();
-        last = atomicAdd(cursor + kSeg * kCntStride, 1) == (int)gridDim.x - 1;
+        last = atomicAdd(cursor + ncur * kCntStride, 1) == (int)gridDim.x - 1;
     }
     if (__builtin_amdgcn_readfirstlane(last)) {
-        for (int j = (int)threadIdx.x; j < kPathCursors; j += kPathLanes) cursor[j * kCntStride] = 0;
+        for (int j = (int)threadIdx.x; j < nreq * kSeg; j += kPathLanes) cursor[j * kCntStride] = 0;
+        if (threadIdx.x == 0) cursor[ncur * kCntStride] = 0;
     }
 }
 
@@ -2594,7 +2721,7 @@ __global__ void __launch_bounds__(kBlk) k_ext_fold(ExtFrame F, ExtWave Wv, ExtFi
             ax += a.x; ay += a.y; az += a.z;
         }
         if (last) {
-            texels[F.p0 + j] = finish_texel(Fin, mk3(ax, ay, az), texels[F.p0 + j]);
+            texels[F.p0 + j] = finish_texel(Fin, mk3(ax, ay, az), texels[F.p0 + j], blend_weight(Fin));
         } else {
             Wv.sum[j] = ax; Wv.sum[F.pc + j] = ay; Wv.sum[2 * F.pc + j] = az;
         }
@@ -2722,10 +2849,12 @@ __global__ void __launch_bounds__(kBlk) k_ext_rel_error(int P, const float* sum,
 struct ExtSceneHost {
     DevAlloc mem;
     ExtSceneDev dev{};
+    const ExtSceneDev* on_device = nullptr;  // a copy of dev
     int stack_need = 0;
     int width = 4;
     bool small_nodes = true;  // every BVH has < 65536 nodes: 16-bit stack entries
     std::vector<int> sdf_kinds;  // kinds present, one march launch per kind
+    int64_t sdf_iters = 0;       // most iterations of an SDF
 };
 
 struct ExtCtxState {
@@ -2737,6 +2866,7 @@ struct ExtCtxState {
     ExtWave lean{};
     int cu = 0;  // compute units of the context's device (grid sizing)
     DevAlloc batch_mem;  // batched waves: header + scene, frame, segment and sink tables of up to kMaxBatch requests
+    DevAlloc path_mem;   // batched waves: the whole-path kernel's cursors
     // pinned host copy of those tables: one asynchronous upload per wave, and
     // an event marking when the staging copy may be rewritten
     void* batch_host = nullptr;
@@ -2993,6 +3123,16 @@ static int upload_ext(pt_ctx* ctx, pt_scene* s, ExtSceneHost* h) {
     h->width = width;
     h->small_nodes = sb.n_nodes < 65536 && (!quad_bvh || qb.n_nodes < 65536);
     h->sdf_kinds = kinds;
+    // the order of the march kernels for the whole-path kernel's extension rays
+    int* link = &h->dev.sdf_first;
+    for (int k : kinds)
+        for (size_t i = 0; i < sdfs.size(); ++i)
+            if (sdfs[i].kind == k) {
+                *link = (int)i;
+                link = &sdfs[i].next;
+                h->sdf_iters = std::max(h->sdf_iters, std::abs((int64_t)sdfs[i].iters));
+            }
+    *link = -1;
 
     size_t bytes = 0;
     auto sz = [&](size_t b) { bytes += ((b + 255) / 256) * 256; };
@@ -3001,6 +3141,7 @@ static int upload_ext(pt_ctx* ctx, pt_scene* s, ExtSceneHost* h) {
     sz(lights.size() * sizeof(ExtLight)); sz(lenses.size() * sizeof(ExtLens)); sz(cycs.size() * sizeof(ExtCyc));
     sz(sb.words.size() * 4); sz(sleaf.size() * 16); sz(sids.size() * 4);
     sz(qb.words.size() * 4); sz(qleaf.size() * 16); sz(qids.size() * 4);
+    sz(sizeof(ExtSceneDev));
     int st = dev_alloc(ctx, h->mem, bytes);
     if (st != PT_OK) return st;
     char* p = static_cast<char*>(h->mem.p);
@@ -3031,7 +3172,6 @@ static int upload_ext(pt_ctx* ctx, pt_scene* s, ExtSceneHost* h) {
     D.qbvh.prims = (const float4*)put(qleaf.data(), qleaf.size() * 16);
     D.qbvh.ids = (const int*)put(qids.data(), qids.size() * 4);
     D.qbvh.count = (int)qids.size();
-    if (fail) return hip_fail(ctx, hipGetLastError(), "extended scene upload");
     D.nsph = (int)sph.size();
     D.nquad = (int)quad_ml.size();
     D.quad_bvh = quad_bvh ? 1 : 0;
@@ -3051,6 +3191,8 @@ static int upload_ext(pt_ctx* ctx, pt_scene* s, ExtSceneHost* h) {
     D.seed = m.render.seed;
     D.camera = m.render.camera;
     D.sdf_steps_max = ctx->cfg.sdf_max_steps > 0 ? ctx->cfg.sdf_max_steps : 256;
+    h->on_device = (const ExtSceneDev*)put(&D, sizeof D);
+    if (fail) return hip_fail(ctx, hipGetLastError(), "extended scene upload");
     s->device_bytes += (int64_t)bytes;
     return PT_OK;
 }
@@ -3090,8 +3232,8 @@ static ExtCtxState* ext_state(pt_ctx* ctx) {
 
 constexpr size_t kCursorBytes = (size_t)(N_CUR * kSeg + kPathCursors) * kCntStride * 4;
 
-static int clear_path_cursors(pt_ctx* ctx, const ExtWave& W) {
-    launch(ctx, "k_ext_clear", k_ext_clear, dim3(1), dim3(64), W.cursor);
+static int clear_path_cursors(pt_ctx* ctx, int* cursor, int n) {
+    launch(ctx, "k_ext_clear", k_ext_clear, dim3(1), dim3(64), cursor, n);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? PT_OK : hip_fail(ctx, e, "extended wave");
 }
@@ -3106,6 +3248,7 @@ static int ensure_lean_wave(pt_ctx* ctx, int cap, ExtWave** W) {
     }
     *W = &st->lean;
     if (st->lean.cap >= cap) return PT_OK;
+    drop_graphs(st);  // they may hold the old wave's addresses
     st->lean = ExtWave{};
     dev_free(ctx, st->lean_mem);
     const size_t n = (size_t)cap;
@@ -3119,7 +3262,7 @@ static int ensure_lean_wave(pt_ctx* ctx, int cap, ExtWave** W) {
     L.cursor = carve_e<int>(p, kCursorBytes / 4);
     L.stats = ctx->d_stats;
     L.cap = cap;
-    return clear_path_cursors(ctx, L);
+    return clear_path_cursors(ctx, L.cursor + CUR_PATH * kSeg * kCntStride, kPathCursors);
 }
 
 static int ensure_ext_wave(pt_ctx* ctx, int cap) {
@@ -3157,7 +3300,7 @@ static int ensure_ext_wave(pt_ctx* ctx, int cap) {
     W.cursor = carve_e<int>(p, kCursorBytes / 4);
     W.stats = ctx->d_stats;
     W.cap = cap;
-    return clear_path_cursors(ctx, W);
+    return clear_path_cursors(ctx, W.cursor + CUR_PATH * kSeg * kCntStride, kPathCursors);
 }
 
 void ext_wave_release(pt_ctx* ctx) {
@@ -3168,6 +3311,7 @@ void ext_wave_release(pt_ctx* ctx) {
     if (st->batch_done) (void)hipEventDestroy(st->batch_done);
     if (st->batch_host) (void)hipHostFree(st->batch_host);
     dev_free(ctx, st->batch_mem);
+    dev_free(ctx, st->path_mem);
     dev_free(ctx, st->lean_mem);
     dev_free(ctx, st->mem);
     delete st;
@@ -3377,6 +3521,23 @@ struct ExtSink {
 // 8.7 % (SDFs).
 constexpr int64_t kDispatchWave = (int64_t)1 << 27;
 
+// The whole-path kernel takes the scene, and no setting asks for the kernels per stage.
+static bool whole_takes(const pt_ctx* ctx, const ExtSceneHost& H) {
+    const bool march = ctx->cfg.march == 0 && ctx->cfg.march_blocks_per_cu == 0 && H.sdf_iters < 1 << 24;
+    return (H.dev.nsdf == 0 || march) && !H.dev.quad_bvh && H.dev.nlens + H.dev.ncyc == 0 && H.width == 2 &&
+           H.small_nodes && H.stack_need <= kPathStack && ctx->cfg.traversal == 0;
+}
+// Waves of the whole-path kernel that the device holds at once.
+static int path_grid(pt_ctx* ctx, bool sdf, bool multi) {
+    int& w = ctx->path_waves[(sdf ? 1 : 0) + (multi ? 2 : 0)];
+    if (w == 0) {
+        auto kernel = multi ? (sdf ? k_ext_path<true, true> : k_ext_path<true, false>)
+                            : (sdf ? k_ext_path<false, true> : k_ext_path<false, false>);
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&w, kernel, kPathLanes, 0) != hipSuccess || w < 1) w = 8;
+    }
+    return ctx->cus * w;
+}
+
 static int ext_run(pt_ctx* ctx, const pt_scene* s, const pt_push_constants* pc, const ExtSink& sink) {
     int st = ext_scene_build(ctx, const_cast<pt_scene*>(s));
     if (st != PT_OK) return st;
@@ -3387,9 +3548,7 @@ static int ext_run(pt_ctx* ctx, const pt_scene* s, const pt_push_constants* pc, 
     int64_t cap = ctx->cfg.wave_paths > 0 ? ctx->cfg.wave_paths : kDispatchWave;
     cap = std::max<int64_t>(1024, std::min<int64_t>(cap, (int64_t)P * std::max(1, pc->samplesPerFrame)));
     // whole paths in one kernel, or a kernel per stage and bounce (k_ext_path has the rule's reasons)
-    const bool whole = H.dev.nsdf == 0 && !H.dev.quad_bvh && H.dev.nlens + H.dev.ncyc == 0 && H.width == 2 &&
-                       H.small_nodes && H.stack_need <= kPathStack && ctx->cfg.traversal == 0 &&
-                       (cap <= kWholePaths || H.dev.nsph <= kWholeSpheres);
+    const bool whole = whole_takes(ctx, H) && (H.dev.nsdf == 0 || cap <= kWholeSdfPaths);
     ExtWave* wave = nullptr;
     if (whole) {
         st = ensure_lean_wave(ctx, (int)cap, &wave);
@@ -3399,11 +3558,6 @@ static int ext_run(pt_ctx* ctx, const pt_scene* s, const pt_push_constants* pc, 
     }
     if (st != PT_OK) return st;
     ExtWave& Wv = *wave;
-    if (whole && ctx->path_waves == 0 &&
-        (hipOccupancyMaxActiveBlocksPerMultiprocessor(&ctx->path_waves, k_ext_path, kPathLanes, 0) != hipSuccess ||
-         ctx->path_waves < 1))
-        ctx->path_waves = 8;
-
     ExtFrame F = frame_of(*pc);
     const int grid_cap = ctx_cus(ctx) * blocks_per_cu(ctx);
     ExtPlan plan;
@@ -3432,9 +3586,11 @@ static int ext_run(pt_ctx* ctx, const pt_scene* s, const pt_push_constants* pc, 
             const int grid = std::min((npaths + kBlk - 1) / kBlk, grid_cap);
             const int count = sink.count && p0 == 0 && k0 == 0;
             if (whole) {
-                const int waves = std::max(1, std::min((npaths + kPathLanes - 1) / kPathLanes, ctx->cus * ctx->path_waves));
-                launch(ctx, "k_ext_path", k_ext_path, dim3(waves), dim3(kPathLanes), H.dev, F, Wv, Fin,
-                       sink.acc ? reinterpret_cast<float4*>(sink.acc->d_texels) : nullptr, direct, (int)plan.aov, count);
+                const int waves = std::max(1, std::min((npaths + kPathLanes - 1) / kPathLanes, path_grid(ctx, H.dev.nsdf > 0, false)));
+                launch(ctx, "k_ext_path", H.dev.nsdf ? k_ext_path<false, true> : k_ext_path<false, false>, dim3(waves),
+                       dim3(kPathLanes), F, Wv, Fin,
+                       sink.acc ? reinterpret_cast<float4*>(sink.acc->d_texels) : nullptr, direct, (int)plan.aov, count,
+                       ExtPathBatch{(PT_RO ExtSceneDev*)H.on_device, nullptr, nullptr, nullptr, nullptr});
                 if (direct) continue;
             } else {
                 launch(ctx, "k_ext_counts", k_ext_counts, dim3(1), dim3(64), Wv.counts, npaths, Wv.stats, count);
@@ -3489,6 +3645,7 @@ int ext_dispatch_batch(pt_ctx* ctx, const ExtBatchItem* items, int n) {
     std::vector<ExtMomentSink> sinks((size_t)n);
     int64_t npaths = 0, npix = 0;
     int depth = 0;
+    bool whole = true;  // every scene is one the whole-path kernel takes
     for (int i = 0; i < n; ++i) {
         const ExtBatchItem& it = items[i];
         int st = ext_scene_build(ctx, const_cast<pt_scene*>(it.scene));
@@ -3500,6 +3657,7 @@ int ext_dispatch_batch(pt_ctx* ctx, const ExtBatchItem* items, int n) {
             ctx->err = "batched wave: scenes with different BVH widths";
             return PT_ERR_STATE;
         }
+        whole = whole && whole_takes(ctx, H);
         plan.stack_need = std::max(plan.stack_need, H.stack_need);
         plan.small_nodes = plan.small_nodes && H.small_nodes;
         plan.any_sdf = plan.any_sdf || H.dev.nsdf > 0;
@@ -3529,10 +3687,17 @@ int ext_dispatch_batch(pt_ctx* ctx, const ExtBatchItem* items, int n) {
         ctx->err = "batched wave: " + std::to_string(npaths) + " paths exceed the wave capacity " + std::to_string(cap);
         return PT_ERR_CAPACITY;
     }
-    int st = ensure_ext_wave(ctx, cap);
+    whole = whole && (!plan.any_sdf || cap <= kWholeSdfPaths);
+    ExtCtxState* cs = ext_state(ctx);
+    if (whole && !cs->path_mem.p) {
+        int st = dev_alloc(ctx, cs->path_mem, (size_t)kBatchCursors * kCntStride * 4);
+        if (st == PT_OK) st = clear_path_cursors(ctx, static_cast<int*>(cs->path_mem.p), kBatchCursors);
+        if (st != PT_OK) return st;
+    }
+    ExtWave* wave = &cs->wave;
+    int st = whole ? ensure_lean_wave(ctx, cap, &wave) : ensure_ext_wave(ctx, cap);
     if (st != PT_OK) return st;
-    ExtCtxState* cs = static_cast<ExtCtxState*>(ctx->ext_state);
-    ExtWave& Wv = cs->wave;
+    ExtWave& Wv = *wave;
     // tables at fixed addresses: header, scenes, frames, segments, sinks
     const size_t o_sc = 256, o_fr = o_sc + (sizeof(ExtSceneDev) * kMaxBatch + 255) / 256 * 256,
                  o_sg = o_fr + (sizeof(ExtFrame) * kMaxBatch + 255) / 256 * 256,
@@ -3583,7 +3748,16 @@ int ext_dispatch_batch(pt_ctx* ctx, const ExtBatchItem* items, int n) {
     const int grid = (int)std::min<int64_t>(((int64_t)cap + kBlk - 1) / kBlk,
                                             (int64_t)ctx_cus(ctx) * blocks_per_cu(ctx));
     plan.cus = ctx_cus(ctx);
+    const int pgrid = whole ? path_grid(ctx, plan.any_sdf, true) : 0;
     auto launch_wave = [&]() {
+        if (whole) {
+            const ExtPathBatch PB{(PT_RO ExtSceneDev*)d_scenes, (PT_RO ExtFrame*)d_frames, (PT_RO ExtSeg*)d_segs,
+                                  (PT_RO ExtBatchHdr*)d_hdr, static_cast<int*>(cs->path_mem.p)};
+            launch(ctx, "k_ext_path", plan.any_sdf ? k_ext_path<true, true> : k_ext_path<true, false>, dim3(pgrid),
+                   dim3(kPathLanes), ExtFrame{}, Wv, ExtFinish{}, static_cast<float4*>(nullptr), 0, 0, 0, PB);
+            launch(ctx, "k_ext_moments", k_ext_moments_batch, dim3(grid), dim3(kBlk), d_segs, d_sinks, d_hdr, Wv);
+            return;
+        }
         launch(ctx, "k_ext_counts", k_ext_counts_batch, dim3(1), dim3(64), Wv.counts, d_hdr);
         launch(ctx, "k_ext_raygen", k_ext_raygen_batch, dim3(grid), dim3(kBlk), plan.B, d_segs, d_hdr, Wv);
         launch_bounces(ctx, plan, Wv, depth, grid);
@@ -3595,7 +3769,7 @@ int ext_dispatch_batch(pt_ctx* ctx, const ExtBatchItem* items, int n) {
         uint32_t kinds = 0;
         for (int k : plan.sdf_kinds) kinds |= 1u << (k & 7);
         const uint64_t key = (uint64_t)plan.width | (uint64_t)(plan.stack_need <= 32) << 4 |
-                             (uint64_t)plan.small_nodes << 5 | (uint64_t)plan.any_sdf << 6 | (uint64_t)kinds << 8 |
+                             (uint64_t)plan.small_nodes << 5 | (uint64_t)plan.any_sdf << 6 | (uint64_t)whole << 7 | (uint64_t)kinds << 8 |
                              (uint64_t)depth << 16 | (uint64_t)grid << 32;
         auto it = cs->graphs.find(key);
         if (it == cs->graphs.end()) {

@@ -125,7 +125,7 @@ struct pt_ctx {
     DevAlloc ref_mem;
     ptk::RefWave ref_wave{};
     int ref_waves[6] = {};  // resident waves per compute unit of k_ref_path, by its KIND + 1
-    int path_waves = 0;  // resident waves per compute unit of k_ext_path (0: not asked yet)
+    int path_waves[4] = {};  // resident waves per compute unit of k_ext_path's forms (0: not asked yet)
     // extended-mode wave (owned by ext_tracer.hip)
     void* ext_state = nullptr;
 };

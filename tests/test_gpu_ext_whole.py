@@ -32,8 +32,10 @@ SCENES = {
     "plane_sky": plane_and_sky,
     "no_light": lambda: plane_and_sky(light=False),
     "quads_only": lambda: json.dumps(dict(scenes.cornell_dict(4, seed=7), sphere=[])),
+    "sdf": lambda: scenes.sdf_scene(seed=3),
+    "sdf_spheres": lambda: json.dumps(dict(json.loads(plane_and_sky()), sdf=json.loads(scenes.sdf_scene(seed=3))["sdf"])),
 }
-COUNTERS = ("segments", "shadow_segments", "paths", "nan_samples", "dispatches", "escaped", "emitter_hits", "lambert_hits",
+COUNTERS = ("sdf_steps", "sdf_exhausted", "segments", "shadow_segments", "paths", "nan_samples", "dispatches", "escaped", "emitter_hits", "lambert_hits",
             "dielectric_hits", "conductor_hits", "bvh_nodes", "shadow_bvh_nodes", "bad_refs")
 
 
@@ -101,3 +103,22 @@ def test_features_and_a_full_wave_in_between():
                 np.testing.assert_array_equal(ctx.features(sc, pc).view(np.uint32), first.view(np.uint32))
             out.append(first)
     np.testing.assert_array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
+
+
+def serve(traversal, names):
+    with pt.Context(0, traversal=traversal) as ctx, pt.Server(ctx) as server:
+        ids = [server.submit(SCENES[n](), 37 + 8 * k, 29, 6, 4 + k, target=1e-6) for k, n in enumerate(names)]
+        while server.step() is not None:
+            pass
+        return [server.read(i) for i in ids], ctx.counters()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("names", [["spheres", "plane_sky"], ["sdf", "spheres", "sdf_spheres", "quads_only", "sdf"]])
+def test_batched_waves(names):
+    """Requests of several scenes in one wave, with and without SDFs: the same images."""
+    a, ca = serve(0, names)
+    b, cb = serve(1, names)
+    for x, y in zip(a, b):
+        np.testing.assert_array_equal(np.asarray(x).view(np.uint32), np.asarray(y).view(np.uint32))
+    assert {c: ca[c] for c in COUNTERS} == {c: cb[c] for c in COUNTERS}
