@@ -3273,6 +3273,7 @@ static int ensure_ext_wave(pt_ctx* ctx, int cap) {
     dev_free(ctx, st->mem);
     st->lean = ExtWave{};  // a full wave serves the whole-path kernel too
     dev_free(ctx, st->lean_mem);
+    dev_free(ctx, st->path_mem);  // made again by a batched wave that has the room
     size_t n = (size_t)cap;
     // per path: record (org, dir, T, aux) 64, acc 16, hit 8, extension queues 4 * 2,
     // material-queue entries 16 * N_MATQ, shadow org/dir/xyz 48, first-hit
@@ -3689,24 +3690,32 @@ int ext_dispatch_batch(pt_ctx* ctx, const ExtBatchItem* items, int n) {
     }
     whole = whole && (!plan.any_sdf || cap <= kWholeSdfPaths);
     ExtCtxState* cs = ext_state(ctx);
-    if (whole && !cs->path_mem.p) {
-        int st = dev_alloc(ctx, cs->path_mem, (size_t)kBatchCursors * kCntStride * 4);
-        if (st == PT_OK) st = clear_path_cursors(ctx, static_cast<int*>(cs->path_mem.p), kBatchCursors);
-        if (st != PT_OK) return st;
-    }
-    ExtWave* wave = &cs->wave;
-    int st = whole ? ensure_lean_wave(ctx, cap, &wave) : ensure_ext_wave(ctx, cap);
-    if (st != PT_OK) return st;
-    ExtWave& Wv = *wave;
     // tables at fixed addresses: header, scenes, frames, segments, sinks
     const size_t o_sc = 256, o_fr = o_sc + (sizeof(ExtSceneDev) * kMaxBatch + 255) / 256 * 256,
                  o_sg = o_fr + (sizeof(ExtFrame) * kMaxBatch + 255) / 256 * 256,
                  o_sk = o_sg + (sizeof(ExtSeg) * kMaxBatch + 255) / 256 * 256,
                  tb = o_sk + (sizeof(ExtMomentSink) * kMaxBatch + 255) / 256 * 256;
+    int st = PT_OK;
     if (!cs->batch_mem.p) {
         st = dev_alloc(ctx, cs->batch_mem, tb);
         if (st != PT_OK) return st;
     }
+    // no room for the cursors (a budget): the kernels per stage, as they need none
+    if (whole && !cs->path_mem.p) {
+        const std::string err = ctx->err;
+        if (dev_alloc(ctx, cs->path_mem, (size_t)kBatchCursors * kCntStride * 4) != PT_OK) {
+            (void)hipGetLastError();
+            ctx->err = err;
+            whole = false;
+        } else {
+            st = clear_path_cursors(ctx, static_cast<int*>(cs->path_mem.p), kBatchCursors);
+            if (st != PT_OK) return st;
+        }
+    }
+    ExtWave* wave = &cs->wave;
+    st = whole ? ensure_lean_wave(ctx, cap, &wave) : ensure_ext_wave(ctx, cap);
+    if (st != PT_OK) return st;
+    ExtWave& Wv = *wave;
     hipError_t e = hipSuccess;
     if (!cs->batch_host) {
         e = hipHostMalloc(&cs->batch_host, tb, hipHostMallocDefault);

@@ -516,7 +516,7 @@ pt_status pt_server_read(pt_server* s, int32_t id, float* host_rgba, size_t n_fl
     if (e == hipSuccess) e = hipMemcpyAsync(n.data(), r.nsamp, P * 4, hipMemcpyDeviceToHost, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) return fail(s, ptk::hip_fail(ctx, e, "pt_server_read"), ctx->err);
-    // the texel units of k_ext_finish: mean per-sample XYZ x apertureSize^2 x ISO
+    // the texel units of k_ext_fold: mean per-sample XYZ x apertureSize^2 x ISO
     const float ex = r.pc.apertureSize * r.pc.apertureSize * (float)r.pc.ISO;
     for (size_t i = 0; i < P; ++i) {
         const float inv = n[i] > 0 ? ex / (float)n[i] : 0.0f;
