@@ -264,7 +264,8 @@ pt_status pt_sync(pt_ctx* ctx);
  * device the library runs on until the process ends; a dispatch of more paths
  * runs as several waves through it, so it has no size limit beyond
  * pt_dispatch's. Texels equal pt_dispatch's bit for bit. All contexts on one
- * device share that array: calls that overlap on one device race. Returns
+ * device share that array: calls that overlap on one device race, which spoils
+ * their own texels and counters and nothing of later calls. Returns
  * PT_ERR_STATE while kernel profiling is enabled (it records events). */
 pt_status pt_dispatch_noalloc(pt_ctx* ctx, const pt_scene* scene, pt_accum* acc, const pt_push_constants* pc);
 

@@ -1095,7 +1095,7 @@ __global__ void __launch_bounds__(kBlock) k_ref_fold(RefFrame F, RefWave Wv, Ref
         Wv.sum[2 * F.pc + j] = acc.z;
     }
 }
-// Zeroes the cursors of new wave memory (a kernel, not a memset).
+// Zeroes the cursors of a wave (a kernel, not a memset).
 __global__ void k_ref_clear(int* cursor) {
     for (int j = (int)threadIdx.x; j <= kSeg; j += blockDim.x) cursor[j * kCntStride] = 0;
 }
@@ -1142,9 +1142,10 @@ static int ensure_ref_wave(pt_ctx* ctx, int cap) {
 // ---- the allocation-free dispatch's wave --------------------------------------------
 // A wave of kStaticWavePaths paths in a static device array: pt_dispatch_noalloc
 // traces through it instead of allocating. Each device holds its own copy for
-// the life of the process. Every launch writes the records it reads (its cursors
-// start at zero, as a static array does, and every launch leaves them so), so
-// nothing needs clearing between calls; calls that overlap on one device race on it.
+// the life of the process. Every launch writes the records it reads, but for its
+// cursors, which it expects and leaves at zero: a call clears them first. Calls that
+// overlap on one device race on the wave, and what they leave in the cursors and the
+// count of ended waves would otherwise stay there and drop paths of every later call.
 constexpr int kStaticWavePaths = 1 << 16;
 constexpr size_t kStaticWaveBytes = ref_wave_bytes(kStaticWavePaths);  // 1,843,456 B
 static __device__ __align__(256) char scratch[kStaticWaveBytes];
@@ -1399,6 +1400,7 @@ int ref_dispatch_static(pt_ctx* ctx, const pt_scene* s, pt_accum* acc, const pt_
     }
     RefWave Wv{};
     carve_ref_wave(base, kStaticWavePaths, ctx->d_stats, Wv);
+    launch(ctx, "k_ref_clear", k_ref_clear, dim3(1), dim3(64), Wv.cursor);
     return ref_dispatch_wave(ctx, s, acc, pc, Wv);
 }
 

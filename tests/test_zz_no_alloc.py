@@ -55,3 +55,23 @@ def test_noalloc_dispatch_rejects_bad_arguments(gpu_ctx):
     pc.frame = pc.currentSamples = 1
     assert pt.lib.pt_dispatch_noalloc(gpu_ctx.h, scene.h, acc.h, C.byref(pc)) == pt.PT_ERR_INVALID_ARG
     assert pt.lib.pt_dispatch_noalloc(None, None, None, None) == pt.PT_ERR_INVALID_ARG
+
+
+@pytest.mark.parametrize("spf", [1, 2])
+def test_overlapping_calls_spoil_no_later_call(spf):
+    """Two contexts' calls in flight at once, which race on the shared wave: their own
+    texels are anyone's guess, but a later call alone gives pt_dispatch's again."""
+    text = SCENES[4].read_text()
+    with pt.Context(0) as a, pt.Context(0) as b:
+        sa, sb = a.scene_from_json(text), b.scene_from_json(text)
+        ra = pt.Renderer(a, sa, 320, 200, spf=1, path_length=6, mode=pt.MODE_REF)
+        rb = pt.Renderer(b, sb, 96, 64, spf=1, path_length=6, mode=pt.MODE_REF)
+        for f in range(1, 4):
+            for ctx, sc, r in ((a, sa, ra), (b, sb, rb), (b, sb, rb)):
+                r.pc.frame = r.pc.currentSamples = f
+                assert pt.lib.pt_dispatch_noalloc(ctx.h, sc.h, r.acc.h, C.byref(r.pc)) == pt.PT_OK
+        a.sync()
+        b.sync()
+        want = run(a, sa, 150, 101, spf, 2, noalloc=False)
+        for ctx, sc in ((a, sa), (b, sb)):
+            assert np.array_equal(run(ctx, sc, 150, 101, spf, 2, noalloc=True), want)
