@@ -1796,7 +1796,8 @@ __global__ void __launch_bounds__(kBlk) k_ext_features(ExtFrame F, ExtWave Wv, f
             const int p = k * F.pc + j;
             float4 a = Wv.acc[p];
             if (a.x != a.x || a.y != a.y || a.z != a.z) { ++nans; continue; }
-            float4 b0 = Wv.aov0[p], b1 = Wv.aov1[p];
+            float4 b0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), b1 = b0;
+            if (F.maxDepth > 0) { b0 = Wv.aov0[p]; b1 = Wv.aov1[p]; }  // else nothing has written them
             s[0] += a.x; s[1] += a.y; s[2] += a.z;
             s[3] += b0.x; s[4] += b0.y; s[5] += b0.z;
             s[6] += b1.x; s[7] += b1.y; s[8] += b1.z;

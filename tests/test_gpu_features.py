@@ -129,3 +129,18 @@ def test_bad_arguments_are_rejected(gpu_ctx):
     pc = pt.push_constants(16, 16, 0, 4)
     with pytest.raises(pt.PTError):
         gpu_ctx.features(sc, pc)
+
+
+@pytest.mark.parametrize("traversal", [0, 1])
+@pytest.mark.parametrize("wave_paths", [0, 1024])
+def test_no_segments_no_features(traversal, wave_paths):
+    """Path length 0: no ray, so no radiance and no first hit, whatever the dispatch before left."""
+    with pt.Context(0, traversal=traversal, wave_paths=wave_paths) as ctx:
+        sc = ctx.scene_from_json(scenes.random_spheres(n=40, scene_seed=3, wavelengths=4, seed=3))
+        pc = pt.push_constants(64, 48, 3, 4)
+        sc.camera(1, pc)
+        pc.frame = pc.currentSamples = 3
+        assert ctx.features(sc, pc)[..., 3:10].any()
+        pc.pathLength = 0
+        got = ctx.features(sc, pc)
+        assert np.all(got[..., :11] == 0) and np.all(got[..., 11] == 3)
