@@ -3239,21 +3239,42 @@ static int clear_path_cursors(pt_ctx* ctx, int* cursor, int n) {
     return e == hipSuccess ? PT_OK : hip_fail(ctx, e, "extended wave");
 }
 
+// Bytes of a wave's arrays per path. Lean: XYZ 16, first-hit features 32, sums 12. Full:
+// record (org, dir, T, aux) 64, hit 8, extension queues 4 * 2, material-queue entries
+// 16 * N_MATQ, shadow org/dir/xyz 48, SDF mask 4, queue-ordered rays 64 on top.
+constexpr size_t kLeanPath = 16 + 32 + 12, kFullPath = kLeanPath + 64 + 8 + 4 * 2 + 16 * N_MATQ + 48 + 4 + 64;
+
+static int ensure_ext_wave(pt_ctx* ctx, int cap);
+
 // A wave for the whole-path kernel (*W): the full one when it is large enough, else the
-// lean one, made for `cap` paths.
+// lean one, made for `cap` paths. A context never holds more than one full wave of its
+// largest dispatch would take: beside a full wave that is nearly large enough none is
+// made, but that one grows, and one that leaves no room for the lean wave is given back.
 static int ensure_lean_wave(pt_ctx* ctx, int cap, ExtWave** W) {
     ExtCtxState* st = ext_state(ctx);
-    if (st->wave.cap >= cap) {
-        *W = &st->wave;
-        return PT_OK;
+    const size_t n = (size_t)cap;
+    const std::string err = ctx->err;
+    *W = &st->wave;
+    if (st->wave.cap >= cap) return PT_OK;
+    if (st->lean.cap < cap && (size_t)st->wave.cap * kFullPath + n * kLeanPath > n * kFullPath) {
+        if (ensure_ext_wave(ctx, cap) == PT_OK) return PT_OK;
+        (void)hipGetLastError();  // no room; the smaller one is gone with the try
+        ctx->err = err;
     }
     *W = &st->lean;
     if (st->lean.cap >= cap) return PT_OK;
     drop_graphs(st);  // they may hold the old wave's addresses
     st->lean = ExtWave{};
     dev_free(ctx, st->lean_mem);
-    const size_t n = (size_t)cap;
-    int rc = dev_alloc(ctx, st->lean_mem, n * (16 + 32 + 12) + 5 * 256 + kCursorBytes);
+    const size_t bytes = n * kLeanPath + 5 * 256 + kCursorBytes;
+    int rc = dev_alloc(ctx, st->lean_mem, bytes);
+    if (rc != PT_OK && st->mem.p) {
+        (void)hipGetLastError();
+        st->wave = ExtWave{};
+        dev_free(ctx, st->mem);
+        rc = dev_alloc(ctx, st->lean_mem, bytes);
+        if (rc == PT_OK) ctx->err = err;
+    }
     if (rc != PT_OK) return rc;
     char* p = static_cast<char*>(st->lean_mem.p);
     ExtWave& L = st->lean;
@@ -3276,12 +3297,8 @@ static int ensure_ext_wave(pt_ctx* ctx, int cap) {
     dev_free(ctx, st->lean_mem);
     dev_free(ctx, st->path_mem);  // made again by a batched wave that has the room
     size_t n = (size_t)cap;
-    // per path: record (org, dir, T, aux) 64, acc 16, hit 8, extension queues 4 * 2,
-    // material-queue entries 16 * N_MATQ, shadow org/dir/xyz 48, first-hit
-    // features 32, SDF mask 4, sums 12, queue-ordered rays 64
-    size_t per_path = 64 + 16 + 8 + 4 * 2 + 16 * N_MATQ + 48 + 32 + 4 + 12 + 64;
     // + 256-byte rounding of 26 arrays + the counters and cursors, one line each
-    int rc = dev_alloc(ctx, st->mem, n * per_path + 28 * 256 + (size_t)N_CNT * kCntStride * 4 + kCursorBytes);
+    int rc = dev_alloc(ctx, st->mem, n * kFullPath + 28 * 256 + (size_t)N_CNT * kCntStride * 4 + kCursorBytes);
     if (rc != PT_OK) return rc;
     char* p = static_cast<char*>(st->mem.p);
     ExtWave& W = st->wave;

@@ -122,3 +122,46 @@ def test_batched_waves(names):
     for x, y in zip(a, b):
         np.testing.assert_array_equal(np.asarray(x).view(np.uint32), np.asarray(y).view(np.uint32))
     assert {c: ca[c] for c in COUNTERS} == {c: cb[c] for c in COUNTERS}
+
+
+def lens_scene():
+    """The spheres' box with a lens in it, which the whole-path kernel does not take."""
+    s = scenes.cornell_dict(4, seed=7)
+    s["lens"] = [{"position": [0.5, 0.5, 0.4], "rotation": [0.0, 0.0, 0.0], "radius": 0.2, "focalLength": 0.3,
+                  "thickness": 0.0, "isConverging": True, "materialID": 1, "lightID": 0}]
+    return json.dumps(s)
+
+
+FULL_PATH, LEAN_PATH = 336, 60  # bytes a path of the two waves
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ratio", [1.1, 4.0])
+def test_budget_of_one_wave_serves_both_kinds_in_turn(ratio):
+    """A dispatch of kernels per stage leaves its wave; a larger whole-path dispatch runs under a
+    budget that holds the wave it would take alone (the full one, or the lean one) but not both."""
+    w, h, spp = 512, 256, 4
+    h2 = int(h * ratio)
+    text = SCENES["spheres"]()
+    want = render(0, text, w, h2, spp, 4, frames=0)[0]
+    full, lean = FULL_PATH * w * h * spp, LEAN_PATH * w * h2 * spp
+    one = FULL_PATH * w * h2 * spp if ratio < 2 else max(full, lean)
+    rest = (w * h + w * h2) * 16 + (4 << 20)  # accumulators; scenes, cursors and counters
+    assert one + (4 << 20) < full + lean
+    with pt.Context(0, hbm_budget=one + rest) as ctx:
+        lens = pt.Renderer(ctx, ctx.scene_from_json(lens_scene()), w, h, spf=spp, path_length=4, mode=pt.MODE_EXT)
+        whole = pt.Renderer(ctx, ctx.scene_from_json(text), w, h2, spf=spp, path_length=4, mode=pt.MODE_EXT)
+        ctx.profile(True)
+        lens.render_frame()
+        assert "k_ext_path" not in ctx.profile_read(True)
+        first = lens.acc.read()
+        for _ in range(2):
+            whole.acc.reset()
+            whole.frame = whole.current = 0
+            whole.render_frame()
+            assert "k_ext_path" in ctx.profile_read(True)
+            np.testing.assert_array_equal(whole.acc.read().view(np.uint32), want.view(np.uint32))
+            lens.acc.reset()
+            lens.frame = lens.current = 0
+            lens.render_frame()
+            np.testing.assert_array_equal(lens.acc.read().view(np.uint32), first.view(np.uint32))
