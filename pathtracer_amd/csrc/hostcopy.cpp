@@ -105,6 +105,18 @@ hipError_t HostCopy::wait(Slot& s) {
     return hipEventSynchronize(s.done);
 }
 
+// Whether p is the caller's pageable memory. What the runtime knows (page-locked memory
+// moves at PCIe speed by itself; managed and device memory is not for the copying threads)
+// is its own to copy: 33 MB back into page-locked memory take 0.59 ms, through the ring 0.75.
+static bool pageable(const void* p) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();  // not an address of the runtime's
+        return true;
+    }
+    return a.type == hipMemoryTypeUnregistered;
+}
+
 // Bytes per chunk of a copy of n. A chunk costs about 20 us of calls and waits, so up
 // to 2 MB go in one and up to 8 MB in two (1 / 2 / 4 / 8 chunks at least: 1.9 MB back
 // in 66 / 79 / 123 / 176 us, 4.2 MB in 149 / 127 / 176 / 222 us; from 15 MB on, where
@@ -118,7 +130,7 @@ hipError_t HostCopy::to_host(void* dst, const void* src, size_t n, hipStream_t s
     const size_t chunk = chunk_of(n, kChunk);
     const size_t chunks = (n + chunk - 1) / chunk;
     const int slots = (int)std::min<size_t>(kRing, chunks);
-    if (n < kLeast || !ready(slots)) {
+    if (n < kLeast || !pageable(dst) || !ready(slots)) {
         hipError_t e = hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, st);
         const hipError_t es = hipStreamSynchronize(st);
         return e != hipSuccess ? e : es;
@@ -150,7 +162,7 @@ hipError_t HostCopy::to_device(void* dst, const void* src, size_t n, hipStream_t
     const size_t chunk = chunk_of(n, kChunk);
     const size_t chunks = (n + chunk - 1) / chunk;
     const int slots = (int)std::min<size_t>(kRing, chunks);
-    if (n < kLeast || !ready(slots)) return hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, st);
+    if (n < kLeast || !pageable(src) || !ready(slots)) return hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, st);
     for (size_t c = 0; c < chunks; ++c) {
         Slot& s = ring_[c % slots];
         const size_t len = std::min(chunk, n - c * chunk);

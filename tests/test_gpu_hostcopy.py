@@ -49,3 +49,25 @@ def test_two_contexts_in_two_threads():
     [x.start() for x in t]
     [x.join() for x in t]
     assert not errors, errors
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("w,h", [(64, 128), (1237, 1531)])
+def test_page_locked_memory(gpu_ctx, w, h):
+    """The same bytes into and out of page-locked memory, which the runtime copies itself."""
+    n = w * h * 4
+    p = pt.C.c_void_p()
+    assert pt.lib.hipHostMalloc(pt.C.byref(p), pt.C.c_size_t(n * 4), 0) == 0  # of the runtime the library uses
+    try:
+        bits = np.random.default_rng(3).integers(0, 2 ** 32, n, dtype=np.uint64).astype(np.uint32)
+        host = np.ctypeslib.as_array(pt.C.cast(p, pt.C.POINTER(pt.C.c_uint32)), (n,))
+        host[:] = bits
+        acc = gpu_ctx.accum(w, h)
+        gpu_ctx.check(pt.lib.pt_accum_write_xyz(acc.h, pt.C.cast(p, pt.C.POINTER(pt.C.c_float)), n))
+        host[:] = 0
+        assert np.array_equal(acc.read().view(np.uint32).reshape(-1), bits)
+        gpu_ctx.check(pt.lib.pt_accum_read_xyz(acc.h, pt.C.cast(p, pt.C.POINTER(pt.C.c_float)), n))
+        assert np.array_equal(host, bits)
+        acc.release()
+    finally:
+        pt.lib.hipHostFree(p)
