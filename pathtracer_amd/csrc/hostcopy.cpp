@@ -79,24 +79,32 @@ HostCopy::~HostCopy() {
     }
 }
 
-// Whether the first `slots` ring buffers are there.
-bool HostCopy::ready(int slots) {
-    for (int i = 0; i < slots; ++i) {
+// Whether the first `slots` ring buffers are there. Their events are made on the device of
+// the stream they will be recorded on, which need not be the caller's current one.
+bool HostCopy::ready(int slots, hipStream_t st) {
+    if (ring_[slots - 1].p) return true;  // they are made in order
+    int current = 0;
+    hipDevice_t device = 0;
+    if (hipGetDevice(&current) != hipSuccess || hipStreamGetDevice(st, &device) != hipSuccess ||
+        (device != current && hipSetDevice(device) != hipSuccess)) {
+        (void)hipGetLastError();
+        return false;
+    }
+    bool ok = true;
+    for (int i = 0; i < slots && ok; ++i) {
         Slot& s = ring_[i];
         if (s.p) continue;
         if (!s.done && hipEventCreateWithFlags(&s.done, hipEventDisableTiming) != hipSuccess) {
             s.done = nullptr;
-            (void)hipGetLastError();
-            return false;
+            ok = false;
         }
         void* p = nullptr;
-        if (hipHostMalloc(&p, kChunk, hipHostMallocDefault) != hipSuccess) {
-            (void)hipGetLastError();
-            return false;
-        }
-        s.p = static_cast<char*>(p);
+        if (ok && hipHostMalloc(&p, kChunk, hipHostMallocDefault) != hipSuccess) ok = false;
+        if (ok) s.p = static_cast<char*>(p);
     }
-    return true;
+    if (!ok) (void)hipGetLastError();
+    if (device != current) (void)hipSetDevice(current);
+    return ok;
 }
 
 hipError_t HostCopy::wait(Slot& s) {
@@ -130,7 +138,7 @@ hipError_t HostCopy::to_host(void* dst, const void* src, size_t n, hipStream_t s
     const size_t chunk = chunk_of(n, kChunk);
     const size_t chunks = (n + chunk - 1) / chunk;
     const int slots = (int)std::min<size_t>(kRing, chunks);
-    if (n < kLeast || !pageable(dst) || !ready(slots)) {
+    if (n < kLeast || !pageable(dst) || !ready(slots, st)) {
         hipError_t e = hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, st);
         const hipError_t es = hipStreamSynchronize(st);
         return e != hipSuccess ? e : es;
@@ -162,7 +170,7 @@ hipError_t HostCopy::to_device(void* dst, const void* src, size_t n, hipStream_t
     const size_t chunk = chunk_of(n, kChunk);
     const size_t chunks = (n + chunk - 1) / chunk;
     const int slots = (int)std::min<size_t>(kRing, chunks);
-    if (n < kLeast || !pageable(src) || !ready(slots)) return hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, st);
+    if (n < kLeast || !pageable(src) || !ready(slots, st)) return hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, st);
     for (size_t c = 0; c < chunks; ++c) {
         Slot& s = ring_[c % slots];
         const size_t len = std::min(chunk, n - c * chunk);

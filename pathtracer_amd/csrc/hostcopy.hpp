@@ -64,7 +64,7 @@ private:
         hipEvent_t done = nullptr;
         bool busy = false;  // `done` has been recorded and not waited for
     };
-    bool ready(int slots);
+    bool ready(int slots, hipStream_t st);
     hipError_t wait(Slot& s);
     Slot ring_[kRing];
     CopyTeam team_;

@@ -2,14 +2,15 @@
 // stand-ins for the HIP calls they make: "device" memory is host memory, copies happen
 // at once, and the stand-ins note which addresses the runtime was given.
 //
-// Usage: hostcopy_sim kind n    kind: pageable | pinned | device | managed
+// Usage: hostcopy_sim kind n [stream_device]    kind: pageable | pinned | device | managed
 // Checks the bytes both ways, and how they went: pageable memory through the ring (the
 // runtime never sees the caller's address), anything the runtime knows in one copy of
-// its own. Prints "ok" or the first violation, and exits 0 or 1.
+// its own. As in HIP, an event belongs to the device that was current when it was made and
+// can be recorded only on that device's streams; the stream here is one of stream_device,
+// the current device 0, which the copies must leave so. Prints "ok" or the first violation, and exits 0 or 1.
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <set>
 #include <string>
 #include <vector>
 
@@ -18,6 +19,7 @@
 static const char* g_known = nullptr;  // the caller's buffer, when the runtime knows it
 static size_t g_len = 0;
 static hipMemoryType g_type = hipMemoryTypeUnregistered;
+static int g_current = 0, g_stream_device = 0;
 static std::vector<std::pair<const void*, size_t>> g_host_side;  // host addresses given to the runtime
 
 extern "C" {
@@ -34,14 +36,28 @@ hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind ki
 }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
-    *e = reinterpret_cast<hipEvent_t>(new int(0));
+    *e = reinterpret_cast<hipEvent_t>(new int(g_current));
     return hipSuccess;
 }
 hipError_t hipEventDestroy(hipEvent_t e) {
     delete reinterpret_cast<int*>(e);
     return hipSuccess;
 }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
+    return *reinterpret_cast<int*>(e) == g_stream_device ? hipSuccess : hipErrorInvalidHandle;
+}
+hipError_t hipGetDevice(int* d) {
+    *d = g_current;
+    return hipSuccess;
+}
+hipError_t hipSetDevice(int d) {
+    g_current = d;
+    return hipSuccess;
+}
+hipError_t hipStreamGetDevice(hipStream_t, hipDevice_t* d) {
+    *d = g_stream_device;
+    return hipSuccess;
+}
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
     *p = std::malloc(n);
@@ -60,7 +76,8 @@ static int fail(const char* what) {
 }
 
 int main(int argc, char** argv) {
-    if (argc != 3) return 2;
+    if (argc != 3 && argc != 4) return 2;
+    if (argc == 4) g_stream_device = std::atoi(argv[3]);
     const std::string kind = argv[1];
     const size_t n = (size_t)std::atoll(argv[2]);
     std::vector<char> caller(n + 1), dev(n + 1);
@@ -90,6 +107,7 @@ int main(int argc, char** argv) {
         if (std::memcmp(caller.data(), want.data(), n)) return fail("to_host: bytes");
         if (ring ? sees_caller() : !direct_once()) return fail("to_host: wrong way");
     }
+    if (g_current != 0) return fail("the current device changed");
     std::printf("ok\n");
     return 0;
 }

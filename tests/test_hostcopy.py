@@ -35,3 +35,9 @@ def run(sim, *args):
 def test_bytes_and_way(sim, kind):
     for n in SIZES:
         run(sim, kind, n)
+
+
+@pytest.mark.parametrize("kind", ["pageable", "pinned"])
+def test_stream_of_another_device_than_the_current_one(sim, kind):
+    for n in SIZES:
+        run(sim, kind, n, 1)
