@@ -5,11 +5,14 @@ segments per second of short renders under candidate pt_config values and
 returns the fastest configuration:
 
   bvh_width x bvh_leaf   BVH arity (2, 4, 8) and primitives per leaf (1, 2, 4)
-  traversal              persistent lanes refilled from the queue (1), or one ray per lane (2)
+  traversal              the library's rule (0: whole paths in one kernel where that is faster, else
+                         a kernel per stage with persistent lanes), or one ray per lane (2); with
+                         SDFs, whose cost the rule cannot know, also the kernels per stage (1)
   wave_paths             paths in flight per wave (queue capacity); each
                          candidate is measured on dispatches that fill its wave
   blocks_per_cu          grid shape of the queue kernels (blocks of 256 lanes per CU)
-  march_blocks_per_cu    grid shape of the persistent SDF march kernels (SDF scenes)
+  march_blocks_per_cu    grid shape of the persistent SDF march kernels (SDF scenes): the library's
+                         choice (0, which leaves whole paths to the rule) or blocks per CU
   sdf_max_steps          the smallest sphere-tracing budget at which at most
                          `sdf_tolerance` of the traced rays (extension and
                          shadow) have a march run out of steps (an exhausted
@@ -43,6 +46,7 @@ LEAVES = (1, 2, 4)
 WAVES = (1 << 24, 1 << 25, 1 << 26, 1 << 27)
 BLOCKS_PER_CU = (4, 8, 16)
 MARCH_BLOCKS_PER_CU = (2, 4, 8, 16)
+TRAVERSALS = (0, 2)
 SDF_BUDGETS = (32, 48, 64, 96, 128, 192, 256)
 
 
@@ -50,10 +54,10 @@ SDF_BUDGETS = (32, 48, 64, 96, 128, 192, 256)
 class Choice:
     bvh_width: int = 2
     bvh_leaf: int = 1
-    traversal: int = 1
+    traversal: int = 0
     wave_paths: int = 1 << 27
     blocks_per_cu: int = 8
-    march_blocks_per_cu: int = 8
+    march_blocks_per_cu: int = 0
     sdf_max_steps: int = 256
 
     def context(self, **over) -> pt.Context:
@@ -128,13 +132,13 @@ def autotune(text: str, width: int, height: int, depth: int, spp: int = 0, repea
                 + (f", {t.sdf_exhausted_frac:.2e} marches exhausted" if has_sdf else ""))
         return t
 
-    # SDF budget first: the smallest that keeps exhausted marches within tolerance
+    # SDF budget first: the smallest that keeps exhausted marches within tolerance (the
+    # kernels per stage: the counters are the same in every traversal)
     if has_sdf:
         for b in SDF_BUDGETS:
-            c = Choice(**{**asdict(res.best), "sdf_max_steps": b})
-            t = run(c)
+            t = run(Choice(**{**asdict(res.best), "sdf_max_steps": b, "traversal": 1}))
             if t.sdf_exhausted_frac <= sdf_tolerance or b == SDF_BUDGETS[-1]:
-                res.best = c
+                res.best = Choice(**{**asdict(res.best), "sdf_max_steps": b})
                 break
     best_rate = 0.0
 
@@ -148,7 +152,7 @@ def autotune(text: str, width: int, height: int, depth: int, spp: int = 0, repea
 
     descend("bvh_width", WIDTHS)
     descend("bvh_leaf", LEAVES)
-    descend("traversal", (1, 2))
+    descend("traversal", TRAVERSALS + ((1,) if has_sdf else ()))
     descend("wave_paths", WAVES)
     descend("blocks_per_cu", BLOCKS_PER_CU)
     if has_sdf:

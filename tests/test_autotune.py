@@ -42,3 +42,16 @@ def test_sdf_budget_is_the_smallest_within_tolerance(monkeypatch):
     assert [c["sdf_max_steps"] for c in calls[:4]] == [32, 48, 64, 96]
     # the rest of the descent keeps the chosen budget
     assert all(c["sdf_max_steps"] == 96 for c in calls[4:])
+
+
+def test_search_starts_from_the_library_defaults(monkeypatch):
+    """An untuned context's traversal is among the candidates, and nothing in the starting point
+    keeps it from the kernels it would take."""
+    d = A.Choice()
+    assert d.traversal == 0 and d.march_blocks_per_cu == 0
+    for text in ('{"sphere": []}', '{"sdf": [{"kind": "menger"}]}'):
+        m, calls = fake_measure({"traversal": 0, "march_blocks_per_cu": 0}, {})
+        monkeypatch.setattr(A, "measure", m)
+        r = A.autotune(text, 64, 64, 8)
+        assert r.best.traversal == 0 and r.best.march_blocks_per_cu == 0
+        assert {c["traversal"] for c in calls} == ({0, 1, 2} if "sdf" in text else {0, 2})

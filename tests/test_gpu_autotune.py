@@ -50,3 +50,15 @@ def test_sdf_budget_choice():
     # exhausted fractions fall as the budget grows
     vals = [fr[x] for x in sorted(fr)]
     assert all(a >= b2 for a, b2 in zip(vals, vals[1:]))
+
+
+@pytest.mark.parametrize("text", [scenes.random_spheres(n=64, scene_seed=7), scenes.sdf_scene(seed=1)], ids=["spheres", "sdf"])
+def test_starting_point_runs_the_default_kernels(text):
+    names = []
+    for ctx in (A.Choice().context(), pt.Context(0)):
+        with ctx:
+            r = pt.Renderer(ctx, ctx.scene_from_json(text), 64, 48, spf=2, path_length=4, mode=pt.MODE_EXT)
+            ctx.profile(True)
+            r.render_frame()
+            names.append(set(ctx.profile_read()))
+    assert names[0] == names[1] and "k_ext_path" in names[0]
