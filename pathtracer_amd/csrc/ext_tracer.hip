@@ -3706,7 +3706,7 @@ int ext_dispatch_batch(pt_ctx* ctx, const ExtBatchItem* items, int n) {
         ctx->err = "batched wave: " + std::to_string(npaths) + " paths exceed the wave capacity " + std::to_string(cap);
         return PT_ERR_CAPACITY;
     }
-    whole = whole && (!plan.any_sdf || cap <= kWholeSdfPaths);
+    whole = whole && (!plan.any_sdf || npaths <= kWholeSdfPaths);  // this wave's paths, not its room
     ExtCtxState* cs = ext_state(ctx);
     // tables at fixed addresses: header, scenes, frames, segments, sinks
     const size_t o_sc = 256, o_fr = o_sc + (sizeof(ExtSceneDev) * kMaxBatch + 255) / 256 * 256,

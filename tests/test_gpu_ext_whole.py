@@ -105,12 +105,22 @@ def test_features_and_a_full_wave_in_between():
     np.testing.assert_array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
 
 
-def serve(traversal, names):
-    with pt.Context(0, traversal=traversal) as ctx, pt.Server(ctx) as server:
+def serve(traversal, names, **cfg):
+    with pt.Context(0, traversal=traversal, **cfg) as ctx, pt.Server(ctx) as server:
         ids = [server.submit(SCENES[n](), 37 + 8 * k, 29, 6, 4 + k, target=1e-6) for k, n in enumerate(names)]
         while server.step() is not None:
             pass
         return [server.read(i) for i in ids], ctx.counters()
+
+
+def served_kernels(text, w, h, spp, min_spp=8, **cfg):
+    """Images and kernel names of a served request (no graphs: their launches have no names)."""
+    with pt.Context(0, graph_mode=1, **cfg) as ctx, pt.Server(ctx, min_spp=min_spp) as server:
+        ctx.profile(True)
+        rid = server.submit(text, w, h, spp, 4, target=1e-6)
+        while server.step() is not None:
+            pass
+        return server.read(rid), set(ctx.profile_read())
 
 
 @pytest.mark.gpu
@@ -165,3 +175,23 @@ def test_budget_of_one_wave_serves_both_kinds_in_turn(ratio):
             lens.frame = lens.current = 0
             lens.render_frame()
             np.testing.assert_array_equal(lens.acc.read().view(np.uint32), first.view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["spheres", "sdf"])
+def test_a_small_wave_in_a_large_capacity(name):
+    """What a served wave holds decides which kernels trace it, not what it could hold."""
+    a, na = served_kernels(SCENES[name](), 64, 48, 8, wave_paths=1 << 26)
+    b, nb = served_kernels(SCENES[name](), 64, 48, 8, traversal=1)
+    assert "k_ext_path" in na and "k_ext_path" not in nb
+    np.testing.assert_array_equal(np.asarray(a).view(np.uint32), np.asarray(b).view(np.uint32))
+
+
+@pytest.mark.gpu
+def test_large_sdf_waves_keep_the_kernels_per_stage():
+    """Above 2^25 paths, a dispatch and a served wave (1920 x 1080, 17 samples: 35 M paths)."""
+    text = SCENES["sdf"]()
+    _, names = served_kernels(text, 1920, 1080, 17, min_spp=17, wave_paths=1 << 26)
+    assert "k_ext_path" not in names and "k_ext_march_mandelbulb" in names
+    assert "k_ext_path" not in render(0, text, 1920, 1080, 17, 2, frames=0)[2]
+    assert "k_ext_path" in render(0, text, 1920, 1080, 16, 2, frames=0)[2]
