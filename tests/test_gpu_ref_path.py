@@ -85,6 +85,22 @@ def test_sdf_kinds(kinds):
     check(sdf_scene(kinds), 96, 80, 2, 5)
 
 
+@pytest.mark.gpu
+def test_a_larger_dispatch_allocates_nothing():
+    """After a context's first dispatch its wave is there: a larger one takes no device memory."""
+    with pt.Context(0) as ctx:
+        sc = ctx.scene_from_json((GOLDEN / "scene0.json").read_text())
+        r = [pt.Renderer(ctx, sc, w, h, spf=2, path_length=3) for w, h in ((32, 24), (640, 480), (1920, 1080))]
+        free, total = C.c_size_t(), C.c_size_t()
+        left = []
+        for x in r:
+            x.render_frame()
+            ctx.sync()
+            assert pt.lib.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+            left.append(free.value)
+        assert left[1:] == left[:1] * 2
+
+
 POW_C = r"""
 #include "ptmath.h"
 void slow(const float* x, float* o, int n, float e) { for (int i = 0; i < n; ++i) o[i] = ptm_pow(x[i], e); }
