@@ -2406,17 +2406,34 @@ constexpr int kPathSteps = 2, kPathVisits = 4;
 // memory. The scene and frame come through scalar loads where they are used, not as
 // by-value arguments loaded at the start, which filled the scalar registers and spilled
 // into vector ones (120 against 96 VGPRs, 4 against 5 waves per SIMD).
-// Rule (whole_takes, ext_run): scenes without SDFs at any size, with SDFs dispatches of at
-// most kWholeSdfPaths: a large wave hides the marches' tails, and the march kernels keep
+// Rule (whole_takes, whole_paths): scenes without SDFs at any size, with SDFs waves of at
+// most whole_paths: a large wave hides the marches' tails, and the march kernels keep
 // their lanes on one estimator. Kernels per stage against this one, ms, 1920 x 1080 at
 // depth 12 with 4 / 16 / 64 samples: 30 spheres 2.81 / 7.38 / 25.6 against 1.64 / 5.63 /
 // 21.8, 300 4.03 / 10.9 / 37.4 against 2.69 / 9.25 / 35.9, 1000 5.07 / 13.3 / 46.2 against
-// 3.44 / 11.9 / 46.0, 4096 5.95 / 14.5 / 49.2 against 3.65 / 12.2 / 46.7; mandelbulb and
-// menger at depth 8 with 1 / 4 / 16 / 32 / 64 samples 5.3 / 7.4 / 15.2 / 24.9 / 44.1 against
-// 1.5 / 3.8 / 12.7 / 24.6 / 48.5. Batched waves of a served burst 32.1 against 10.5 ms.
+// 3.44 / 11.9 / 46.0, 4096 5.95 / 14.5 / 49.2 against 3.65 / 12.2 / 46.7, 32000 (1 / 16 /
+// 64) 3.1 / 13.3 / 45.5 against 1.5 / 11.6 / 44.1; mandelbulb and menger at depth 8 with
+// 1 / 4 / 16 / 32 / 64 samples 5.3 / 7.4 / 15.2 / 24.9 / 44.1 against 1.5 / 3.8 / 12.7 /
+// 24.6 / 48.5, and 2.1 to 2.7 times as fast at 1, 1.2 to 2.0 at 16 for each estimator
+// alone. Batched waves of a served burst 32.1 against 10.5 ms.
 // `direct`: the dispatch has one sample per pixel, all in this wave, and the paths'
 // texels are finished here instead of by k_ext_fold.
-constexpr int kWholeSdfPaths = 1 << 25;
+// Paths up to which a scene with SDFs goes whole (whole_paths). Without spheres the line is
+// kWholeSdfPaths: at 16 samples of 1920 x 1080 (33 M paths, depth 8, a parallelogram light)
+// 1.00 (terrain) to 1.47 times as fast as the kernels per stage for each estimator and the
+// four together. Among spheres a ray waits for the wave's scene work twice, after the BVH and
+// after the march, and the marches run on fewer lanes; how much of the tails is left to win
+// depends on the estimator. 3 and 100 spheres, under a sky and with a sphere light, at 4.1 /
+// 8.3 / 16.6 / 33 M paths: blob 1.5 to 2.1 / 1.3 to 1.9 / 1.1 to 1.9 / 1.0 to 1.7; menger 1.6 to
+// 1.8 / 1.3 to 1.6 / 1.1 to 1.4 / 0.94 to 1.3; mandelbulb, alone, with menger and with all, 1.5 to
+// 2.2 / 1.25 to 1.8 / 1.01 to 1.4 / 0.85 to 1.1; terrain, alone, with blob and with menger, whose
+// marches are short and whose normals cost the shading 6 evaluations of 22 sines, 1.1 to 1.4 /
+// 0.9 to 1.2 / 0.7 to 1.0 / 0.7 to 0.9, and one whose terrain fills the image 1.02 at 2.8 M and 0.95
+// at 3.7 M. Served waves (npaths of all requests; their kernels per stage march one ray per
+// lane) keep the line of scenes without spheres: 1.04 to 2.6 times as fast up to their usual
+// 4.2 M. Estimators whose box cuts them down to a solid core have no tails: in a box of 30 to
+// 300 spheres 1.15 to 1.2 at 4.1 M, 0.83 to 1.0 from there on, 0.77 to 0.9 in served waves.
+constexpr int kWholeSdfPaths = 1 << 25, kWholeSdfSpheres = 1 << 24, kWholeTerrainSpheres = 3 << 20;
 // A batched wave's tables (in constant memory for the kernel's length, so that a
 // request's scene comes through scalar loads), and its cursors: kSeg a request, then the
 // count of ended waves.
@@ -3546,6 +3563,14 @@ static bool whole_takes(const pt_ctx* ctx, const ExtSceneHost& H) {
     return (H.dev.nsdf == 0 || march) && !H.dev.quad_bvh && H.dev.nlens + H.dev.ncyc == 0 && H.width == 2 &&
            H.small_nodes && H.stack_need <= kPathStack && ctx->cfg.traversal == 0;
 }
+// The most paths of a dispatch of this scene that go whole (k_ext_path has the reasons).
+static int64_t whole_paths(const ExtSceneHost& H) {
+    if (H.dev.nsdf == 0) return INT64_MAX;
+    auto has = [&](int kind) { return std::find(H.sdf_kinds.begin(), H.sdf_kinds.end(), kind) != H.sdf_kinds.end(); };
+    const bool only_blob = H.sdf_kinds.size() == 1 && has(PT_SDF_BLOB);
+    if (H.dev.nsph == 0 || only_blob) return kWholeSdfPaths;
+    return has(PT_SDF_TERRAIN) && !has(PT_SDF_MANDELBULB) ? kWholeTerrainSpheres : kWholeSdfSpheres;
+}
 // Waves of the whole-path kernel that the device holds at once.
 static int path_grid(pt_ctx* ctx, bool sdf, bool multi) {
     int& w = ctx->path_waves[(sdf ? 1 : 0) + (multi ? 2 : 0)];
@@ -3566,8 +3591,8 @@ static int ext_run(pt_ctx* ctx, const pt_scene* s, const pt_push_constants* pc, 
     // allocated for what this dispatch needs, up to that capacity.
     int64_t cap = ctx->cfg.wave_paths > 0 ? ctx->cfg.wave_paths : kDispatchWave;
     cap = std::max<int64_t>(1024, std::min<int64_t>(cap, (int64_t)P * std::max(1, pc->samplesPerFrame)));
-    // whole paths in one kernel, or a kernel per stage and bounce (k_ext_path has the rule's reasons)
-    const bool whole = whole_takes(ctx, H) && (H.dev.nsdf == 0 || cap <= kWholeSdfPaths);
+    // whole paths in one kernel, or a kernel per stage and bounce
+    const bool whole = whole_takes(ctx, H) && cap <= whole_paths(H);
     ExtWave* wave = nullptr;
     if (whole) {
         st = ensure_lean_wave(ctx, (int)cap, &wave);

@@ -195,3 +195,28 @@ def test_large_sdf_waves_keep_the_kernels_per_stage():
     assert "k_ext_path" not in names and "k_ext_march_mandelbulb" in names
     assert "k_ext_path" not in render(0, text, 1920, 1080, 17, 2, frames=0)[2]
     assert "k_ext_path" in render(0, text, 1920, 1080, 16, 2, frames=0)[2]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kinds,size,whole", [
+    (("mandelbulb", "menger"), (1920, 1080, 8), True),  # 16.6 M paths
+    (("mandelbulb", "menger"), (1920, 1080, 9), False),
+    (("terrain", "mandelbulb"), (1920, 1080, 2), True),
+    (("terrain",), (1280, 720, 3), True),  # 2.8 M
+    (("terrain",), (1280, 720, 4), False),
+    (("terrain", "blob"), (1280, 720, 4), False),
+    (("blob",), (1920, 1080, 16), True),  # 33.2 M
+    (("blob",), (1920, 1080, 17), False),
+])
+def test_sdfs_among_spheres_go_whole_up_to_a_size(kinds, size, whole):
+    """Where the line lies, and the same images on both sides of it."""
+    s = json.loads(SCENES["sdf_spheres"]())
+    base = {d["kind"]: d for d in s["sdf"]}
+    base["terrain"] = {"kind": "terrain", "position": [0, 0.5, 2.5], "boundingSize": [8, 6, 8], "material": 1.0}
+    base["blob"] = dict(base["terrain"], kind="blob", position=[0, 1, 2.5], boundingSize=[3, 3, 3])
+    s["sdf"] = [base[k] for k in kinds]
+    w, h, spp = size
+    a, _, na = render(0, json.dumps(s), w, h, spp, 3, frames=0)
+    b, _, nb = render(1, json.dumps(s), w, h, spp, 3, frames=0)
+    assert ("k_ext_path" in na) == whole and "k_ext_path" not in nb
+    np.testing.assert_array_equal(a.view(np.uint32), b.view(np.uint32))
