@@ -2446,6 +2446,8 @@ struct ExtPathBatch {
     int* cursor;
 };
 constexpr int kBatchCursors = kMaxBatch * kSeg + 1;
+// F0 has to stay the first parameter: a single scene's frame is read where it lies at the
+// start of the kernel-argument segment.
 template <bool MULTI, bool SDF>
 __global__ void __launch_bounds__(kPathLanes, 5) k_ext_path(ExtFrame F0, ExtWave Wv, ExtFinish Fin,
                                                             float4* texels, int direct, int aov, int count_dispatch,

@@ -46,9 +46,13 @@ def test_atomics_without_memory_for_partials():
     n, h, w = 3, 20, 68
     p, feat, target = setup(n, h, w)
     with pt.Context(0) as ctx:
+        ctx.profile(True)
         _, g = gradients(ctx, n, h, w, p, feat, target)
+        assert "k_dn_grad_sum" in ctx.profile_read()
     with pt.Context(0, hbm_budget=20 << 20) as ctx:  # the denoiser takes 17 MB, the partials more than the rest
+        ctx.profile(True)
         _, a = gradients(ctx, n, h, w, p, feat, target)
+        assert "k_dn_grad_sum" not in ctx.profile_read()
     assert np.linalg.norm(a - g) <= 4080 * 2.0 ** -24 * np.linalg.norm(g)
 
 

@@ -1,9 +1,9 @@
-"""The extended mode's whole-path kernel (small dispatches and scenes) against the
-kernels per stage and bounce (traversal = 1), bit for bit with equal counters: the
-two are the same device functions in the same order per path. Image edges around
-a wave, one sample (finished in the kernel) and several, waves smaller than the
-image, path lengths 0 and 1, scenes with and without spheres, planes, sky and
-sphere lights, and the features sink."""
+"""The extended mode's whole-path kernel against the kernels per stage and bounce
+(traversal = 1), bit for bit with equal counters: the two are the same device
+functions in the same order per path. Image edges around a wave, one sample (finished
+in the kernel) and several, waves smaller than the image, path lengths 0 and 1, scenes
+with and without spheres, planes, sky and sphere lights, the features sink, served
+waves, and which of the two forms runs: by scene, by size, by the memory there is."""
 import json
 
 import numpy as np
@@ -26,6 +26,14 @@ def plane_and_sky(spheres=3, light=True):
     return json.dumps(s)
 
 
+def lens_scene():
+    """The spheres' box with a lens in it, which the whole-path kernel does not take."""
+    s = scenes.cornell_dict(4, seed=7)
+    s["lens"] = [{"position": [0.5, 0.5, 0.4], "rotation": [0.0, 0.0, 0.0], "radius": 0.2, "focalLength": 0.3,
+                  "thickness": 0.0, "isConverging": True, "materialID": 1, "lightID": 0}]
+    return json.dumps(s)
+
+
 SCENES = {
     "spheres": lambda: scenes.random_spheres(n=500, scene_seed=2, wavelengths=4, seed=7),
     "cornell1": lambda: scenes.cornell(1, seed=7),
@@ -33,6 +41,7 @@ SCENES = {
     "no_light": lambda: plane_and_sky(light=False),
     "quads_only": lambda: json.dumps(dict(scenes.cornell_dict(4, seed=7), sphere=[])),
     "sdf": lambda: scenes.sdf_scene(seed=3),
+    "lens": lens_scene,
     "sdf_spheres": lambda: json.dumps(dict(json.loads(plane_and_sky()), sdf=json.loads(scenes.sdf_scene(seed=3))["sdf"])),
 }
 COUNTERS = ("sdf_steps", "sdf_exhausted", "segments", "shadow_segments", "paths", "nan_samples", "dispatches", "escaped", "emitter_hits", "lambert_hits",
@@ -59,7 +68,7 @@ def check(text, w, h, spp, depth, **k):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("name", SCENES)
+@pytest.mark.parametrize("name", [n for n in SCENES if n != "lens"])
 @pytest.mark.parametrize("spp", [1, 3])
 def test_scenes(name, spp):
     check(SCENES[name](), 61, 37, spp, 7)
@@ -85,32 +94,50 @@ def test_waves_smaller_than_the_image(spp):
 
 
 @pytest.mark.gpu
-def test_features_and_a_full_wave_in_between():
-    """First-hit features of both forms; and a context whose full wave (a scene the
-    whole-path kernel does not take) serves the whole-path kernel afterwards."""
+@pytest.mark.parametrize("full_first", [False, True])
+def test_features_and_a_full_wave_in_between(full_first):
+    """First-hit features of both forms; and a context whose full wave (a scene the whole-path
+    kernel does not take) serves the whole-path kernel afterwards, in place of a lean one or
+    before there is one, with the cursors that wave holds, in dispatches and served waves."""
     text = SCENES["spheres"]()
     out = []
     for tr in (0, 1):
-        with pt.Context(0, traversal=tr) as ctx:
+        with pt.Context(0, traversal=tr, graph_mode=1, wave_paths=8192) as ctx:  # what the full wave holds
+            ctx.profile(True)
+            ran = lambda: "k_ext_path" in ctx.profile_read(True)  # noqa: E731
             sc = ctx.scene_from_json(text)
             pc = pt.push_constants(45, 31, 3, 5)
             sc.camera(1, pc)
             pc.frame = pc.currentSamples = 3
-            first = ctx.features(sc, pc)
-            sdf = ctx.scene_from_json(scenes.sdf_scene(seed=3))
-            pt.Renderer(ctx, sdf, 64, 48, spf=4, path_length=3, mode=pt.MODE_EXT).render_frame()
-            for _ in range(2):
-                np.testing.assert_array_equal(ctx.features(sc, pc).view(np.uint32), first.view(np.uint32))
-            out.append(first)
-    np.testing.assert_array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
+            images = []
+            for full in ((True, False, False) if full_first else (False, True, False)):
+                if full:
+                    lens = ctx.scene_from_json(lens_scene())
+                    pt.Renderer(ctx, lens, 64, 48, spf=4, path_length=3, mode=pt.MODE_EXT).render_frame()
+                    assert not ran()
+                images.append(ctx.features(sc, pc))
+                assert ran() == (tr == 0)
+                with pt.Server(ctx) as server:
+                    rid = server.submit(text, 24, 16, 8, 4, target=1e-6)
+                    while server.step() is not None:
+                        pass
+                    images.append(np.asarray(server.read(rid)))
+                assert ran() == (tr == 0)
+            for x in images:
+                np.testing.assert_array_equal(x.view(np.uint32), images[x.shape[-1] != pt.FEATURES].view(np.uint32))
+            out.append(images[:2])
+    for x, y in zip(*out):
+        np.testing.assert_array_equal(x.view(np.uint32), y.view(np.uint32))
 
 
 def serve(traversal, names, **cfg):
+    """Images, counters and kernel names (only of graph_mode 1: a graph's launches have none)."""
     with pt.Context(0, traversal=traversal, **cfg) as ctx, pt.Server(ctx) as server:
+        ctx.profile(cfg.get("graph_mode") == 1)
         ids = [server.submit(SCENES[n](), 37 + 8 * k, 29, 6, 4 + k, target=1e-6) for k, n in enumerate(names)]
         while server.step() is not None:
             pass
-        return [server.read(i) for i in ids], ctx.counters()
+        return [np.asarray(server.read(i)) for i in ids], ctx.counters(), set(ctx.profile_read())
 
 
 def served_kernels(text, w, h, spp, min_spp=8, **cfg):
@@ -126,20 +153,61 @@ def served_kernels(text, w, h, spp, min_spp=8, **cfg):
 @pytest.mark.gpu
 @pytest.mark.parametrize("names", [["spheres", "plane_sky"], ["sdf", "spheres", "sdf_spheres", "quads_only", "sdf"]])
 def test_batched_waves(names):
-    """Requests of several scenes in one wave, with and without SDFs: the same images."""
-    a, ca = serve(0, names)
-    b, cb = serve(1, names)
+    """Requests of several scenes in one wave, with and without SDFs: the same images, from a
+    captured graph and from launches one by one."""
+    a, ca, _ = serve(0, names)
+    g, cg, ng = serve(0, names, graph_mode=1)
+    b, cb, nb = serve(1, names, graph_mode=1)
+    assert "k_ext_path" in ng and "k_ext_path" not in nb
+    for x, y, z in zip(a, g, b):
+        np.testing.assert_array_equal(x.view(np.uint32), z.view(np.uint32))
+        np.testing.assert_array_equal(y.view(np.uint32), z.view(np.uint32))
+    assert {c: ca[c] for c in COUNTERS} == {c: cg[c] for c in COUNTERS} == {c: cb[c] for c in COUNTERS}
+
+
+@pytest.mark.gpu
+def test_a_wave_with_a_scene_the_kernel_does_not_take():
+    """One lens among the requests: the wave runs the kernels per stage, with the same images as
+    every form, and as the other requests get without it."""
+    names = ["spheres", "sdf", "lens", "quads_only"]
+    a, ca, na = serve(0, names, graph_mode=1)
+    b, cb, _ = serve(1, names)
+    alone, _, nl = serve(0, names[:2], graph_mode=1)
+    assert "k_ext_path" not in na and "k_ext_path" in nl
     for x, y in zip(a, b):
-        np.testing.assert_array_equal(np.asarray(x).view(np.uint32), np.asarray(y).view(np.uint32))
+        np.testing.assert_array_equal(x.view(np.uint32), y.view(np.uint32))
+    for x, y in zip(a, alone):
+        np.testing.assert_array_equal(x.view(np.uint32), y.view(np.uint32))
     assert {c: ca[c] for c in COUNTERS} == {c: cb[c] for c in COUNTERS}
 
 
-def lens_scene():
-    """The spheres' box with a lens in it, which the whole-path kernel does not take."""
-    s = scenes.cornell_dict(4, seed=7)
-    s["lens"] = [{"position": [0.5, 0.5, 0.4], "rotation": [0.0, 0.0, 0.0], "radius": 0.2, "focalLength": 0.3,
-                  "thickness": 0.0, "isConverging": True, "materialID": 1, "lightID": 0}]
-    return json.dumps(s)
+@pytest.mark.gpu
+def test_no_room_for_the_batch_cursors():
+    """The smallest budgets that serve a request beside a full wave have no room for the whole-path
+    kernel's batch cursors: the kernels per stage serve it; with more room the kernel does."""
+    text = SCENES["spheres"]()
+    want, _ = served_kernels(text, 40, 24, 8, traversal=1)
+    served = []
+    paths, step = 1 << 16, 64 << 10
+    for budget in range(FULL_PATH * paths, FULL_PATH * paths + (4 << 20), step):
+        with pt.Context(0, graph_mode=1, wave_paths=paths, hbm_budget=budget) as ctx:
+            try:
+                lens = ctx.scene_from_json(lens_scene())
+                pt.Renderer(ctx, lens, 64, 64, spf=16, path_length=2, mode=pt.MODE_EXT).render_frame()
+                ctx.profile(True)
+                with pt.Server(ctx) as server:
+                    rid = server.submit(text, 40, 24, 8, 4, target=1e-6)
+                    while server.step() is not None:
+                        pass
+                    got = np.asarray(server.read(rid))
+            except pt.PTError as e:
+                assert e.status == pt.PT_ERR_BUDGET and not served
+                continue
+            np.testing.assert_array_equal(got.view(np.uint32), np.asarray(want).view(np.uint32))
+            served.append("k_ext_path" in ctx.profile_read())
+        if served[-1]:
+            break
+    assert len(served) > 1 and served == [False] * (len(served) - 1) + [True]
 
 
 FULL_PATH, LEAN_PATH = 336, 60  # bytes a path of the two waves
