@@ -24,8 +24,8 @@ paths); the timed region is exactly `--steps` dispatches bracketed by stream
 synchronisation, with the scene, BVH and path buffers resident in HBM.
 
 Prints one JSON line: metric, value (spectral path-segments/s), roofline of
-the dominant kernel (algorithmic bytes, or for a sphere-tracing kernel FP32
-operations, over its average HIP-event duration), and the CPU baseline (the
+the dominant kernel (algorithmic bytes, or for a sphere-tracing or whole-path
+kernel FP32 operations, over its average HIP-event duration), and the CPU baseline (the
 oracle timed on this host on a bounded sample).
 """
 from __future__ import annotations
@@ -71,12 +71,23 @@ BYTES_PER_UNIT = {
     "k_ext_classify": [(32, "segments")],
     "k_ext_shadow": [(68, "shadow_segments")],
     "k_ext_shade_lambert": [(160, "lambert_hits")],
-    # reference mode: a path stays in its lane's registers and leaves its XYZ, 16 B, which the
-    # fold reads (the kernel is bound by VALU issue, the shader's transcendentals restated)
-    "k_ref_path": [(16, "paths")],
-    # extended mode's whole paths: the same
-    "k_ext_path": [(16, "paths")],
+    # reference mode's fold of several samples: a path's XYZ
     "k_ref_fold": [(16, "paths")],
+}
+
+# The whole-path kernels keep a path in registers from the camera to its end (16 B of XYZ
+# leave it) and are bound by VALU issue. Priced here by the FP32 operations that no
+# traversal can do without, one per add, multiply, min or max, two per fused multiply-add;
+# shading, random numbers and new rays come on top:
+#   k_ext_path: 48 per BVH node visited (two children's slabs: 6 fused multiply-adds, 6 min and 6
+#     max each), extension and shadow rays alike, plus the counted operations of its marches
+#   k_ref_path, on scene1.json: 97 per ray (its 3 spheres 20 each, the plane 5, 2 boxes' bounding
+#     spheres 16 each)
+OPS_PER_UNIT = {
+    "k_ext_path": [(48, "bvh_nodes"), (48, "shadow_bvh_nodes"), (1, "march_flops_mandelbulb"),
+                   (1, "march_flops_menger"), (1, "march_flops_blob"), (1, "march_flops_terrain"),
+                   (1, "shadow_march_flops")],
+    "k_ref_path": [(97, "segments"), (97, "shadow_segments")],
 }
 
 # Sphere-tracing kernels are bound by FP32 VALU work, not HBM. Their algorithmic
@@ -143,8 +154,11 @@ def parse_args():
     ap.add_argument("--bvh-width", type=int, default=0)
     ap.add_argument("--bvh-leaf", type=int, default=0)
     ap.add_argument("--wave-paths", type=int, default=0)
-    ap.add_argument("--traversal", type=int, default=0, help="0 default (persistent), 1 persistent lanes refilled from the queue, 2 one ray per lane")
-    ap.add_argument("--march", type=int, default=0, help="SDF march: 0 persistent lanes refilled from the queue, 1 one ray per lane")
+    ap.add_argument("--traversal", type=int, default=0,
+                    help="0 default (whole paths in one kernel where it takes the scene, else 1), 1 a kernel per stage "
+                         "with persistent lanes, 2 the same with one ray per lane")
+    ap.add_argument("--march", type=int, default=0,
+                    help="SDF march of the kernels per stage: 0 persistent lanes refilled from the queue, 1 one ray per lane")
     ap.add_argument("--march-blocks", type=int, default=0, help="blocks per CU of the persistent march (0 = default)")
     ap.add_argument("--cpu-seconds", type=float, default=12.0, help="target CPU-baseline sample duration")
     ap.add_argument("--no-cpu-baseline", action="store_true")
@@ -269,18 +283,20 @@ def measured_peaks():
 def roofline_of(prof: dict, pcnt: dict, workload: str, tag: str):
     """The roofline object of the dominant kernel: prof maps kernel names to
     (launches, total ms) from the HIP events, pcnt holds the device counters of
-    the same dispatches. SDF marches are priced in FP32 flops against the VALU
-    peak, the other kernels in algorithmic bytes against HBM; both carry the
-    measured peak beside the published one."""
+    the same dispatches. SDF marches and whole paths are priced in FP32 flops
+    against the VALU peak, the other kernels in algorithmic bytes against HBM;
+    both carry the measured peak beside the published one."""
     roofline = None
     mp = measured_peaks()
     if prof:
         dom = max(prof.items(), key=lambda kv: kv[1][1])
         name, (launches, total_ms) = dom
         terms = BYTES_PER_UNIT.get(name)
-        fl = FLOPS_COUNTER.get(name) if workload == "sdf" else None
-        if fl and launches > 0:
-            flops = pcnt.get(fl, 0)
+        ops = OPS_PER_UNIT.get(name)
+        if workload == "sdf" and name in FLOPS_COUNTER:
+            ops = [(1, FLOPS_COUNTER[name])]
+        if ops and launches > 0:
+            flops = sum(n * pcnt.get(unit, 0) for n, unit in ops)
             achieved = flops / (total_ms * 1e-3) / 1e12
             roofline = {
                 "bound": "valu",

@@ -860,13 +860,13 @@ constexpr int kRefLanes = 64;  // threads per block: one wave, so that few paths
 // without SDF objects, PT_SDF_* when all are of one kind, 0 when they are mixed.
 // It replaced a kernel per stage and bounce (36 launches for a frame of 5 bounces,
 // path records of 168 bytes in memory between them, one ray per lane in the
-// marches) and is bound by VALU issue in analytic scenes (rocprofv3: saturated, 34 of
-// 64 lanes active, about 1650 instructions of a lane per segment with its shading and
-// shadow ray): 1280x720x1 5 bounces 966 -> 230 us, 1920x1080x8 8 bounces 15.8 ->
+// marches) and is bound by VALU issue in analytic scenes (rocprofv3, 3 spheres, a plane and
+// 2 boxes at 512x512x8: 0.82 wave instructions per unit and clock, 27 of 64 lanes active, 1660
+// instructions of a lane per segment with its shading and shadow ray): 1280x720x1 5 bounces 966 -> 230 us, 1920x1080x8 8 bounces 15.8 ->
 // 2.8 ms, 150x101x1 288 -> 81 us of kernels (one launch, its length the chain of a
 // path's bounces). SDF scenes are bound by the chain of their longest path (512x512x4
 // mandelbulb: up to 728 distance evaluations of 8 iterations, about 3.8 us each):
-// 29.2 -> 5.7 ms. Registers: 165 (analytic) and 191 (SDF) leave 3 and 2 waves per SIMD;
+// 29.2 -> 5.7 ms. Registers: 165 (analytic) and 184 to 190 (SDF) leave 3 and 2 waves per SIMD;
 // asking for 4 spills and was 20 % slower, and the path state in LDS while marching gave
 // nothing.
 // `direct`: the dispatch has one sample per pixel, all in this wave, and the

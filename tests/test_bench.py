@@ -59,13 +59,13 @@ def launch_names():
 def test_roofline_tables_name_launched_kernels():
     names = launch_names()
     assert "k_ext_intersect" in names and "k_ext_march_mandelbulb" in names
-    for k in list(bench.BYTES_PER_UNIT) + list(bench.FLOPS_COUNTER):
+    for k in list(bench.BYTES_PER_UNIT) + list(bench.FLOPS_COUNTER) + list(bench.OPS_PER_UNIT):
         assert k in names, k
 
 
 def test_roofline_units_are_counters():
     fields = {f for f, _ in pt.Counters._fields_}
-    for terms in bench.BYTES_PER_UNIT.values():
+    for terms in list(bench.BYTES_PER_UNIT.values()) + list(bench.OPS_PER_UNIT.values()):
         for bytes_per_unit, unit in terms:
             assert bytes_per_unit > 0 and unit in fields, unit
     for counter in bench.FLOPS_COUNTER.values():
@@ -84,7 +84,7 @@ def test_peak_probe_flag():
 
 
 def test_roofline_of_an_hbm_kernel():
-    """The headline's dominant kernel priced in algorithmic bytes against the
+    """A kernel of the per-stage traversal priced in algorithmic bytes against the
     published and the measured HBM peaks, traffic from its committed profile."""
     name = "k_ext_intersect"
     (bpu, unit), = bench.BYTES_PER_UNIT[name]
@@ -98,6 +98,21 @@ def test_roofline_of_an_hbm_kernel():
     assert r["peak_measured"] == mp["GB/s"] and r["frac_measured"] == round(achieved / mp["GB/s"], 5)
     assert r["traffic"] == bench.traffic_from_profiles(name, "spheres4096_1920x1080") and r["traffic"] > 0
     assert r["avg_launch_ms"] == 3.0 and r["algorithmic_bytes_per_launch"] == round(bpu * 1e9 / 12)
+
+
+@pytest.mark.parametrize("workload,tag", [("spheres", "spheres4096_1920x1080"), ("cornell", "cornell_512x512"),
+                                          ("sdf", "sdf_1920x1080")])
+def test_roofline_of_whole_paths(workload, tag):
+    """The headline's dominant kernel priced in FP32 operations, with the issue share and the
+    traffic of its committed profile."""
+    pcnt = {"bvh_nodes": 10**9, "shadow_bvh_nodes": 3 * 10**8, "march_flops_menger": 5 * 10**9, "paths": 10**6}
+    r = bench.roofline_of({"k_ext_path": (4, 20.0), "k_ext_fold": (4, 1.0)}, pcnt, workload, tag)
+    flops = 48 * 1.3e9 + 5e9
+    achieved = flops / 20e-3 / 1e12
+    assert r["bound"] == "valu" and r["kernel"] == "k_ext_path" and r["unit"] == "TFLOP/s"
+    assert r["achieved"] == round(achieved, 3) and r["frac"] == round(achieved / bench.FP32_PEAK_TFLOPS, 5)
+    assert r["algorithmic_flops_per_launch"] == round(flops / 4) and r["avg_launch_ms"] == 5.0
+    assert r["valu_issue_share"] > 0.5 and r["traffic"] > 0
 
 
 def test_roofline_of_an_sdf_march():
