@@ -4,10 +4,10 @@ For one workload (scene JSON, resolution, path length) it measures traced
 segments per second of short renders under candidate pt_config values and
 returns the fastest configuration:
 
-  bvh_width x bvh_leaf   BVH arity (2, 4, 8) and primitives per leaf (1, 2, 4)
+  bvh_width x bvh_leaf   BVH arity (2, 4, 8) and primitives per leaf (1, 2, 4), for scenes that
+                         have a BVH (elsewhere noise would choose, and only arity 2 goes whole)
   traversal              the library's rule (0: whole paths in one kernel where that is faster, else
-                         a kernel per stage with persistent lanes), or one ray per lane (2); with
-                         SDFs, whose cost the rule cannot know, also the kernels per stage (1)
+                         a kernel per stage with persistent lanes), or one ray per lane (2)
   wave_paths             paths in flight per wave (queue capacity); each
                          candidate is measured on dispatches that fill its wave
   blocks_per_cu          grid shape of the queue kernels (blocks of 256 lanes per CU)
@@ -150,9 +150,10 @@ def autotune(text: str, width: int, height: int, depth: int, spp: int = 0, repea
             if t.segments_per_s > best_rate:
                 best_rate, res.best = t.segments_per_s, c
 
-    descend("bvh_width", WIDTHS)
-    descend("bvh_leaf", LEAVES)
-    descend("traversal", TRAVERSALS + ((1,) if has_sdf else ()))
+    if any(f'"{k}"' in text for k in ("sphere", "quad", "box")):
+        descend("bvh_width", WIDTHS)
+        descend("bvh_leaf", LEAVES)
+    descend("traversal", TRAVERSALS)
     descend("wave_paths", WAVES)
     descend("blocks_per_cu", BLOCKS_PER_CU)
     if has_sdf:

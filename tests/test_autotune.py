@@ -54,4 +54,13 @@ def test_search_starts_from_the_library_defaults(monkeypatch):
         monkeypatch.setattr(A, "measure", m)
         r = A.autotune(text, 64, 64, 8)
         assert r.best.traversal == 0 and r.best.march_blocks_per_cu == 0
-        assert {c["traversal"] for c in calls} == ({0, 1, 2} if "sdf" in text else {0, 2})
+        assert {c["traversal"] for c in calls if c["sdf_max_steps"] == r.best.sdf_max_steps} >= {0, 2}
+
+
+def test_no_bvh_parameters_without_a_bvh(monkeypatch):
+    """Whatever their noise: a scene of planes and SDFs keeps the defaults for both."""
+    m, calls = fake_measure({"bvh_width": 4, "bvh_leaf": 2}, {})
+    monkeypatch.setattr(A, "measure", m)
+    r = A.autotune('{"plane": [], "sdf": [{"kind": "menger"}]}', 64, 64, 8)
+    assert (r.best.bvh_width, r.best.bvh_leaf) == (2, 1) and {c["bvh_width"] for c in calls} == {2}
+    assert A.autotune('{"box": [], "sdf": [{"kind": "menger"}]}', 64, 64, 8).best.bvh_width == 4
