@@ -125,23 +125,29 @@ typedef enum pt_mode { PT_MODE_REF = 0, PT_MODE_EXT = 1 } pt_mode;
 
 /* Launch/tuning knobs (0 = library default). */
 typedef struct pt_config {
-    int32_t wave_paths;    /* paths in flight per wave (queue capacity); 0 = 2^27 for pt_dispatch (allocated as a
-                              dispatch needs, about 330 B per path) and 2^22 for a server's batched waves */
+    int32_t wave_paths;    /* paths in flight per wave (queue capacity); 0 = 2^27 for extended-mode dispatches
+                              (allocated as a dispatch needs, 60 B per path where whole paths are traced in one
+                              kernel, else 336 B), 2^22 for a server's batched waves and 2^23 in reference mode
+                              (28 B per path, allocated whole by the first dispatch unless hbm_budget is set) */
     int32_t block_size;    /* threads per block of the queue kernels: 0 or 256 (they are compiled for 256
                               lanes, 4 wavefronts; other values are rejected) */
     int32_t bvh_width;     /* 2, 4 or 8 (0 = 2) */
     int32_t sdf_max_steps; /* sphere-tracing budget of the extended mode */
     int64_t hbm_budget;    /* bytes this context may allocate (0 = no limit) */
-    int32_t traversal;     /* extended mode, single-scene dispatches: 0 = the default (whole paths in one kernel for
-                              small dispatches and scenes, else 1), 1 = a kernel per stage and bounce, persistent
-                              lanes refilled from the queue, 2 = the same with one ray per lane. Batched waves and
-                              scenes with a parallelogram BVH take one ray per lane. */
+    int32_t traversal;     /* extended mode: 0 = the default: whole paths in one kernel, in dispatches and in a
+                              server's batched waves, for scenes of spheres (bvh_width 2, up to 65535 nodes), at most
+                              16 parallelograms, planes and SDFs, those with SDFs up to 2^25 paths (fewer among
+                              spheres, by estimator), unless march or march_blocks_per_cu is set; else 1. 1 = a
+                              kernel per stage and bounce, persistent lanes refilled from the queue; 2 = the same
+                              with one ray per lane, as batched waves and scenes with a parallelogram BVH always
+                              do there. Images are the same bit for bit. */
     int32_t bvh_leaf;      /* most primitives per BVH leaf, 1..16 (0 = 1) */
     int32_t graph_mode;    /* batched serving waves: 0 = captured once per launch shape into a hipGraph and
                               replayed, 1 = kernels launched one by one */
-    int32_t blocks_per_cu; /* extended mode: grid of the queue kernels, blocks per compute unit, 1..64 (0 = 8) */
-    int32_t march;         /* extended mode, SDF sphere tracing: 0 = persistent lanes refilled from the queue,
-                              1 = one ray per lane */
+    int32_t blocks_per_cu; /* extended mode: grid of the per-stage queue kernels, blocks per compute unit, 1..64
+                              (0 = 8) */
+    int32_t march;         /* extended mode, SDF sphere tracing per stage: 0 = persistent lanes refilled from the
+                              queue, 1 = one ray per lane (and no whole paths for scenes with SDFs) */
     int32_t march_blocks_per_cu; /* extended mode: grid of the persistent march kernels, blocks per compute unit,
                                     1..64 (0 = the default) */
 } pt_config;

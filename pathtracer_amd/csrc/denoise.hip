@@ -3,7 +3,8 @@
 // reference.
 //
 // Network (NHWC BF16 activations, FP32 accumulation, FP32 master weights):
-//   in  16 ch: log1p(XYZ) (3), albedo (3), normal (3), 1 / (1 + depth) (1), zeros (6)
+//   in  16 ch: log1p(XYZ) (3), albedo (3), normal (3), 1 / (1 + depth) (1), log1p(standard error) (1),
+//              1 / sqrt(samples) (1), zeros (4)
 //   e0: conv 16->32, conv 32->32                      (H x W)      skip0
 //   e1: avgpool 2, conv 32->64, conv 64->64           (H/2)        skip1
 //   b : avgpool 2, conv 64->128, conv 128->128        (H/4)
@@ -24,9 +25,10 @@
 //     tile; backward-data runs the forward kernel on the output gradient with
 //     the weights flipped and transposed;
 //   backward-weights: rows = output channels, columns = input channels,
-//     K = pixels; each wave stages 16 pixels x 32 channels of both operands in
-//     LDS to read them transposed, and adds its partial sums into the FP32
-//     gradient with atomics.
+//     K = pixels; a block stages tiles of 4 x 32 pixels of both operands in LDS,
+//     transposed, for all 9 taps, and writes its FP32 partial sums, which
+//     k_grad_sum adds in order (into the gradient with atomics where there is
+//     no memory for partials).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
