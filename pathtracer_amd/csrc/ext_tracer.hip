@@ -3749,21 +3749,29 @@ int ext_dispatch_batch(pt_ctx* ctx, const ExtBatchItem* items, int n) {
         st = dev_alloc(ctx, cs->batch_mem, tb);
         if (st != PT_OK) return st;
     }
-    // no room for the cursors (a budget): the kernels per stage, as they need none
-    if (whole && !cs->path_mem.p) {
-        const std::string err = ctx->err;
-        if (dev_alloc(ctx, cs->path_mem, (size_t)kBatchCursors * kCntStride * 4) != PT_OK) {
-            (void)hipGetLastError();
-            ctx->err = err;
-            whole = false;
-        } else {
-            st = clear_path_cursors(ctx, static_cast<int*>(cs->path_mem.p), kBatchCursors);
-            if (st != PT_OK) return st;
+    ExtWave* wave = &cs->wave;
+    if (whole) {
+        st = ensure_lean_wave(ctx, cap, &wave);
+        if (st != PT_OK) return st;
+        // the cursors after the wave: growing a full wave takes their room back. No room for
+        // them (a budget): the kernels per stage, as they need none
+        if (!cs->path_mem.p) {
+            const std::string err = ctx->err;
+            if (dev_alloc(ctx, cs->path_mem, (size_t)kBatchCursors * kCntStride * 4) != PT_OK) {
+                (void)hipGetLastError();
+                ctx->err = err;
+                whole = false;
+            } else {
+                st = clear_path_cursors(ctx, static_cast<int*>(cs->path_mem.p), kBatchCursors);
+                if (st != PT_OK) return st;
+            }
         }
     }
-    ExtWave* wave = &cs->wave;
-    st = whole ? ensure_lean_wave(ctx, cap, &wave) : ensure_ext_wave(ctx, cap);
-    if (st != PT_OK) return st;
+    if (!whole) {
+        st = ensure_ext_wave(ctx, cap);
+        if (st != PT_OK) return st;
+        wave = &cs->wave;
+    }
     ExtWave& Wv = *wave;
     hipError_t e = hipSuccess;
     if (!cs->batch_host) {

@@ -288,3 +288,29 @@ def test_sdfs_among_spheres_go_whole_up_to_a_size(kinds, size, whole):
     b, _, nb = render(1, json.dumps(s), w, h, spp, 3, frames=0)
     assert ("k_ext_path" in na) == whole and "k_ext_path" not in nb
     np.testing.assert_array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("graph_mode", [0, 1])
+def test_a_served_wave_grows_a_full_one(graph_mode):
+    """A full wave nearly as large as the served waves' capacity grows for them, which takes the
+    batch cursors back: they are made after it. Before, between and after dispatches of both kinds."""
+    text = SCENES["spheres"]()
+    with pt.Context(0, wave_paths=16384, graph_mode=graph_mode) as ctx:
+        lens, sc = ctx.scene_from_json(lens_scene()), ctx.scene_from_json(text)
+        images = []
+        for (w, h) in ((None, None), (120, 120), (128, 128), (16, 16)):
+            if w:
+                pt.Renderer(ctx, lens, w, h, spf=1, path_length=3, mode=pt.MODE_EXT).render_frame()
+                pt.Renderer(ctx, sc, w, h, spf=1, path_length=3, mode=pt.MODE_EXT).render_frame()
+            ctx.profile(graph_mode == 1)
+            ctx.profile_read(True)
+            with pt.Server(ctx) as server:
+                rid = server.submit(text, 40, 24, 8, 4, target=1e-6)
+                while server.step() is not None:
+                    pass
+                images.append(np.asarray(server.read(rid)))
+            assert graph_mode == 0 or "k_ext_path" in ctx.profile_read(True)
+            ctx.profile(False)
+        for x in images[1:]:
+            np.testing.assert_array_equal(x.view(np.uint32), images[0].view(np.uint32))
