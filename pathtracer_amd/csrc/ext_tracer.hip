@@ -2418,7 +2418,7 @@ constexpr int kPathSteps = 2, kPathVisits = 4;
 // 3.44 / 11.9 / 46.0, 4096 5.95 / 14.5 / 49.2 against 3.65 / 12.2 / 46.7, 32000 (1 / 16 /
 // 64) 3.1 / 13.3 / 45.5 against 1.5 / 11.6 / 44.1; mandelbulb and menger at depth 8 with
 // 1 / 4 / 16 / 32 / 64 samples 5.3 / 7.4 / 15.2 / 24.9 / 44.1 against 1.5 / 3.8 / 12.7 /
-// 24.6 / 48.5, and 2.1 to 2.7 times as fast at 1, 1.2 to 2.0 at 16 for each estimator
+// 24.6 / 48.5, and 2.1 to 2.6 times as fast at 1, 1.2 to 2.0 at 16 for each estimator
 // alone. Batched waves of a served burst 32.1 against 10.5 ms.
 // `direct`: the dispatch has one sample per pixel, all in this wave, and the paths'
 // texels are finished here instead of by k_ext_fold.
@@ -2432,12 +2432,12 @@ constexpr int kPathSteps = 2, kPathVisits = 4;
 // 1.8 / 1.3 to 1.6 / 1.1 to 1.4 / 0.94 to 1.3; mandelbulb, alone, with menger and with all, 1.5 to
 // 2.2 / 1.25 to 1.8 / 1.01 to 1.4 / 0.85 to 1.1; terrain, alone, with blob and with menger, whose
 // marches are short and whose normals cost the shading 6 evaluations of 22 sines, 1.1 to 1.4 /
-// 0.9 to 1.2 / 0.7 to 1.0 / 0.7 to 0.9, and one whose terrain fills the image 1.02 at 2.8 M and 0.95
-// at 3.7 M. Served waves (npaths of all requests; their kernels per stage march one ray per
+// 0.9 to 1.2 / 0.7 to 1.0 / 0.7 to 0.9, and one whose terrain fills the image 1.02 at 2.8 M, 0.95 at
+// 3.7 and 4.1 M, 0.79 at 7.4 M. Served waves (npaths of all requests; their kernels per stage march one ray per
 // lane) keep the line of scenes without spheres: 1.04 to 2.6 times as fast up to their usual
 // 4.2 M. Estimators whose box cuts them down to a solid core have no tails: in a box of 30 to
 // 300 spheres 1.15 to 1.2 at 4.1 M, 0.83 to 1.0 from there on, 0.77 to 0.9 in served waves.
-constexpr int kWholeSdfPaths = 1 << 25, kWholeSdfSpheres = 1 << 24, kWholeTerrainSpheres = 3 << 20;
+constexpr int kWholeSdfPaths = 1 << 25, kWholeSdfSpheres = 1 << 24, kWholeTerrainSpheres = 1 << 22;
 // A batched wave's tables (in constant memory for the kernel's length, so that a
 // request's scene comes through scalar loads), and its cursors: kSeg a request, then the
 // count of ended waves.

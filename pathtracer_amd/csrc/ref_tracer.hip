@@ -862,9 +862,9 @@ constexpr int kRefLanes = 64;  // threads per block: one wave, so that few paths
 // path records of 168 bytes in memory between them, one ray per lane in the
 // marches) and is bound by VALU issue in analytic scenes (rocprofv3, 3 spheres, a plane and
 // 2 boxes at 512x512x8: 0.82 wave instructions per unit and clock, 27 of 64 lanes active, 1660
-// instructions of a lane per segment with its shading and shadow ray): 1280x720x1 5 bounces 966 -> 230 us, 1920x1080x8 8 bounces 15.8 ->
-// 2.8 ms, 150x101x1 288 -> 81 us of kernels (one launch, its length the chain of a
-// path's bounces). SDF scenes are bound by the chain of their longest path (512x512x4
+// instructions of a lane per segment with its shading and shadow ray): 1280x720x1 5
+// bounces 966 -> 230 us, 1920x1080x8 8 bounces 15.8 -> 2.8 ms, 150x101x1 288 -> 81 us of
+// kernels (one launch, its length the chain of a path's bounces). SDF scenes are bound by the chain of their longest path (512x512x4
 // mandelbulb: up to 728 distance evaluations of 8 iterations, about 3.8 us each):
 // 29.2 -> 5.7 ms. Registers: 165 (analytic) and 184 to 190 (SDF) leave 3 and 2 waves per SIMD;
 // asking for 4 spills and was 20 % slower, and the path state in LDS while marching gave
@@ -1145,7 +1145,8 @@ static int ensure_ref_wave(pt_ctx* ctx, int cap) {
 // the life of the process. Every launch writes the records it reads, but for its
 // cursors, which it expects and leaves at zero: a call clears them first. Calls that
 // overlap on one device race on the wave, and what they leave in the cursors and the
-// count of ended waves would otherwise stay there and drop paths of every later call.
+// count of ended waves would otherwise stay there and drop paths of every later call (the
+// clearing launch: 1 us of a call among others, 3 of one alone; 150x101x1 takes 80 and 87).
 constexpr int kStaticWavePaths = 1 << 16;
 constexpr size_t kStaticWaveBytes = ref_wave_bytes(kStaticWavePaths);  // 1,843,456 B
 static __device__ __align__(256) char scratch[kStaticWaveBytes];

@@ -270,9 +270,9 @@ def test_large_sdf_waves_keep_the_kernels_per_stage():
     (("mandelbulb", "menger"), (1920, 1080, 8), True),  # 16.6 M paths
     (("mandelbulb", "menger"), (1920, 1080, 9), False),
     (("terrain", "mandelbulb"), (1920, 1080, 2), True),
-    (("terrain",), (1280, 720, 3), True),  # 2.8 M
-    (("terrain",), (1280, 720, 4), False),
-    (("terrain", "blob"), (1280, 720, 4), False),
+    (("terrain",), (1280, 720, 4), True),  # 3.7 M
+    (("terrain",), (1280, 720, 5), False),
+    (("terrain", "blob"), (1280, 720, 5), False),
     (("blob",), (1920, 1080, 16), True),  # 33.2 M
     (("blob",), (1920, 1080, 17), False),
 ])
