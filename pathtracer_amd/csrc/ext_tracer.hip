@@ -3834,9 +3834,11 @@ int ext_dispatch_batch(pt_ctx* ctx, const ExtBatchItem* items, int n) {
     } else {
         uint32_t kinds = 0;
         for (int k : plan.sdf_kinds) kinds |= 1u << (k & 7);
+        // everything that launch_wave's kernels and their order depend on
         const uint64_t key = (uint64_t)plan.width | (uint64_t)(plan.stack_need <= 32) << 4 |
-                             (uint64_t)plan.small_nodes << 5 | (uint64_t)plan.any_sdf << 6 | (uint64_t)whole << 7 | (uint64_t)kinds << 8 |
-                             (uint64_t)depth << 16 | (uint64_t)grid << 32;
+                             (uint64_t)plan.small_nodes << 5 | (uint64_t)plan.any_sdf << 6 | (uint64_t)whole << 7 |
+                             (uint64_t)kinds << 8 | (uint64_t)plan.extras << 15 | (uint64_t)depth << 16 |
+                             (uint64_t)grid << 32;
         auto it = cs->graphs.find(key);
         if (it == cs->graphs.end()) {
             hipGraph_t g = nullptr;

@@ -258,3 +258,36 @@ def test_denoising_falls_back_to_plain(gpu_ctx):
         assert all(st[i].state == pt.REQ_DONE and not st[i].denoised for i in ids)
         assert all(st[i].rel_error == st[i].rel_plain for i in ids)
         dn.close()
+
+
+def test_a_lens_after_waves_of_the_same_shape_without_one():
+    """Waves replay captured graphs by their shape, of which the lens and cyclide kernels are a part:
+    a lens scene served after one of many parallelograms, in the same launch shape but for those,
+    gives the image it gives alone."""
+    def quads():
+        s = scenes.cornell_dict(4, seed=3)
+        for i in range(20):
+            s["quad"].append({"position": [0.1 + 0.04 * i, 0.1, 0.5], "edge1": [0.03, 0.0, 0.0],
+                              "edge2": [0.0, 0.3, 0.02], "materialID": 1, "lightID": 0})
+        return json.dumps(s)
+
+    def lens():
+        s = json.loads(quads())
+        s["lens"] = [{"position": [0.5, 0.5, 0.3], "rotation": [0.0, 0.0, 0.0], "radius": 0.25, "focalLength": 0.3,
+                      "thickness": 0.0, "isConverging": True, "materialID": 1, "lightID": 0}]
+        return json.dumps(s)
+
+    def served(*texts):
+        with pt.Context(0) as ctx:
+            for text in texts:
+                with pt.Server(ctx) as server:
+                    rid = server.submit(text, 64, 48, 8, 5, target=1e-6)
+                    while server.step() is not None:
+                        pass
+                    image = np.asarray(server.read(rid))
+            return image
+
+    alone = served(lens())
+    assert (alone != served(quads())).any()
+    np.testing.assert_array_equal(served(quads(), lens()).view(np.uint32), alone.view(np.uint32))
+    np.testing.assert_array_equal(served(lens(), quads()).view(np.uint32), served(quads()).view(np.uint32))
